@@ -92,3 +92,30 @@ def test_device_buffers_and_a_stream_outside_the_vocabulary_reads_nothing():
     w_out, w_found, _ = oracle.copy_mean_rows(heads, tok[keep], lens[keep])
     np.testing.assert_array_equal(out[keep], w_out)
     np.testing.assert_array_equal(found[keep], w_found)
+
+
+@pytest.mark.parametrize("rule", ["mean", "latest-nearest", "longest-exact"])
+@pytest.mark.parametrize("shape", [
+    # (width, heads, kept, stride): the lanes' layouts (rows of whole quads or not, one to four
+    # groups of 256 coordinates), heads in and past one group of four, chunks of 64 and 256
+    # positions filled, one short and one over, the LDS limit's two stream counts a block.
+    (7, 1, 1, 66), (50, 5, 3, 130), (260, 4, 32, 258), (516, 6, 16, 514), (1020, 3, 8, 322),
+    (1022, 2, 8, 130), (256, 4, 16, 3841), (8, 16, 32, 1026)])
+def test_streams_at_the_edges_of_chunks_and_widths_match_the_oracle(rule, shape):
+    width, copy, kept, stride = shape
+    vocab = 23  # few tokens: distances and matches repeat, so ties reach across chunks
+    heads = K.random_heads(width + copy, vocab=vocab, width=width, copy=copy, kept=kept, rule=rule)
+    rng = np.random.default_rng(stride)
+    lens = [0, 1, 2, 3, 4, 64, 65, 66, 67, 129, 130, 257, 258, 259, 321, 513, 514, stride - 1, stride]
+    lens = np.array([n for n in lens if n <= stride], np.int32)
+    tok = rng.integers(0, vocab, (len(lens), stride)).astype(np.uint32)
+    print(f"copy edges {rule} {shape}", flush=True)
+    gpu = CopyHeads(heads)
+    try:
+        out, found, chosen = gpu.mean_rows(tok, lens)
+    finally:
+        gpu.close()
+    w_out, w_found, w_chosen = oracle.copy_mean_rows(heads, tok, lens)
+    np.testing.assert_array_equal(chosen, w_chosen)
+    np.testing.assert_array_equal(found, w_found)
+    np.testing.assert_array_equal(out, w_out)

@@ -5,13 +5,13 @@
 // hamming.rs:266-538; nearest :690-701, latest_of :584-598, longest_of :601-615, mean_by
 // :506-538).
 //
-// One wavefront reads one stream, four streams per block. Per head the lanes take the candidate
-// positions 64 at a time: under the mean rule the distances are staged in LDS and the kept
-// positions come out in (distance, position) order as successive wave minima of packed keys;
-// the latest and longest rules are wave maxima over the matching positions. The weighted sums
-// run with the lanes over the table row's coordinates, in 64-bit integers: a weight is at most
-// 2^31 and a table value at most 2^15 in magnitude, so a head's sum over at most 32 positions
-// stays below 2^51.
+// One wavefront reads one stream, four streams per block. The lanes take the candidate positions
+// 64 at a time, four heads at once: under the mean rule the distances are staged in LDS with a
+// histogram per head, whose running count gives the distance up to which positions are kept, and
+// the kept ones are ranked by (distance, position); the latest and longest rules are wave minima
+// and maxima over the matching positions. The weighted sums run with the lanes over the table
+// row's coordinates, in 64-bit integers: a weight is at most 2^31 and a table value at most 2^15
+// in magnitude, so a head's sum over at most 32 positions stays below 2^51.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -24,11 +24,14 @@
 
 namespace copyread {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kPerLane = UOR_COPY_MAX_WIDTH / 64;
+constexpr int kWaves = 4;          // streams a block reads, one per wavefront
+constexpr int kHeads = 4;          // heads that one pass over the positions serves
+constexpr int kChunks = 4;         // chunks of 64 positions whose codes are in flight together
+constexpr int kRows = 8;           // table rows in flight in a head's sum
+constexpr uint32_t kBins = 68;     // distances 0..64, padded
 constexpr uint32_t kPosBits = 20;  // positions below UOR_COPY_MAX_STRIDE fit
 constexpr uint32_t kPosMask = (1u << kPosBits) - 1;
+constexpr uint32_t kNone = 0xffffffffu;
 
 struct Dev {
   uint32_t vocab, width, copy, kept, rule, has_marker, m0, m1;
@@ -38,10 +41,10 @@ struct Dev {
   const int16_t *table;
 };
 
-struct WaveLds {
-  uint8_t dist[UOR_COPY_MAX_STRIDE];
-  uint32_t pick[UOR_COPY_MAX_KEPT];  // s | distance << 24
-};
+// A wavefront's LDS: the distances [kHeads][pitch] (bytes), the heads' histograms [kHeads][kBins],
+// then one head's picked keys.
+constexpr uint32_t kFixedLds = 4 * (kHeads * kBins + UOR_COPY_MAX_KEPT);
+inline uint32_t wave_lds_bytes(uint32_t stride) { return kFixedLds + kHeads * ((stride + 63u) & ~63u); }
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp32(uint32_t v) {
@@ -71,20 +74,54 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The value of the lane before, and `first` on lane 0.
+__device__ __forceinline__ uint64_t lane_before(uint64_t v, uint64_t first) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)first, (int)(uint32_t)v, 0x138, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(first >> 32), (int)(uint32_t)(v >> 32), 0x138, 0xf, 0xf, false);
+  return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ uint64_t lane64(uint64_t v, int l) {
+  return (uint64_t)lane32((uint32_t)(v >> 32), l) << 32 | lane32((uint32_t)v, l);
+}
+
 __device__ __forceinline__ uint64_t code(const Dev &D, uint32_t token, uint32_t h) {
   return D.codes[(uint64_t)token * D.copy + h];
 }
+// The token's codes of heads h0 .. h0 + kHeads - 1 (a head past the last repeats the last): two
+// 16-byte loads where the token's codes are whole pairs of them.
+__device__ __forceinline__ void codes_of(const Dev &D, uint32_t token, uint32_t h0, uint64_t (&c)[kHeads]) {
+  const uint64_t *at = D.codes + (uint64_t)token * D.copy;
+  if (D.copy % kHeads == 0) {
+    const ulonglong2 a = *(const ulonglong2 *)(at + h0), b = *(const ulonglong2 *)(at + h0 + 2);
+    c[0] = a.x, c[1] = a.y, c[2] = b.x, c[3] = b.y;
+  } else {
+#pragma unroll
+    for (int g = 0; g < kHeads; g++) c[g] = at[h0 + g < D.copy ? h0 + g : D.copy - 1];
+  }
+}
 // joined (:379-385): under copy key 2 the near token's first half and the far token's second.
-__device__ __forceinline__ uint64_t joined(const Dev &D, uint32_t near, uint32_t far, uint32_t h) {
-  const uint64_t c = code(D, near, h), first = D.pair[h];
-  return first ? (c & first) | (code(D, far, h) & ~first) : c;
+__device__ __forceinline__ uint64_t joined(uint64_t near, uint64_t far, uint64_t first) {
+  return first ? (near & first) | (far & ~first) : near;
 }
 
-// n / k rounded toward zero (Rust's i128 division), for k >= 1, in the integer division of
-// fbs_int.h: the kernels divide by no variable with the compiler's `/`, whose expansion goes
-// through a float reciprocal estimate.
-__device__ __forceinline__ int64_t div_trunc(int64_t n, uint32_t k) {
-  const uint64_t q = fbs::div128_64(fbs::uabs64(n), k);
+// floor(n / k) for n < 2^59 and k in [1, 32], without a division (the kernels divide by no
+// variable with the compiler's `/`, whose expansion goes through a float reciprocal estimate): the
+// high 64 bits of n m with m = ceil(2^64 / k), as m exceeds 2^64 / k by less than 1 and so n m / 2^64
+// exceeds n / k by less than n / 2^64 < 1 / k.
+struct Magic {
+  uint64_t m[33];
+};
+constexpr Magic make_magic() {
+  Magic g{};
+  for (uint64_t k = 2; k <= 32; k++) g.m[k] = ~0ull / k + 1;  // m[1] stays 0: no factor below 2^64
+  return g;
+}
+__constant__ const Magic kMagic = make_magic();
+static_assert(UOR_COPY_MAX_KEPT <= 32 && UOR_COPY_MAX_HEADS <= 32, "the divisors' table");
+// n / k rounded toward zero (Rust's i128 division): |n| is a sum of at most 32 products of 2^31
+// and 2^15, or of 16 such quotients.
+__device__ __forceinline__ int64_t div_trunc(int64_t n, uint64_t m) {
+  const uint64_t q = m ? __umul64hi(fbs::uabs64(n), m) : fbs::uabs64(n);
   return n < 0 ? -(int64_t)q : (int64_t)q;
 }
 
@@ -93,113 +130,252 @@ __device__ __forceinline__ uint64_t weight_q31(int32_t margin, uint32_t d) {
   return fbs::copy_weight_q31(margin, d);
 }
 
-__global__ __launch_bounds__(kThreads) void copy_mean_rows(Dev D, const uint32_t *tokens,
-                                                           const int32_t *lengths,
-                                                           const uint8_t *opening, uint32_t rows,
-                                                           uint32_t stride, int64_t *out,
-                                                           uint8_t *found, int32_t *chosen) {
-  __shared__ WaveLds lds[kWaves];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t row = blockIdx.x * kWaves + wave;
+// One wavefront reads one stream. NV > 0: the lanes own four neighbouring coordinates each, NV
+// groups of 256 (a width that is a multiple of 4, whose rows load as 8 bytes a lane); NV = 0:
+// coordinates 64 apart, any width.
+//
+// Bound by latency: 4,096 streams are four wavefronts a SIMD, so the passes over the positions and
+// the kept rows count by their round trips. One pass over the positions serves kHeads heads (a
+// position's codes lie side by side) with the codes of kChunks chunks in flight, and the far key
+// half comes from the lane before. Under the mean rule the distances go to LDS with a histogram
+// a head; the kept positions are those below the distance at which the histogram reaches `kept`
+// and the earliest at it, one further pass of ballots (the first form took `kept` successive wave
+// minima, a pass each). The head's sum loads kRows rows at a time. 4,096 streams of up to 1,024
+// tokens, 4 heads keeping 16: 505 us before, 94 us now.
+template <int NV>
+__global__ __launch_bounds__(64 * kWaves) void copy_mean_rows(Dev D, const uint32_t *__restrict__ tokens,
+                                                              const int32_t *__restrict__ lengths,
+                                                              const uint8_t *__restrict__ opening, uint32_t rows,
+                                                              uint32_t stride, uint32_t pitch,
+                                                              int64_t *__restrict__ out,
+                                                              uint8_t *__restrict__ found,
+                                                              int32_t *__restrict__ chosen) {
+  constexpr int kVals = NV ? 4 * NV : UOR_COPY_MAX_WIDTH / 64;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint32_t row = blockIdx.x * (blockDim.x >> 6) + wave;
   if (row >= rows) return;
-  WaveLds &w = lds[wave];
+  uint8_t *mine = lds + wave * (kFixedLds + kHeads * pitch);
+  uint32_t *hist = (uint32_t *)mine;
+  uint32_t *pick = hist + kHeads * kBins;
+  uint8_t *dist = mine + kFixedLds;
   const uint32_t *tok = tokens + (uint64_t)row * stride;
   int len = lengths[row];
   if (len < 0 || len > (int)stride) len = 0;  // outside the row: reads nothing
-  bool bad = false;
-  for (int i = lane; i < len; i += 64) bad |= tok[i] >= D.vocab;
-  if (__any(bad)) len = 0;                     // a token outside the vocabulary: reads nothing
   const int t = len - 1;
-  const bool opens = D.has_marker ? (len >= 2 && tok[t - 1] == D.m0 && tok[t] == D.m1)
+  // The row's own token and the one before; a token outside the vocabulary reads nothing.
+  const uint32_t raw_own = len ? tok[t] : 0, raw_prev = t > 0 ? tok[t - 1] : raw_own;
+  bool bad = raw_own >= D.vocab || raw_prev >= D.vocab;
+  const uint32_t own = bad ? 0 : raw_own, prev = bad ? 0 : raw_prev;
+  const bool opens = D.has_marker ? (len >= 2 && raw_prev == D.m0 && raw_own == D.m1)
                                   : (opening != nullptr && opening[row] != 0);
-  int64_t sum[kPerLane];
+  uint32_t rule = D.rule;
+  if (rule == UOR_COPY_LONGEST_AFTER_OPENING)
+    rule = opens ? UOR_COPY_LATEST_EXACT : UOR_COPY_LONGEST_EXACT;
+  int64_t sum[kVals];
 #pragma unroll
-  for (int j = 0; j < kPerLane; j++) sum[j] = 0;
+  for (int j = 0; j < kVals; j++) sum[j] = 0;
   int heads_found = 0;
-  for (uint32_t h = 0; h < D.copy; h++) {
-    int n = 0;
-    if (len >= 1) {
-      const uint64_t q = joined(D, tok[t], tok[t > 0 ? t - 1 : 0], h);
-      uint32_t rule = D.rule;
-      if (rule == UOR_COPY_LONGEST_AFTER_OPENING)
-        rule = opens ? UOR_COPY_LATEST_EXACT : UOR_COPY_LONGEST_EXACT;
-      if (rule == UOR_COPY_MEAN) {
-        for (int s = 1 + lane; s < t; s += 64)
-          w.dist[s] = (uint8_t)__popcll(q ^ joined(D, tok[s - 1], tok[s >= 2 ? s - 2 : 0], h));
-        wave_sync();
-        uint32_t last = 0;  // every key is at least 1 (positions start at 1)
-        for (uint32_t r = 0; r < D.kept; r++) {
-          uint32_t loc = 0xffffffffu;
-          for (int s = 1 + lane; s < t; s += 64) {
-            const uint32_t k = (uint32_t)w.dist[s] << kPosBits | (uint32_t)s;
-            if (k > last && k < loc) loc = k;
+  for (uint32_t h0 = 0; h0 < D.copy; h0 += kHeads) {
+    uint64_t q[kHeads], first[kHeads], carry[kHeads], before[kHeads];
+    {
+      uint64_t a[kHeads], b[kHeads];
+      codes_of(D, own, h0, a);
+      codes_of(D, prev, h0, b);
+#pragma unroll
+      for (int g = 0; g < kHeads; g++) {
+        first[g] = D.pair[h0 + g < D.copy ? h0 + g : D.copy - 1];
+        q[g] = joined(a[g], b[g], first[g]);
+        carry[g] = before[g] = 0;
+      }
+    }
+    if (rule == UOR_COPY_LONGEST_EXACT && len && !bad) {
+#pragma unroll
+      for (int g = 0; g < kHeads; g++) {
+        const int kd = first[g] ? 2 : 1;
+        const uint32_t far = t >= kd ? tok[t - kd] : 0;
+        before[g] = far < D.vocab ? code(D, far, h0 + g < D.copy ? h0 + g : D.copy - 1) : 0;
+      }
+    }
+    for (uint32_t i = lane; i < kHeads * kBins; i += 64) hist[i] = 0;
+    wave_sync();
+    // Latest rules: least distance << 20 | (mask - s). Longest: the latest exact match and the
+    // latest whose token before the key matches too.
+    uint32_t best[kHeads], longer[kHeads];
+#pragma unroll
+    for (int g = 0; g < kHeads; g++) {
+      best[g] = rule == UOR_COPY_LONGEST_EXACT ? 0 : kNone;
+      longer[g] = 0;
+    }
+    for (int s0 = 1; s0 < t; s0 += 64 * kChunks) {
+      uint32_t near[kChunks];
+      uint64_t c[kChunks][kHeads];
+#pragma unroll
+      for (int u = 0; u < kChunks; u++) {
+        const int s = s0 + 64 * u + (int)lane;
+        near[u] = s < t ? tok[s - 1] : 0;
+        bad |= near[u] >= D.vocab;
+        near[u] = near[u] < D.vocab ? near[u] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kChunks; u++)
+        if (s0 + 64 * u < t) codes_of(D, near[u], h0, c[u]);
+#pragma unroll
+      for (int u = 0; u < kChunks; u++) {
+        if (s0 + 64 * u >= t) break;
+        const int s = s0 + 64 * u + (int)lane;
+        const bool in = s < t;
+#pragma unroll
+        for (int g = 0; g < kHeads; g++) {
+          if (h0 + g >= D.copy) break;
+          uint64_t far = 0;
+          if (first[g]) {  // position 1's far token is its near one
+            far = lane_before(c[u][g], s0 == 1 && u == 0 ? lane64(c[u][g], 0) : carry[g]);
+            carry[g] = lane64(c[u][g], 63);
           }
-          const uint32_t m = wave_min32(loc);
-          if (m == 0xffffffffu) break;
-          if (lane == 0) w.pick[r] = (m & kPosMask) | (m >> kPosBits) << 24;
-          last = m;
-          n++;
-        }
-      } else if (rule == UOR_COPY_LATEST_EXACT || rule == UOR_COPY_LATEST_NEAREST) {
-        uint32_t best = 0xffffffffu;  // distance << 20 | (mask - s): least distance, latest s
-        for (int s = 1 + lane; s < t; s += 64) {
-          const uint32_t d = __popcll(q ^ joined(D, tok[s - 1], tok[s >= 2 ? s - 2 : 0], h));
-          if (rule == UOR_COPY_LATEST_EXACT && d != 0) continue;
-          best = min(best, d << kPosBits | (kPosMask - (uint32_t)s));
-        }
-        const uint32_t m = wave_min32(best);
-        if (m != 0xffffffffu) {
-          if (lane == 0) w.pick[0] = (kPosMask - (m & kPosMask)) | (m >> kPosBits) << 24;
-          n = 1;
-        }
-      } else {  // longest exact (:601-615) with longer_at (:349-352)
-        const int kd = D.pair[h] ? 2 : 1;
-        uint32_t ex = 0, lg = 0;
-        const uint64_t before = t >= kd ? code(D, tok[t - kd], h) : 0;
-        for (int s = 1 + lane; s < t; s += 64) {
-          if (joined(D, tok[s - 1], tok[s >= 2 ? s - 2 : 0], h) != q) continue;
-          ex = max(ex, (uint32_t)s);
-          if (s > kd && code(D, tok[s - 1 - kd], h) == before) lg = max(lg, (uint32_t)s);
-        }
-        ex = wave_max32(ex);
-        lg = wave_max32(lg);
-        const uint32_t pick = lg ? lg : ex;
-        if (pick) {
-          if (lane == 0) w.pick[0] = pick;
-          n = 1;
+          const uint32_t d = (uint32_t)__popcll(q[g] ^ joined(c[u][g], far, first[g]));
+          if (rule == UOR_COPY_MEAN) {
+            if (in) {
+              dist[g * pitch + s] = (uint8_t)d;
+              atomicAdd(&hist[g * kBins + d], 1u);
+            }
+          } else if (rule == UOR_COPY_LONGEST_EXACT) {
+            if (in && d == 0) {
+              const int kd = first[g] ? 2 : 1;
+              best[g] = max(best[g], (uint32_t)s);
+              const uint32_t past = s > kd ? tok[s - 1 - kd] : kNone;
+              if (past < D.vocab && code(D, past, h0 + g) == before[g]) longer[g] = max(longer[g], (uint32_t)s);
+            }
+          } else if (in && (d == 0 || rule == UOR_COPY_LATEST_NEAREST)) {
+            best[g] = min(best[g], d << kPosBits | (kPosMask - (uint32_t)s));
+          }
         }
       }
     }
+    bad = __any(bad);
     wave_sync();
-    if (chosen != nullptr && lane < (int)D.kept)
-      chosen[((uint64_t)row * D.copy + h) * D.kept + lane] = lane < n ? (int32_t)w.pick[lane] : -1;
-    int64_t head[kPerLane];
 #pragma unroll
-    for (int j = 0; j < kPerLane; j++) head[j] = 0;
-    int count = 0;
-    for (int k = 0; k < n; k++) {
-      const uint32_t p = w.pick[k];
-      const uint64_t wt = weight_q31(D.margins[h], p >> 24);
-      if (wt == 0) continue;
-      count++;
-      const int16_t *trow = D.table + (uint64_t)tok[p & 0xffffff] * D.width;
+    for (int g = 0; g < kHeads; g++) {
+      const uint32_t h = h0 + g;
+      if (h >= D.copy) break;
+      // This head's picks, one a lane in the order read: (s | distance << 24); n of them.
+      uint32_t mypick = 0;
+      int n = 0;
+      if (bad || t <= 1) {
+        // nothing to read
+      } else if (rule == UOR_COPY_MEAN) {
+        // The distance `at` where the positions below it are fewer than `kept` and those up to it
+        // are not (64 where the positions are no more than `kept`): lane b counts distance b.
+        uint32_t upto = hist[g * kBins + lane];
+        const uint32_t mineb = upto;
 #pragma unroll
-      for (int j = 0; j < kPerLane; j++) {
-        const uint32_t c = (uint32_t)lane + 64u * j;
-        if (c < D.width) head[j] += (int64_t)trow[c] * (int64_t)wt;
+        for (int m = 1; m < 64; m <<= 1) {
+          const uint32_t o = (uint32_t)__shfl_up((int)upto, m, 64);
+          upto += (int)lane >= m ? o : 0;
+        }
+        const uint64_t full = __ballot(upto >= D.kept);
+        const uint32_t at = full ? (uint32_t)__ffsll((unsigned long long)full) - 1 : 64u;
+        const uint32_t below = full ? lane32(upto - mineb, (int)at) : lane32(upto, 63);
+        uint32_t lows = 0, ties = 0, tie_cap = D.kept - below;
+        for (int s0 = 1; s0 < t; s0 += 64) {
+          const int s = s0 + (int)lane;
+          const uint32_t d = s < t ? dist[g * pitch + s] : 255u;
+          const uint64_t lo = __ballot(d < at), eq = __ballot(d == at);
+          if (lo | eq) {
+            const uint64_t under = (1ull << lane) - 1;
+            const uint32_t lr = lows + __popcll(lo & under), er = ties + __popcll(eq & under);
+            if (d < at) pick[lr] = d << kPosBits | (uint32_t)s;
+            if (d == at && er < tie_cap) pick[below + er] = d << kPosBits | (uint32_t)s;
+            lows += __popcll(lo);
+            ties += __popcll(eq);
+          }
+        }
+        n = (int)(below + min(ties, tie_cap));
+        wave_sync();
+        // In (distance, position) order: a pick's place is the number of smaller keys.
+        const uint32_t key = (int)lane < n ? pick[lane] : kNone;
+        uint32_t place = 0;
+        for (int k = 0; k < n; k++) place += lane32(key, k) < key ? 1u : 0u;
+        wave_sync();
+        if ((int)lane < n) pick[place] = (key & kPosMask) | (key >> kPosBits) << 24;
+        wave_sync();
+        mypick = (int)lane < n ? pick[lane] : 0;
+      } else if (rule == UOR_COPY_LONGEST_EXACT) {
+        const uint32_t ex = wave_max32(best[g]), lg = wave_max32(longer[g]);
+        mypick = lg ? lg : ex;
+        n = mypick != 0;
+      } else {
+        const uint32_t m = wave_min32(best[g]);
+        if (m != kNone) {
+          mypick = (kPosMask - (m & kPosMask)) | (m >> kPosBits) << 24;
+          n = 1;
+        }
       }
-    }
-    if (count) {
+      if (chosen != nullptr && lane < D.kept)
+        chosen[((uint64_t)row * D.copy + h) * D.kept + lane] = (int)lane < n ? (int32_t)mypick : -1;
+      // Each pick's weight and row, a lane each. Weights fall with the distance, so those above
+      // zero lead. The negated weight is at least -2^31, a signed 32-bit factor.
+      const uint64_t wt = (int)lane < n ? weight_q31(D.margins[h], mypick >> 24) : 0;
+      const uint32_t neg = 0u - (uint32_t)wt;
+      const int count = __popcll(__ballot(wt != 0));
+      if (count == 0) continue;
+      const uint32_t rowtok = (int)lane < n ? tok[mypick & 0xffffff] : 0;
+      int64_t head[kVals];
+#pragma unroll
+      for (int j = 0; j < kVals; j++) head[j] = 0;
+      if constexpr (NV > 0) {
+        for (int k0 = 0; k0 < count; k0 += kRows) {
+          short4 v[kRows][NV];
+#pragma unroll
+          for (int k = 0; k < kRows; k++)
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+              const uint32_t c = 4 * (lane + 64u * j);
+              v[k][j] = make_short4(0, 0, 0, 0);
+              if (k0 + k < count && c < D.width)
+                v[k][j] = *(const short4 *)(D.table + (uint64_t)lane32(rowtok, k0 + k) * D.width + c);
+            }
+#pragma unroll
+          for (int k = 0; k < kRows; k++) {
+            const int32_t w = k0 + k < count ? (int32_t)lane32(neg, k0 + k) : 0;
+#pragma unroll
+            for (int j = 0; j < NV; j++) {
+              head[4 * j] += (int64_t)v[k][j].x * w;
+              head[4 * j + 1] += (int64_t)v[k][j].y * w;
+              head[4 * j + 2] += (int64_t)v[k][j].z * w;
+              head[4 * j + 3] += (int64_t)v[k][j].w * w;
+            }
+          }
+        }
+      } else {
+        for (int k = 0; k < count; k++) {
+          const int32_t w = (int32_t)lane32(neg, k);
+          const int16_t *trow = D.table + (uint64_t)lane32(rowtok, k) * D.width;
+#pragma unroll
+          for (int j = 0; j < kVals; j++) {
+            const uint32_t c = lane + 64u * j;
+            if (c < D.width) head[j] += (int64_t)trow[c] * w;
+          }
+        }
+      }
       heads_found++;
+      const uint64_t m = kMagic.m[count];
 #pragma unroll
-      for (int j = 0; j < kPerLane; j++) sum[j] += div_trunc(head[j], count);
+      for (int j = 0; j < kVals; j++) sum[j] += div_trunc(-head[j], m);
     }
     wave_sync();
+    if (bad) break;
   }
+  if (bad) {  // every group of heads sees the same tokens, so the first one finds it
+    heads_found = 0;
+    if (chosen != nullptr)
+      for (uint32_t i = lane; i < D.copy * D.kept; i += 64) chosen[(uint64_t)row * D.copy * D.kept + i] = -1;
+  }
+  const uint64_t m = kMagic.m[heads_found];
 #pragma unroll
-  for (int j = 0; j < kPerLane; j++) {
-    const uint32_t c = (uint32_t)lane + 64u * j;
-    if (c < D.width) out[(uint64_t)row * D.width + c] = heads_found ? div_trunc(sum[j], heads_found) : 0;
+  for (int j = 0; j < kVals; j++) {
+    const uint32_t c = NV ? 4 * (lane + 64u * (j / 4)) + j % 4 : lane + 64u * j;
+    if (c < D.width) out[(uint64_t)row * D.width + c] = heads_found ? div_trunc(sum[j], m) : 0;
   }
   if (lane == 0) found[row] = heads_found > 0;
 }
@@ -310,8 +486,14 @@ extern "C" int uor_copy_mean_rows_async(void *handle, const uint32_t *d_tokens,
   int prev = 0;
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(h->device);
-  hipLaunchKernelGGL(copy_mean_rows, dim3((rows + kWaves - 1) / kWaves), dim3(kThreads), 0,
-                     (hipStream_t)stream, h->d, d_tokens, d_lengths, d_opening, rows, stride,
+  // Four streams a block, or two where their distances would pass 64 KB of LDS (strides above
+  // 3,840). The vector form wants rows of whole 8-byte pieces.
+  const uint32_t pitch = (stride + 63u) & ~63u;
+  const uint32_t waves = kWaves * wave_lds_bytes(stride) <= (64u << 10) ? kWaves : kWaves / 2;
+  const uint32_t w = h->d.width;
+  auto *kernel = w % 4 ? copy_mean_rows<0> : w <= 256 ? copy_mean_rows<1> : w <= 512 ? copy_mean_rows<2> : copy_mean_rows<4>;
+  hipLaunchKernelGGL(kernel, dim3((rows + waves - 1) / waves), dim3(64 * waves), waves * wave_lds_bytes(stride),
+                     (hipStream_t)stream, h->d, d_tokens, d_lengths, d_opening, rows, stride, pitch,
                      d_out, d_found, d_chosen);
   const hipError_t e = hipGetLastError();
   (void)hipSetDevice(prev);
