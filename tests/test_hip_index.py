@@ -286,3 +286,24 @@ def test_middle_blocks_and_extreme_distances():
     t, idx = device(extreme)
     assert ix.build(t, idx) == ix.Status.Ok
     check_scan(ix.probe(t, q[None], 1, idx), extreme, q[None], 1, oracle_built(extreme))
+
+
+@pytest.mark.parametrize("width", [16, 20, 32, 36, 60, 64, 100, 256])
+@pytest.mark.parametrize("count,cells", [(9, 2), (64, 1), (65, 1), (129, 2), (700, 3), (3000, 256)])
+def test_probe_at_the_edges_of_row_segments_and_batches(width, count, cells):
+    """Row widths around the staged 32 words, candidate counts around 64, equal distances (few
+    distinct rows), differences of the whole int32 range, fewer than 8 candidates."""
+    rng = np.random.default_rng(count * 1000 + width)
+    table = random_table(rng, count, width, absent_frac=0.02, cells=cells)
+    few = rng.integers(0, 4, count)
+    if width > 16:
+        values = rng.choice(np.array([-(1 << 31), -1, 0, 1, (1 << 31) - 1]), (4, width - 16))
+        table[:, 8:-8] = np.where(rng.random((count, 1)) < 0.7, values[few], table[:, 8:-8])
+    t, idx = device(table)
+    assert ix.build(t, idx, True) == ix.Status.Ok
+    host = oracle_built(table, True)
+    queries = random_table(rng, 5, width)
+    queries[0] = table[count // 2]
+    print(f"probe {width} {count} {cells}", flush=True)
+    for k in (1, 16):
+        check_scan(ix.probe(t, queries, k, idx), table, queries, k, host)

@@ -612,6 +612,26 @@ __device__ __forceinline__ int64_t row_l1(const int32_t *q, const int32_t *row, 
   return (int64_t)s;
 }
 
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp64(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, false);
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ uint64_t lane64(uint64_t v, int l) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
+__device__ __forceinline__ uint64_t min64(uint64_t a, uint64_t b) { return a < b ? a : b; }
+// The wave's minimum, uniform: butterflies inside each row of 16 lanes, then the rows as scalars.
+__device__ __forceinline__ uint64_t wave_low64(uint64_t v) {
+  v = min64(v, dpp64<0xb1>(v));
+  v = min64(v, dpp64<0x4e>(v));
+  v = min64(v, dpp64<0x141>(v));
+  v = min64(v, dpp64<0x140>(v));
+  return min64(min64(lane64(v, 0), lane64(v, 16)), min64(lane64(v, 32), lane64(v, 48)));
+}
+
 // fill_admitted (inverted_file.cpp:83-96) on one wave: the k nearest non-empty cells by
 // cell_distance (:38-47), ties to the lower cell; adm[0..16) on every lane, ABSENT-padded.
 // rd: 32 words of LDS for this wave. Called by every wave of the block (it synchronises).
@@ -635,15 +655,70 @@ __device__ void admit_wave(const int32_t *sq, uint32_t width, const int32_t *sro
     uint64_t mine = key[0];
 #pragma unroll
     for (int j = 1; j < 4; j++) mine = key[j] < mine ? key[j] : mine;
-    const uint64_t m = i < k ? wave_min64(mine) : ~0ull;
+    const uint64_t m = i < k ? wave_low64(mine) : ~0ull;
     adm[i] = m == ~0ull ? kAbsent : (uint32_t)(m & 255);
 #pragma unroll
     for (int j = 0; j < 4; j++) key[j] = key[j] == m ? ~0ull : key[j];
   }
 }
 
+// acc + |a - b| for biased (unsigned) words: a 32-bit absolute difference and a 64-bit add.
+__device__ __forceinline__ uint64_t sad_add(uint64_t acc, uint32_t a, uint32_t b) {
+  uint32_t d;
+  asm("v_sad_u32 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
+  asm("v_mad_u64_u32 %0, vcc, %1, 1, %0" : "+v"(acc) : "v"(d) : "vcc");
+  return acc;
+}
+
+// The wave's 8 best (distance, token), ascending, entry i on lane i (the other lanes idle).
+struct Best8 {
+  uint64_t d = (uint64_t)kFar;
+  uint32_t t = kAbsent;
+  // Takes every lane's candidate (x, y) where `in`: those before the last entry are inserted one
+  // by one (about 40 of 2,048 candidates in no order), the list moving up past each. Where many
+  // would pass (the first candidates), the nearest goes first: eight insertions then settle them.
+  __device__ __forceinline__ void take(uint64_t x, uint32_t y, bool in) {
+    const uint32_t lane = threadIdx.x % 64;
+    uint64_t ld = lane64(d, 7);
+    uint32_t lt = (uint32_t)__builtin_amdgcn_readlane((int)t, 7);
+    uint64_t todo = __ballot(in & ((x < ld) | ((x == ld) & (y < lt))));
+    while (todo) {
+      int l = __builtin_ctzll(todo);
+      if (__popcll(todo) > 16) {
+        const bool mine = (todo >> lane) & 1;
+        const uint64_t low = wave_low64(mine ? x : ~0ull);
+        l = __builtin_ctzll(__ballot(mine & (x == low)));
+      }
+      const uint64_t nx = lane64(x, l);
+      const uint32_t ny = (uint32_t)__builtin_amdgcn_readlane((int)y, l);
+      const uint64_t less = __ballot((lane < 8) & ((d < nx) | ((d == nx) & (t < ny))));
+      const bool there = __ballot((lane < 8) & (d == nx) & (t == ny)) != 0;
+      const uint32_t at = (uint32_t)__popcll(less);
+      const uint64_t pd = dpp64<0x111>(d);  // the entry on the lane before
+      const uint32_t pt = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t, 0x111, 0xf, 0xf, false);
+      if (!there && lane < 8) {
+        d = lane > at ? pd : lane == at ? nx : d;
+        t = lane > at ? pt : lane == at ? ny : t;
+      }
+      ld = lane64(d, 7);
+      lt = (uint32_t)__builtin_amdgcn_readlane((int)t, 7);
+      todo &= ~(1ull << l);
+      todo &= __ballot((x < ld) | ((x == ld) & (y < lt)));
+    }
+  }
+};
+
 // probe (inverted_file.cpp:250-258; kernel uor_if_probe, kernels.cu:198-213) for one query row
 // per wave. The index is not validated here: callers validate it once per change.
+//
+// Bound by the rows' way into the lanes: a candidate row on every lane makes each 16-byte load
+// touch 64 cache lines. Eight lanes therefore load a row (each load 8 whole 128-byte rows), the
+// rows pass through LDS with their pieces rotated by the row, so that neither side meets bank
+// conflicts, and come back a row a lane; the next candidates' rows are in flight meanwhile and the
+// members of those after them. 65,536 queries over 65,536 tokens at k 8 (2,048 candidate rows of
+// 128 bytes each): 2.00 ms with a row a lane and a list of 8 on every lane, 1.1 ms so; the vector unit
+// is then busy two thirds of the time (three instructions a row word).
+constexpr uint32_t kSegWords = 32;  // row words staged at once
 __global__ __launch_bounds__(64 * kProbeWaves) void index_probe(
     const int32_t *__restrict__ table, uint32_t count, uint32_t width,
     const int32_t *__restrict__ roots, const int32_t *__restrict__ queries, uint32_t rows,
@@ -653,6 +728,8 @@ __global__ __launch_bounds__(64 * kProbeWaves) void index_probe(
   __shared__ __align__(16) int32_t sroots[128];
   __shared__ __align__(16) int32_t sq[kProbeWaves][UOR_FBS_INDEX_MAX_WIDTH];
   __shared__ int64_t rd[kProbeWaves][32];
+  __shared__ __align__(16) uint4 stage[kProbeWaves][64 * kSegWords / 4];
+  __shared__ uint32_t range[kProbeWaves][32];  // the admitted cells' first members, then counts
   const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const uint32_t row = blockIdx.x * kProbeWaves + wave;
   const uint32_t src = row < rows ? row : rows - 1;  // surplus waves repeat the last row, unwritten
@@ -662,48 +739,107 @@ __global__ __launch_bounds__(64 * kProbeWaves) void index_probe(
   uint32_t adm[16];
   admit_wave(sq[wave], width, sroots, offsets, k, rd[wave], adm);
   // The admitted cells' member ranges, concatenated; lane j takes positions j, j + 64, ...
-  uint32_t lo[16], n[16], total = 0;
+  uint32_t total = 0;
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < 16; i++) {
-    lo[i] = n[i] = 0;
+    uint32_t lo = 0, n = 0;
     if (adm[i] != kAbsent) {
       const uint32_t a = offsets[adm[i]], b = offsets[adm[i] + 1];
       if (b < a || b > count)
         bad = true;
       else
-        lo[i] = a, n[i] = b - a;
+        lo = a, n = b - a;
     }
-    total += n[i];
+    if (lane == 0) range[wave][i] = lo, range[wave][16 + i] = n;
+    total += n;
   }
-  Top8 best;
-  best.clear();
-  for (uint32_t j = lane; j < total; j += 64) {
-    uint32_t p = j, at = 0;
-    bool found = false;
+  // The query biased to unsigned words, as the rows are.
+  for (uint32_t i = lane; i < width; i += 64) sq[wave][i] ^= (int32_t)0x80000000;
+  wave_sync();
+  const uint32_t *lo = range[wave], *num = range[wave] + 16;
+  // This lane's next candidate: position `left` past the start of range `cell`.
+  uint32_t cell = 0, left = lane, pos = lane;
+  auto next_member = [&]() -> uint32_t {  // its token (ABSENT past the last), and on by 64
+    uint32_t t = kAbsent;
+    if (pos < total) {
+      while (left >= num[cell]) left -= num[cell++];  // pos < total: a range holds it
+      t = members[lo[cell] + left];
+      if (t >= count) bad = true, t = kAbsent;
+    }
+    left += 64;
+    pos += 64;
+    return t;
+  };
+  const uint32_t pieces = width / 4, sub = lane & 7, grp = lane >> 3;
+  uint4 r[8];
+  // The rows of the wave's 64 candidates: load g takes rows 8 g .. 8 g + 7, eight lanes a row,
+  // lane `sub` its pieces p0 + sub (the last piece past the row's end; row 0 where none is).
+  auto load_rows = [&](uint32_t t, uint32_t p0) {
+    const uint32_t piece = p0 + sub < pieces ? p0 + sub : pieces - 1;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      if (!found && p < n[i]) at = lo[i] + p, found = true;
-      if (!found) p -= n[i];
+    for (uint32_t g = 0; g < 8; g++) {
+      const uint32_t id = (uint32_t)__shfl((int)t, (int)(8 * g + grp), 64);
+      r[g] = ((const uint4 *)(table + (uint64_t)(id == kAbsent ? 0 : id) * width))[piece];
     }
-    const uint32_t t = members[at];
-    if (t >= count) {
-      bad = true;
-      continue;
+  };
+  Best8 best;
+  uint32_t tok = next_member();
+  load_rows(tok, 0);
+  uint32_t tok_next = next_member();
+  uint4 *const st = stage[wave];
+  for (uint32_t j = 0; j < total; j += 64) {
+    uint64_t dist = 0;
+    for (uint32_t p0 = 0; p0 < pieces; p0 += 8) {
+      // Row 8 g + grp's piece `sub` goes to place sub ^ grp of the row (grp = row mod 8).
+#pragma unroll
+      for (uint32_t g = 0; g < 8; g++) {
+        uint4 v = r[g];
+        v.x ^= 0x80000000u, v.y ^= 0x80000000u, v.z ^= 0x80000000u, v.w ^= 0x80000000u;
+        st[8 * (8 * g + grp) + (sub ^ grp)] = v;
+      }
+      wave_sync();
+      if (p0 + 8 < pieces)
+        load_rows(tok, p0 + 8);
+      else
+        load_rows(tok_next, 0);
+      const uint32_t here = pieces - p0 < 8 ? pieces - p0 : 8;
+      const uint4 *q = (const uint4 *)(sq[wave]) + p0;
+      if (here == 8) {
+#pragma unroll
+        for (uint32_t s = 0; s < 8; s++) {
+          const uint4 a = st[8 * lane + (s ^ (lane & 7))], b = q[s];
+          dist = sad_add(dist, a.x, b.x);
+          dist = sad_add(dist, a.y, b.y);
+          dist = sad_add(dist, a.z, b.z);
+          dist = sad_add(dist, a.w, b.w);
+        }
+      } else {
+        for (uint32_t s = 0; s < here; s++) {
+          const uint4 a = st[8 * lane + (s ^ (lane & 7))], b = q[s];
+          dist = sad_add(dist, a.x, b.x);
+          dist = sad_add(dist, a.y, b.y);
+          dist = sad_add(dist, a.z, b.z);
+          dist = sad_add(dist, a.w, b.w);
+        }
+      }
+      wave_sync();
     }
-    best.add(row_l1(sq[wave], table + (uint64_t)t * width, width), t);
+    best.take(dist, tok, tok != kAbsent);
+    tok = tok_next;
+    tok_next = next_member();
   }
-  uint32_t out[8];
-  int64_t dist[8];
-  best.wave_best(out, dist);
   bad = __any(bad);
-  if (row < rows && lane == 0) {
-    predictions[row] = out[0];
+  if (row < rows) {
+    if (lane < 8) top8[(uint64_t)row * 8 + lane] = best.t;
+    uint32_t mine = adm[0];
 #pragma unroll
-    for (int i = 0; i < 8; i++) top8[(uint64_t)row * 8 + i] = out[i];
-#pragma unroll
-    for (int i = 0; i < 16; i++) admitted[(uint64_t)row * 16 + i] = adm[i];
-    status[row] = bad ? kCsr : out[0] == kAbsent ? kInvalid : kOk;
+    for (int i = 1; i < 16; i++) mine = lane == (uint32_t)i ? adm[i] : mine;
+    if (lane < 16) admitted[(uint64_t)row * 16 + lane] = mine;
+    if (lane == 0) {
+      predictions[row] = best.t;
+      status[row] = bad ? kCsr : best.t == kAbsent ? kInvalid : kOk;
+    }
   }
 }
 
