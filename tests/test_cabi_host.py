@@ -472,3 +472,52 @@ def test_norm_factor_pow2_at_its_edges(hp):
     eps = np.array([v for v in vals if 0 < v < 2**63], dtype=np.int64)
     sums = np.zeros(len(eps), np.uint64)
     assert hp.fbs_hp_norm_factor_check(sums.ctypes.data_as(P), eps.ctypes.data_as(P), len(eps), 5) == 0
+
+
+def test_norm_factor_direct_and_the_32bit_apply_equal_the_general_forms(hp):
+    # The kernels' first form of the RMSNorm factor (refused inputs go to norm_factor_wave): exact
+    # wherever it accepts, and it accepts what usual activations give; sums on and next to the
+    # squares where the factor's floor moves; then the 32-bit normalised value against the general
+    # one at every mean square it is taken for, with the largest entry that a sum allows.
+    direct = hp.fbs_hp_norm_factor_direct_check
+    direct.argtypes = [P, P, C.c_uint64, C.c_uint32, P]
+    direct.restype = C.c_uint64
+    apply32 = hp.fbs_hp_norm_apply32_check
+    apply32.argtypes = [P, P, P, C.c_uint64, C.c_uint32, P]
+    apply32.restype = C.c_uint64
+    rng = np.random.default_rng(131)
+    no = C.c_uint64()
+
+    def run(f, log2n, *arrays):
+        n = len(arrays[0])
+        assert f(*[np.ascontiguousarray(a).ctypes.data_as(P) for a in arrays], n, log2n, C.byref(no)) == 0
+        return no.value / n
+
+    for log2n in (5, 8, 10):
+        for bits in range(28, 62):
+            ms = rng.integers(1 << (bits - 1), 1 << bits, 20000, dtype=np.uint64)
+            refused = run(direct, log2n, np.minimum(ms, np.uint64(1 << (63 - log2n))) << np.uint64(log2n),
+                          np.zeros(len(ms), np.int64))
+            if 38 <= bits <= 48:
+                assert refused < 0.02, bits
+        # Mean squares around (2^62 / r)^2: R passes an integer there.
+        r = rng.integers(1 << 33, 1 << 47, 60000, dtype=np.int64)
+        near = np.array([((1 << 124) // (int(v) * int(v))) for v in r], dtype=np.int64)
+        near = np.concatenate([near + k for k in (-1, 0, 1)])
+        near = near[(near >= 1 << 30) & (near < 1 << 50)]
+        run(direct, log2n, near.astype(np.uint64) << np.uint64(log2n), np.zeros(len(near), np.int64))
+        run(direct, log2n, np.zeros(len(near), np.uint64), near)
+    edge = [v + k for b in range(1, 61) for v in (1 << b,) for k in (-1, 0, 1)] + [1, 2, 3]
+    edge = np.array([v for v in edge if v > 0], np.int64)
+    run(direct, 8, np.zeros(len(edge), np.uint64), edge)
+    for log2n in (5, 8, 10):
+        n = 200000
+        y = (rng.integers(0, (1 << 24) + 1, n) >> rng.integers(0, 25, n)).astype(np.int64)
+        rest = (rng.integers(0, 1 << 48, n) >> rng.integers(0, 49, n)).astype(np.int64)
+        rest[: n // 4] = 0  # all of the sum in one entry
+        sums = (y * y + rest).astype(np.uint64)
+        y = np.where(rng.random(n) < 0.5, y, -y).astype(np.int32)
+        eps = rng.choice(np.array([0, 1, 42950, 1 << 20, 1 << 40, 1 << 58, (1 << 59) - 1, 1 << 60, 1 << 62],
+                                  dtype=np.int64), n)
+        refused = run(apply32, log2n, sums, eps, y)
+        assert refused < 0.5

@@ -694,8 +694,8 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
         if (td[i] == kGridDescSlow) M.taps_fast = 0;
       }
       for (uint32_t i = 0; i < d; i++) {
-        rg[i] = grid_desc(ly.rec_gain[i]);
-        mg[i] = grid_desc(ly.mlp_gain[i]);
+        rg[i] = tap_desc(ly.rec_gain[i]);
+        mg[i] = tap_desc(ly.mlp_gain[i]);
         if (rg[i] == kGridDescSlow || mg[i] == kGridDescSlow) M.gains_fast = 0;
       }
       if ((st = h->upload(td.data(), td.size(), &dl.taps_desc))) return done(st);
@@ -736,7 +736,7 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
   {
     std::vector<uint16_t> fg(d);
     for (uint32_t i = 0; i < d; i++) {
-      fg[i] = grid_desc(m->final_gain[i]);
+      fg[i] = tap_desc(m->final_gain[i]);
       if (fg[i] == kGridDescSlow) M.gains_fast = 0;
     }
     if ((st = h->upload(fg.data(), fg.size(), &M.final_gain_desc))) return done(st);

@@ -3,7 +3,7 @@
 //
 // Layout in HBM (all tables uploaded once by uor_fbs_model_create, read by every sequence):
 //   per layer: gains (d i16), window taps ((W+1) x d i16, tap s = s positions back) and their
-//              descriptor forms (grid_desc for gains, tap_desc for taps; fbs_int.h),
+//              descriptor forms (tap_desc; fbs_int.h),
 //              conv_bias (d i32), gate_bias (d/4 + d i32), decay_offset (d/4 i32), and the
 //              layer's gather program: [slot][64 lanes] u16 LDS word indices that carry out the
 //              six FBS projections (stack_fbs_gather, session.rs:4037-4053) for this lane mapping;
@@ -103,7 +103,7 @@ struct DevModel {
   uint32_t xbar_words;      // 2 * max(d, m)
   uint32_t identity_rows;   // the nearest head: one drawer holding every token
   uint32_t taps_fast;       // every window tap has a descriptor (tap_desc != kGridDescSlow)
-  uint32_t gains_fast;      // every norm gain (rec, mlp, final) has a descriptor (grid_desc)
+  uint32_t gains_fast;      // every norm gain (rec, mlp, final) has a descriptor (tap_desc)
   uint32_t log2d;           // log2(d) when d is a power of two, else 0xff
   uint32_t writer_memory;   // 1: a query equal to the writer's last one takes its result
   uint64_t w_recip;         // floor(2^32 / W): the ring slot of a position without division

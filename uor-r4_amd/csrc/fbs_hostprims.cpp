@@ -98,27 +98,65 @@ uint64_t fbs_hp_recip_q63(uint32_t d) { return recip_q63(d); }
 
 int64_t fbs_hp_shift(int64_t v, int32_t s) { return shift(v, s); }
 int64_t fbs_hp_grid_apply(int64_t v, int16_t code) { return grid_apply(v, code); }
-int64_t fbs_hp_grid32_desc(int32_t v, int16_t code) { return grid_apply32_desc(v, grid_desc(code), code); }
-int64_t fbs_hp_grid64_desc(int64_t v, int16_t code) { return grid_apply64_desc(v, grid_desc(code), code); }
 
-// Every valid grid code against n inputs v[]: mismatches of the descriptor forms (the gains'
-// grid_desc forms, and the taps' tap_desc form in both halves of a word).
+// Every valid grid code against n inputs v[] (their low 32 bits): mismatches of the descriptor
+// form in both halves of a word, and of the gained norms' publish from its unhalved value.
 uint64_t fbs_hp_grid_check(const int64_t *v, uint64_t n) {
   uint64_t bad = 0;
   for (int32_t code = -2047; code <= 2047; code++) {
     uint32_t field = (uint32_t)(code < 0 ? -code : code) >> 4;
     if (code != 0 && (field < 1 || field > 127)) continue;
-    uint16_t d = grid_desc((int16_t)code);
     uint16_t t = tap_desc((int16_t)code);
+    if (t == kGridDescSlow) continue;
     const uint32_t word0 = 0xa5a50000u | t, word1 = ((uint32_t)t << 16) | 0x5a5au;
     for (uint64_t i = 0; i < n; i++) {
-      bad += grid_apply64_desc(v[i], d, (int16_t)code) != grid_apply(v[i], (int16_t)code);
       int32_t v32 = (int32_t)v[i];
       const int64_t want = grid_apply((int64_t)v32, (int16_t)code);
-      bad += grid_apply32_desc(v32, d, (int16_t)code) != want;
-      if (t != kGridDescSlow) bad += (tap_desc_apply(v32, word0, 0) != want) + (tap_desc_apply(v32, word1, 1) != want);
+      bad += (tap_desc_apply(v32, word0, 0) != want) + (tap_desc_apply(v32, word1, 1) != want);
+      const int64_t h = tap_desc_half(v32, word1, 1);
+      bad += ((h + 1) >> 1 != want) + (tap_desc_half(v32, word0, 0) != h);
+      int32_t p, q;
+      publish_half_pair(h, &p, &q);
+      bad += p != to_exp_i32(want, kNormFineExp, kResidualExp);
+      bad += q != to_exp_i32(sat_neg64(want), kNormFineExp, kResidualExp);
     }
   }
+  return bad;
+}
+
+// norm_factor_direct against norm_factor on n (sum, eps) pairs at 2^log2n: mismatches among the
+// inputs it accepts, and in *refused those it sends to the fallback.
+uint64_t fbs_hp_norm_factor_direct_check(const uint64_t *sum, const int64_t *eps, uint64_t n,
+                                         uint32_t log2n, uint64_t *refused) {
+  uint64_t bad = 0, no = 0;
+  for (uint64_t i = 0; i < n; i++) {
+    uint64_t r;
+    if (!norm_factor_direct(sum[i], log2n, eps[i], Seeds(), r)) {
+      no++;
+      continue;
+    }
+    const NormFactor a = norm_factor(sum[i], 1u << log2n, eps[i]);
+    bad += a.huge || a.r != r;
+  }
+  *refused = no;
+  return bad;
+}
+
+// norm_apply32 against norm_apply24 on n (sum, eps, y) at 2^log2n (y^2 <= sum) where norm_fits32
+// holds: mismatches; *refused: where it does not hold.
+uint64_t fbs_hp_norm_apply32_check(const uint64_t *sum, const int64_t *eps, const int32_t *y,
+                                   uint64_t n, uint32_t log2n, uint64_t *refused) {
+  uint64_t bad = 0, no = 0;
+  for (uint64_t i = 0; i < n; i++) {
+    const NormFactor f = norm_factor(sum[i], 1u << log2n, eps[i]);
+    if (!norm_fits32(f, sum[i], log2n, eps[i])) {
+      no++;
+      continue;
+    }
+    const int32_t v = norm_apply32((int32_t)(f.r & 0x7fffffffu), (int32_t)(f.r >> 31), y[i]);
+    bad += v != norm_apply24(f, y[i]) || v > INT32_MAX - 1 || v < -INT32_MAX;
+  }
+  *refused = no;
   return bad;
 }
 

@@ -108,34 +108,15 @@ FBS_HD int64_t grid_apply(int64_t v, int16_t code) {
 // The same for a 32-bit input, whose product (16 + m) v never wraps.
 FBS_HD int64_t grid_apply32(int32_t v, int16_t code) { return grid_apply((int64_t)v, code); }
 
-// A grid code prepared for the kernels (16 bits): bits 0-5 the multiplier 16 + m (0 for the zero
-// code), bit 6 the sign, bits 7-12 the right shift sh = 4 - e. With the sign folded in,
-// grid_apply(v, code) = (v (+-(16 + m)) + 2^(sh-1) - [code < 0]) >> sh, because
-// -floor((p + 2^(sh-1)) / 2^sh) = floor((-p + 2^(sh-1) - 1) / 2^sh). The form holds whenever
-// 1 <= sh <= 62 and |v| (16 + m) + 2^(sh-1) < 2^63: always for a 32-bit v, and for a 64-bit v
-// below 2^57 in magnitude. `grid_desc` returns kGridDescSlow for a code outside 1 <= sh <= 62.
+// A grid code prepared for the kernels (16 bits, two per word), for the window taps and the norms'
+// gains. kGridDescSlow marks a code whose right shift sh = 4 - e lies outside 1..62.
 constexpr uint16_t kGridDescSlow = 0xffff;
 
-FBS_HD uint16_t grid_desc(int16_t code) {
-  if (code == 0) return (uint16_t)(1u << 7);  // multiplier 0, shift 1: (0 + 1) >> 1 = 0
-  uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
-  int32_t sh = 4 - ((int32_t)(c >> 4) - kGridExpBias);
-  if (sh < 1 || sh > 62) return kGridDescSlow;
-  return (uint16_t)((16 + (c & 15)) | (code < 0 ? 64u : 0u) | ((uint32_t)sh << 7));
-}
-
-FBS_HD int64_t grid_desc_apply(int64_t v, uint16_t desc) {
-  const int32_t mag = desc & 63, neg = (desc >> 6) & 1;
-  const uint32_t sh = (desc >> 7) & 63;
-  const int32_t mul = (mag ^ -neg) + neg;
-  return (v * mul + (((int64_t)1 << (sh - 1)) - neg)) >> sh;
-}
-
-// The window taps' descriptor (16 bits, two per word): bits 0-5 the signed multiplier
+// Bits 0-5 the signed multiplier
 // +-(16 + m) (0 for the zero code), bits 6-11 the shift sh - 1. For a 32-bit v, with
 // p = v mul and neg = [code < 0] (the multiplier's sign bit),
 // grid_apply(v, code) = floor((p - neg + 2^(sh-1)) / 2^sh) = ((p - neg) >> (sh - 1)) + 1) >> 1.
-// Valid for the codes grid_desc serves (1 <= sh <= 62); |p| < 2^36.
+// Valid for the codes with 1 <= sh <= 62; |p| < 2^36.
 FBS_HD uint16_t tap_desc(int16_t code) {
   if (code == 0) return 0;  // multiplier 0, shift 1: ((0 >> 0) + 1) >> 1 = 0
   const uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
@@ -153,20 +134,11 @@ FBS_HD int64_t tap_desc_apply(int32_t v, uint32_t word, int h) {
   return ((p >> shm1) + 1) >> 1;
 }
 
-// grid_apply for a 32-bit input through its descriptor (every valid code has one or is slow).
-FBS_HD int64_t grid_apply32_desc(int32_t v, uint16_t desc, int16_t code) {
-  if (desc == kGridDescSlow) return grid_apply((int64_t)v, code);
-  const int32_t mag = desc & 63, neg = (desc >> 6) & 1;
-  const uint32_t sh = (desc >> 7) & 63;
-  const int32_t mul = (mag ^ -neg) + neg;
-  return ((int64_t)v * (int64_t)mul + (((int64_t)1 << (sh - 1)) - neg)) >> sh;
-}
-
-// grid_apply for a 64-bit input: the descriptor form below 2^57, the reference routine above.
-FBS_HD int64_t grid_apply64_desc(int64_t v, uint16_t desc, int16_t code) {
-  if (desc == kGridDescSlow || v >= ((int64_t)1 << 57) || v <= -((int64_t)1 << 57))
-    return grid_apply(v, code);
-  return grid_desc_apply(v, desc);
+// The floor before the last halving of tap_desc_apply: grid_apply(v, code) = (h + 1) >> 1.
+FBS_HD int64_t tap_desc_half(int32_t v, uint32_t word, int h) {
+  const int32_t mul = (int32_t)(word << (26 - 16 * h)) >> 26;
+  const uint32_t shm1 = (word >> (16 * h + 6)) & 63u;
+  return ((int64_t)v * mul + (mul >> 31)) >> shm1;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -620,6 +592,57 @@ FBS_HD NormFactor norm_factor_wave(uint64_t sum, uint32_t log2n, int64_t eps_int
   return out;
 }
 
+// norm_factor_pow2 where the factor's real value decides its floor: with m = ms in [2^30, 2^59],
+// r = floor(2^96 / s) for s = floor(2^34 sqrt(m)), and 2^96 / s exceeds R = 2^62 / sqrt(m) by less
+// than 2^28 / m. R 2^w comes from the 32-bit reciprocal square root y ~ 2^62 / sqrt(mn)
+// (mn = m 2^(4 + z) in [2^62, 2^64), relative error below 2^-28.6 with mn's truncation to mt) by one
+// Newton step, y (1 + E / 2) with E = 1 - y^2 mn / 2^124: rq = 2^86 / sqrt(mn) = R 2^(22 - z / 2)
+// within (-1.4, +0.1] (the step's own error is below 1.5 2^-57.2 of it, that of E's top 31 bits
+// below 2^-59). Its integer part is r unless its fraction lies within 1 of 0, or within 2 and the
+// 2^28 / m (at most 2^(z / 2 - 8) of its units) of the next integer: then, or for another m, false
+// and the caller takes norm_factor_wave (0.7 % of the inputs near m = 2^36, 27 % just above 2^30).
+FBS_HD bool norm_factor_direct(uint64_t sum, uint32_t log2n, int64_t eps_int, const Seeds &sd,
+                               uint64_t &r) {
+  const uint64_t ms = (sum >> log2n) + (uint64_t)eps_int;
+  if (ms - (1ull << 30) >= (1ull << 59) - (1ull << 30)) return false;
+  const uint64_t M = ms << 4;
+  const int z = clz64(M) & ~1;                        // [0, 28]
+  const uint64_t mn = M << z;
+  const uint32_t mt = (uint32_t)(mn >> 32), ml = (uint32_t)mn;
+  const uint32_t y = rsqrt_q46(mt, sd.rsq_seed);
+  const uint64_t y2 = (uint64_t)y * y;
+  const uint32_t yh = (uint32_t)(y2 >> 32), yl = (uint32_t)y2;
+  const uint64_t p = (uint64_t)yh * mt + ((uint64_t)mulhi32(yh, ml) + mulhi32(yl, mt));  // y^2 mn / 2^64
+  const int32_t e = (int32_t)((int64_t)((1ull << 60) - p) >> 2);
+  const uint64_t rq = ((uint64_t)y << 24) + (uint64_t)(((int64_t)e * (int64_t)(uint64_t)y) >> 35);
+  const int w = 22 - (z >> 1);                        // [8, 22]
+  r = rq >> w;
+  const uint32_t frac = (uint32_t)rq & ((1u << w) - 1), slack = 3 + ((1u << (z >> 1)) >> 8);
+  return frac - 2 < (1u << w) - 2 - slack;            // 2 <= frac < 2^w - slack
+}
+
+// The normalised value in 32 bits, round(r y / 2^38) for |y| <= 2^24 and r = hi 2^31 + lo < 2^62
+// where it fits (norm_fits32): floor((r y + 2^37) / 2^38) from two 32 x 32 products.
+FBS_HD int32_t norm_apply32(int32_t lo, int32_t hi, int32_t y) {
+  const int64_t a = (int64_t)y * lo + (1ll << 37);
+  return (int32_t)(((int64_t)y * hi + (a >> 31)) >> 7);
+}
+// Whether every |round(r y / 2^38)| is below 2^31 - 1: r < 2^44 with |y| <= 2^24; or the mean square
+// ms = floor(sum / n) + eps taken as it is (eps >= 0, below the 60-bit mask), r in two 31-bit
+// parts: y^2 <= sum < 2 n ms,
+// so the value stays below sqrt(2 n) 2^24 + 1 <= 2^29.6 for n <= 1024.
+FBS_HD bool norm_fits32(NormFactor f, uint64_t sum, uint32_t log2n, int64_t eps_int) {
+  return !f.huge && (f.r < (1ull << 44) || ((sum >> log2n) + (uint64_t)eps_int - 1 < (1ull << 59) - 1 &&
+                                            f.r < (1ull << 62)));
+}
+// to_exp_i32(g, -24, -16) and to_exp_i32(-g, -24, -16) of a gained value g = (h + 1) >> 1 with
+// |h| < 2^38 (both fit 32 bits, so nothing clamps): floor((g + 128) / 2^8) = floor((h + 257) / 2^9)
+// and floor((128 - g) / 2^8) = floor((256 - h) / 2^9).
+FBS_HD void publish_half_pair(int64_t h, int32_t *p, int32_t *n) {
+  *p = (int32_t)((h + 257) >> 9);
+  *n = (int32_t)((256 - h) >> 9);
+}
+
 // One normalised value: round(r y / 2^38) with the sign of y, clamped to i64.
 FBS_HD int64_t norm_apply(NormFactor f, int64_t y) {
   uint64_t u = uabs64(y);
@@ -631,17 +654,10 @@ FBS_HD int64_t norm_apply(NormFactor f, int64_t y) {
   return (int64_t)r;
 }
 
-// norm_apply for |y| < 2^24 (every pre-shifted norm input) and r < 2^62 (every factor but the
+// norm_apply for |y| <= 2^24 (every pre-shifted norm input) where r < 2^62 (every factor but the
 // huge one): with P = r |y| = A + B 2^32 (A = r_lo |y|, B = r_hi |y|), floor((P + h) / 2^38) =
 // floor((B + floor((A + h) / 2^32)) / 2^6); h = 2^37 for y >= 0, 2^37 - 1 for the negated form
 // (floor((-P + 2^37) / 2^38) = -floor((P + 2^37 - 1) / 2^38)).
-FBS_HD int64_t norm_apply24_fast(NormFactor f, int64_t y) {
-  const uint32_t u = (uint32_t)(y < 0 ? -y : y);
-  const uint64_t A = (uint64_t)(uint32_t)f.r * u, B = (f.r >> 32) * (uint64_t)u;
-  const uint64_t h = y < 0 ? (1ull << 37) - 1 : (1ull << 37);
-  const int64_t mag = (int64_t)((B + ((A + h) >> 32)) >> 6);
-  return y < 0 ? -mag : mag;
-}
 FBS_HD int64_t norm_apply24(NormFactor f, int64_t y) {
   if (f.huge) return norm_apply(f, y);
   const uint32_t u = (uint32_t)(y < 0 ? -y : y);

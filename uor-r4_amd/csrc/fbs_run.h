@@ -99,20 +99,6 @@ __device__ __forceinline__ uint64_t wave_reduce64(uint64_t v, Op op) {
   v = op(v, dpp64<kDppMirror>(v));
   return op(op(lane64(v, 0), lane64(v, 16)), op(lane64(v, 32), lane64(v, 48)));
 }
-// The wave's maximum of m and sum of s together, both returned uniform: each exchange step is
-// applied to both before the next, so one reduction's DPP waits are filled with the other's work.
-__device__ __forceinline__ void wave_max32_add64(uint32_t &m, uint64_t &s) {
-  m = OpMax()(m, dpp32<kDppXor1>(m));
-  s += dpp64<kDppXor1>(s);
-  m = OpMax()(m, dpp32<kDppXor2>(m));
-  s += dpp64<kDppXor2>(s);
-  m = OpMax()(m, dpp32<kDppHalfMirror>(m));
-  s += dpp64<kDppHalfMirror>(s);
-  m = OpMax()(m, dpp32<kDppMirror>(m));
-  s += dpp64<kDppMirror>(s);
-  m = OpMax()(OpMax()(lane32(m, 0), lane32(m, 16)), OpMax()(lane32(m, 32), lane32(m, 48)));
-  s = (lane64(s, 0) + lane64(s, 16)) + (lane64(s, 32) + lane64(s, 48));
-}
 // The bit length of the wave's largest magnitude from each lane's largest: the bit length of a
 // maximum is the maximum of the bit lengths, so a 32-bit reduction takes the place of a 64-bit one.
 __device__ __forceinline__ int32_t wave_bitlen_max(uint64_t v) {
@@ -198,12 +184,11 @@ __device__ __noinline__ NormFactor norm_factor_lds(uint64_t sum, uint32_t log2n,
   if (!ok) f = norm_factor_pow2(sum, log2n, eps, sd);
   return f;
 }
-__device__ __noinline__ int64_t norm_gain_slow(uint64_t r, uint32_t huge, int64_t y, uint32_t desc,
-                                               int32_t code) {
+__device__ __noinline__ int64_t norm_gain_slow(uint64_t r, uint32_t huge, int64_t y, int32_t code) {
   NormFactor f;
   f.r = r;
   f.huge = huge != 0;
-  return grid_apply64_desc(norm_apply24(f, y), (uint16_t)desc, (int16_t)code);
+  return grid_apply(norm_apply24(f, y), (int16_t)code);
 }
 // shift_wide(mh 2^32 + ml + (keep wide) << 16, 31) (raw: the split form of hamilton32_hl) or of
 // (mh 2^64 + ml) + (keep wide) << 16 (a snapped transition's i128).
@@ -218,85 +203,123 @@ __device__ __noinline__ int64_t gate_wide14(int64_t gh, int64_t gl) {
   return shift_wide(((i128)gh << 32) + (i128)gl, 14);
 }
 
-// Fine RMSNorm then the per-channel grid gain, for the lane's channels
-// (RS stack/kernels.rs:569-620, session.rs:4057-4061). gain: the lane's 4 codes per quaternion.
+// The norm's factor over the lane's channels: y their pre-shifted values (|y| <= 2^24), f the
+// factor. Returns whether the gained values may be formed in the 32-bit form (norm_fits32 and every
+// gain has a descriptor): the common case, one uniform branch.
+// Bound by the instructions on the wave's serial chain, about 5 cycles each whatever they are: the
+// factor takes its real-valued form (about 75 instructions; norm_factor_wave's three rounds of
+// candidates take 205 and a call), and the largest magnitude is looked at only where a square
+// reaches 2^48.
 template <int Q>
-__device__ __forceinline__ void norm_gain(const DevModel &M, const Seeds &sd,
-                                          const int32_t (&x)[Q][4], const bool (&qv)[Q],
-                                          const short4 (&gain)[Q], const ushort4 (&gdesc)[Q],
-                                          int64_t (&out)[Q][4]) {
-  // The largest magnitude and, beside it, the sum of squares as if the pre-shift were 0 (it is
-  // wherever the largest magnitude is below 2^24, and then every square is below 2^48): both
-  // reductions run interleaved, and only a non-zero pre-shift sums the shifted values again.
-  uint32_t mx = 0;
+__device__ __forceinline__ bool norm_scale(const DevModel &M, const Seeds &sd, const int32_t (&x)[Q][4],
+                                           int32_t (&y)[Q][4], NormFactor &f) {
+  // The sum of squares as if the pre-shift were 0 (it is wherever every magnitude is below 2^24). A
+  // pair's sum fits 64 bits, and a magnitude of 2^24 shows in its high word.
   uint64_t sum = 0;
+  uint32_t high = 0;
 #pragma unroll
-  for (int k = 0; k < Q; k++)
-    if (qv[k])
+  for (int k = 0; k < Q; k++) {
+    const uint64_t a = (uint64_t)((int64_t)x[k][0] * x[k][0]) + (uint64_t)((int64_t)x[k][1] * x[k][1]);
+    const uint64_t b = (uint64_t)((int64_t)x[k][2] * x[k][2]) + (uint64_t)((int64_t)x[k][3] * x[k][3]);
+    high |= (uint32_t)(a >> 32) | (uint32_t)(b >> 32);
+    sum += a + b;
+#pragma unroll
+    for (int c = 0; c < 4; c++) y[k][c] = x[k][c];
+  }
+  int64_t eps = M.eps0;
+  if (__any(high >> 16)) {
+    uint32_t mx = 0;
+#pragma unroll
+    for (int k = 0; k < Q; k++)
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const uint32_t a = uabs32(x[k][c]);
         mx = a > mx ? a : mx;
-        sum += (uint64_t)a * a;  // used only when every a < 2^24
       }
-  wave_max32_add64(mx, sum);
-  int32_t sh = bitlen64(mx) - 24;
-  if (sh < 0) sh = 0;
-#pragma unroll
-  for (int k = 0; k < Q; k++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) out[k][c] = qv[k] ? (int64_t)x[k][c] : 0;
-  if (sh > 0) {
+    int32_t sh = bitlen64(wave_reduce32(mx, OpMax())) - 24;
+    if (sh < 0) sh = 0;
+    if (sh > 0) eps = M.eps_int[sh];
     sum = 0;
 #pragma unroll
     for (int k = 0; k < Q; k++)
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        const int64_t y = qv[k] ? shift((int64_t)x[k][c], sh) : 0;
-        out[k][c] = y;
-        const uint32_t a = (uint32_t)uabs64(y);  // |y| <= 2^24: the shift leaves 24 bits
+        const int32_t v = (int32_t)shift((int64_t)x[k][c], sh);
+        y[k][c] = v;
+        const uint32_t a = uabs32(v);  // |v| <= 2^24: the shift leaves 24 bits
         sum += (uint64_t)a * a;
       }
-    sum = wave_reduce64(sum, OpAdd());
   }
-  const int64_t eps = sh == 0 ? M.eps0 : M.eps_int[sh];
-  const NormFactor f = M.log2d != 0xffu ? norm_factor_lds(sum, M.log2d, eps, (lds_u32 *)sd.rsq_seed)
-                                         : norm_factor_slow(sum, M.d, eps);
-  if (!f.huge && M.gains_fast) {
-    // The common case, one uniform branch: r < 2^62 and |y| <= 2^24 keep every normed value
-    // below 2^48 in magnitude, where each gain's descriptor form is exact.
+  sum = wave_reduce64(sum, OpAdd());
+  f.huge = false;
+  if (M.log2d != 0xffu) {
+    if (__all(norm_factor_direct(sum, M.log2d, eps, sd, f.r))) return M.gains_fast;
+    f = norm_factor_lds(sum, M.log2d, eps, (lds_u32 *)sd.rsq_seed);
+    return M.gains_fast && __all(norm_fits32(f, sum, M.log2d, eps));
+  }
+  f = norm_factor_slow(sum, M.d, eps);
+  return M.gains_fast && __all(!f.huge && f.r < (1ull << 44));
+}
+
+// Fine RMSNorm then the per-channel grid gain, for the lane's channels
+// (RS stack/kernels.rs:569-620, session.rs:4057-4061). gain: the lane's 4 codes per quaternion.
+template <int Q>
+__device__ __forceinline__ void norm_gain(const DevModel &M, const Seeds &sd,
+                                          const int32_t (&x)[Q][4], const short4 (&gain)[Q],
+                                          const uint2 (&gdesc)[Q], int64_t (&out)[Q][4]) {
+  int32_t y[Q][4];
+  NormFactor f;
+  if (norm_scale<Q>(M, sd, x, y, f)) {
+    const int32_t lo = (int32_t)(f.r & 0x7fffffffu), hi = (int32_t)(f.r >> 31);
 #pragma unroll
-    for (int k = 0; k < Q; k++) {
-      const uint16_t gd[4] = {gdesc[k].x, gdesc[k].y, gdesc[k].z, gdesc[k].w};
+    for (int k = 0; k < Q; k++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) out[k][c] = grid_desc_apply(norm_apply24_fast(f, out[k][c]), gd[c]);
-    }
+      for (int c = 0; c < 4; c++)
+        out[k][c] = tap_desc_apply(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1);
     return;
   }
 #pragma unroll
   for (int k = 0; k < Q; k++) {
     const int16_t gc[4] = {gain[k].x, gain[k].y, gain[k].z, gain[k].w};
-    const uint16_t gd[4] = {gdesc[k].x, gdesc[k].y, gdesc[k].z, gdesc[k].w};
 #pragma unroll
-    for (int c = 0; c < 4; c++) out[k][c] = norm_gain_slow(f.r, f.huge, out[k][c], gd[c], gc[c]);
+    for (int c = 0; c < 4; c++) out[k][c] = norm_gain_slow(f.r, f.huge, y[k][c], gc[c]);
   }
 }
 
-// Publish v (exponent -24) for the FBS gathers: word 2 i + s holds to_exp_i32 of v_i (s = 0)
-// or of its saturating negation (s = 1), at exponent -16 (session.rs:4037-4053: the negation
-// comes before the rounding shift).
+// The norm and gain published for the FBS gathers: word 2 i + s holds to_exp_i32 of the gained
+// value v_i at exponent -24 (s = 0) or of its saturating negation (s = 1), at exponent -16
+// (session.rs:4037-4053: the negation comes before the rounding shift).
 template <int Q>
-__device__ __forceinline__ void publish64(int32_t *xbar, const int64_t (&v)[Q][4],
-                                          const bool (&qv)[Q], const uint32_t (&qi)[Q]) {
+__device__ __forceinline__ void norm_publish(const DevModel &M, const Seeds &sd,
+                                             const int32_t (&x)[Q][4], const bool (&qv)[Q],
+                                             const uint32_t (&qi)[Q], const short4 (&gain)[Q],
+                                             const uint2 (&gdesc)[Q], int32_t *xbar) {
+  int32_t y[Q][4];
+  NormFactor f;
+  const bool fast = norm_scale<Q>(M, sd, x, y, f);
+  int32_t p[Q][4], n[Q][4];
+  if (fast) {
+    const int32_t lo = (int32_t)(f.r & 0x7fffffffu), hi = (int32_t)(f.r >> 31);
+#pragma unroll
+    for (int k = 0; k < Q; k++)
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        publish_half_pair(tap_desc_half(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1),
+                          &p[k][c], &n[k][c]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < Q; k++) {
+      const int16_t gc[4] = {gain[k].x, gain[k].y, gain[k].z, gain[k].w};
+#pragma unroll
+      for (int c = 0; c < 4; c++) publish64_pair(norm_gain_slow(f.r, f.huge, y[k][c], gc[c]), &p[k][c], &n[k][c]);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < Q; k++)
     if (qv[k]) {
-      int32_t p[4], n[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) publish64_pair(v[k][c], &p[c], &n[c]);
       int4 *dst = (int4 *)(xbar + 8 * qi[k]);
-      dst[0] = make_int4(p[0], n[0], p[1], n[1]);
-      dst[1] = make_int4(p[2], n[2], p[3], n[3]);
+      dst[0] = make_int4(p[k][0], n[k][0], p[k][1], n[k][1]);
+      dst[1] = make_int4(p[k][2], n[k][2], p[k][3], n[k][3]);
     }
 }
 
@@ -974,7 +997,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     // The layer's loads first: gains, biases and the gather program.
     short4 g_rec[Q], g_mlp[Q], tap0[Q];
-    ushort4 gd_rec[Q], gd_mlp[Q];
+    uint2 gd_rec[Q], gd_mlp[Q];
     uint2 td0[Q];
     int4 cbias[Q], rbias[Q];
     int32_t dbias[Q], doff[Q];
@@ -985,8 +1008,8 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       g_rec[k] = *(const short4 *)(ly.rec_gain + ch);
       g_mlp[k] = *(const short4 *)(ly.mlp_gain + ch);
       tap0[k] = *(const short4 *)(ly.taps + ch);
-      gd_rec[k] = *(const ushort4 *)(ly.rec_gain_desc + ch);
-      gd_mlp[k] = *(const ushort4 *)(ly.mlp_gain_desc + ch);
+      gd_rec[k] = *(const uint2 *)(ly.rec_gain_desc + ch);
+      gd_mlp[k] = *(const uint2 *)(ly.mlp_gain_desc + ch);
       td0[k] = *(const uint2 *)(ly.taps_desc + ch);
       cbias[k] = *(const int4 *)(ly.conv_bias + ch);
       rbias[k] = *(const int4 *)(ly.gate_bias + nq + ch);
@@ -1003,9 +1026,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       pw_dec[k] = prog_word(ly.prog, M.s_rec_gate + k, lane);
     }
     // ---- recurrence block
-    int64_t v[Q][4];
-    norm_gain<Q>(M, S.seeds, x, qv, g_rec, gd_rec, v);
-    publish64<Q>(S.xbar, v, qv, qi);
+    norm_publish<Q>(M, S.seeds, x, qv, qi, g_rec, gd_rec, S.xbar);
     wave_sync();
     int32_t drive[Q][4], gv[Q][4], rot[Q][4], dec[Q];
 #pragma unroll
@@ -1168,8 +1189,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       pg[c] = prog_word(ly.prog, M.s_mlp_gate + c, lane);
       pu[c] = prog_word(ly.prog, M.s_mlp_up + c, lane);
     }
-    norm_gain<Q>(M, S.seeds, x, qv, g_mlp, gd_mlp, v);
-    publish64<Q>(S.xbar, v, qv, qi);
+    norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     wave_sync();
     uint64_t mmx = 0;
 #pragma unroll 1
@@ -1227,14 +1247,14 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
   }
   // Final norm, gain and the Q12 query (session.rs:4294-4295, 4364-4366).
   short4 g_fin[Q];
-  ushort4 gd_fin[Q];
+  uint2 gd_fin[Q];
 #pragma unroll
   for (int k = 0; k < Q; k++) {
     g_fin[k] = *(const short4 *)(M.final_gain + 4 * (qv[k] ? qi[k] : 0));
-    gd_fin[k] = *(const ushort4 *)(M.final_gain_desc + 4 * (qv[k] ? qi[k] : 0));
+    gd_fin[k] = *(const uint2 *)(M.final_gain_desc + 4 * (qv[k] ? qi[k] : 0));
   }
   int64_t v[Q][4];
-  norm_gain<Q>(M, S.seeds, x, qv, g_fin, gd_fin, v);
+  norm_gain<Q>(M, S.seeds, x, g_fin, gd_fin, v);
   if (HM) {  // the readout read on the final norm's output (session.rs:4296-4320)
     const int32_t r = M.ham.at[M.L];
     if (r >= 0) ham_readout<Q, DT>(M, M.ham.reads[r], (uint32_t)r, S, t, pay, lane, qv, qi, v, dc);
@@ -1490,7 +1510,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
   for (uint32_t l = 0; l < M.L; l++) {
     const DevLayer ly = M.layers[l];
     short4 g_rec[Q], g_mlp[Q];
-    ushort4 gd_rec[Q], gd_mlp[Q];
+    uint2 gd_rec[Q], gd_mlp[Q];
     int4 rbias[Q];
     int32_t dbias[Q], doff[Q];
     uint32_t pw_rot[Q][4], pw_dec[Q], pw_out[Q][4], pw_down[Q][4];
@@ -1502,7 +1522,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
       for (int k = 0; k < Q; k++) {
         const uint32_t ch = 4 * (qv[k] ? qi[k] : 0);
         g_mlp[k] = *(const short4 *)(ly.mlp_gain + ch);
-        gd_mlp[k] = *(const ushort4 *)(ly.mlp_gain_desc + ch);
+        gd_mlp[k] = *(const uint2 *)(ly.mlp_gain_desc + ch);
 #pragma unroll
         for (int c = 0; c < 4; c++) pw_down[k][c] = prog_word(ly.prog, M.s_mlp_down + 4 * k + c, lane);
       }
@@ -1511,7 +1531,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     for (int k = 0; k < Q; k++) {
       const uint32_t qq = qv[k] ? qi[k] : 0, ch = 4 * qq;
       g_rec[k] = *(const short4 *)(ly.rec_gain + ch);
-      gd_rec[k] = *(const ushort4 *)(ly.rec_gain_desc + ch);
+      gd_rec[k] = *(const uint2 *)(ly.rec_gain_desc + ch);
       rbias[k] = *(const int4 *)(ly.gate_bias + nq + ch);
       dbias[k] = ly.gate_bias[qq];
       doff[k] = ly.decay_offset[qq];
@@ -1524,9 +1544,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     }
     if constexpr (Q == 1) load_ffn();
     clk.lap(kPartLoads);
-    int64_t v[Q][4];
-    norm_gain<Q>(M, S.seeds, x, qv, g_rec, gd_rec, v);
-    publish64<Q>(S.xbar, v, qv, qi);
+    norm_publish<Q>(M, S.seeds, x, qv, qi, g_rec, gd_rec, S.xbar);
     // Two or more quaternions a lane keep the state in the block's global buffer (each lane its
     // own channels): its loads are issued here, to land during the barrier's wait.
     int64_t hg[Q][4];
@@ -1710,8 +1728,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     clk.lap(kPartResidualRec);
     // ---- feed-forward block: wave 0 takes the even quaternion groups.
     if constexpr (Q != 1) load_ffn();
-    norm_gain<Q>(M, S.seeds, x, qv, g_mlp, gd_mlp, v);
-    publish64<Q>(S.xbar, v, qv, qi);
+    norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     clk.sync(kPartNormMlp, kPartSync3);  // 3: the normed activations
     const uint64_t mbl = pair_mlp(M, S, ly, lane, 0, pg, pu);
     if (lane == 0) S.pair[0] = mbl;
@@ -1736,14 +1753,14 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
   if (!want_writer && !readout) return 0;
   // Final norm, gain and the Q12 query (session.rs:4294-4295, 4364-4366).
   short4 g_fin[Q];
-  ushort4 gd_fin[Q];
+  uint2 gd_fin[Q];
 #pragma unroll
   for (int k = 0; k < Q; k++) {
     g_fin[k] = *(const short4 *)(M.final_gain + 4 * (qv[k] ? qi[k] : 0));
-    gd_fin[k] = *(const ushort4 *)(M.final_gain_desc + 4 * (qv[k] ? qi[k] : 0));
+    gd_fin[k] = *(const uint2 *)(M.final_gain_desc + 4 * (qv[k] ? qi[k] : 0));
   }
   int64_t v[Q][4];
-  norm_gain<Q>(M, S.seeds, x, qv, g_fin, gd_fin, v);
+  norm_gain<Q>(M, S.seeds, x, g_fin, gd_fin, v);
   if constexpr (HM) {  // the readout read on the final norm's output (session.rs:4296-4320)
     if (readout) {
       const uint32_t r = (uint32_t)M.ham.at[M.L];
