@@ -521,3 +521,29 @@ def test_norm_factor_direct_and_the_32bit_apply_equal_the_general_forms(hp):
                                   dtype=np.int64), n)
         refused = run(apply32, log2n, sums, eps, y)
         assert refused < 0.5
+
+
+def test_fast_requantize_and_split_product_equal_the_general_forms(hp):
+    # The requantize's element form without saturation at every shift that holds the value, and the
+    # Hamilton product with the right operand's halves split once (everything but the top 2^31
+    # values of 64 bits, which it refuses).
+    q = hp.fbs_hp_quantize_fast_check
+    q.argtypes, q.restype = [P, C.c_uint64], C.c_uint64
+    rng = np.random.default_rng(177)
+    v = rng.integers(-2**63, 2**63 - 1, 20000, dtype=np.int64) >> rng.integers(1, 63, 20000)
+    v = np.concatenate([v] + [np.array([s * ((1 << b) + k) for s in (-1, 1)], np.int64)
+                              for b in range(0, 62) for k in (-2, -1, 0, 1)])
+    assert q(v.ctypes.data_as(P), len(v)) == 0
+    h = hp.fbs_hp_hamilton_split_check
+    h.argtypes, h.restype = [P, P, C.c_uint64, P], C.c_uint64
+    n = 100000
+    a = rng.integers(-(1 << 30), (1 << 30) + 1, (n, 4)).astype(np.int32)  # |a| sums to 2^31 at most
+    a //= 2
+    b = rng.integers(-2**63, 2**63 - 1, (n, 4), dtype=np.int64) >> rng.integers(0, 63, (n, 4))
+    b[::7, 1] = (b[::7, 1] & ~np.int64(0xffffffff)) | np.int64(0x80000000)
+    b[::11, 2] = 2**63 - 1
+    b[1::11, 3] = 2**63 - 2**31 - 1
+    b[2::11, 0] = -2**63
+    no = C.c_uint64()
+    assert h(a.ctypes.data_as(P), b.ctypes.data_as(P), n, C.byref(no)) == 0
+    assert n // 11 <= no.value < n // 5

@@ -81,6 +81,37 @@ uint64_t fbs_hp_publish_check(const int64_t *v, uint64_t n) {
   return bad;
 }
 
+// quantize_elem_fast against quantize_elem on n values at the shift of every magnitude that holds
+// them (62 bits at most).
+uint64_t fbs_hp_quantize_fast_check(const int64_t *v, uint64_t n) {
+  uint64_t bad = 0;
+  for (uint64_t i = 0; i < n; i++)
+    for (int32_t bl = bitlen64(uabs64(v[i])); bl <= 62; bl++) {
+      const int32_t s = bl > 15 ? bl - 15 : 0;
+      bad += quantize_elem_fast(v[i], (1ull << s) >> 1, s) != quantize_elem(v[i], s);
+    }
+  return bad;
+}
+
+// hamilton32_split against hamilton32_hl on n pairs whose right operands pass split_ok (others are
+// counted in *refused).
+uint64_t fbs_hp_hamilton_split_check(const int32_t *a, const int64_t *b, uint64_t n, uint64_t *refused) {
+  uint64_t bad = 0, no = 0;
+  for (uint64_t i = 0; i < n; i++) {
+    const int64_t *r = b + 4 * i;
+    if (!(split_ok(r[0]) && split_ok(r[1]) && split_ok(r[2]) && split_ok(r[3]))) {
+      no++;
+      continue;
+    }
+    int64_t h0[4], l0[4], h1[4], l1[4];
+    hamilton32_hl(a + 4 * i, r, h0, l0);
+    hamilton32_split(a + 4 * i, r, h1, l1);
+    for (int k = 0; k < 4; k++) bad += h0[k] != h1[k] || l0[k] != l1[k];
+  }
+  *refused = no;
+  return bad;
+}
+
 // hamilton32x32 then shift_i64(.., 14) against hamilton32 and shift_wide(.., 14).
 uint64_t fbs_hp_hamilton_mlp_check(const int32_t *a, const int32_t *b, uint64_t n) {
   uint64_t bad = 0;

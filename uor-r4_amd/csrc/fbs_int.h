@@ -46,8 +46,12 @@ FBS_HD int64_t sat_add64(int64_t a, int64_t b) {
 }
 FBS_HD int64_t sat_neg64(int64_t v) { return v == INT64_MIN ? INT64_MAX : -v; }
 FBS_HD int32_t sat_add32(int32_t a, int32_t b) {
+#if __has_builtin(__builtin_elementwise_add_sat)
+  return __builtin_elementwise_add_sat(a, b);  // one saturating add
+#else
   int64_t s = (int64_t)a + b;
   return s > INT32_MAX ? INT32_MAX : s < INT32_MIN ? INT32_MIN : (int32_t)s;
+#endif
 }
 FBS_HD int32_t clamp_i32(int64_t v) {
   return v > INT32_MAX ? INT32_MAX : v < INT32_MIN ? INT32_MIN : (int32_t)v;
@@ -226,6 +230,36 @@ FBS_HD uint32_t rsqrt_q46(uint32_t t, const uint32_t *tab) {
   return y;
 }
 FBS_HD uint32_t rsqrt_q46(uint32_t t) { return rsqrt_q46(t, rsqrt_seed_table()); }
+
+// The high 32 bits of a signed 32 x 32 product.
+FBS_HD int32_t mulhi32s(int32_t a, int32_t b) { return (int32_t)(((int64_t)a * b) >> 32); }
+
+// rsqrt_q46 in fewer steps: y below 2^31, within 2^-28.3 of 2^46 / sqrt(t), relative (checked over
+// every input). Newton in its residual form, y -= y (t y^2 / 2^92 - 1) / 2: after the seed t y^2 /
+// 2^60 lies within 2^25 of 2^32, so its low 32 bits are the signed residual; y stays below 2^31
+// where it is a signed factor.
+FBS_HD uint32_t rsqrt_q46s(uint32_t t, const uint32_t *tab) {
+  uint32_t y = tab[(t >> 23) - 128];
+#pragma unroll
+  for (int it = 0; it < 2; it++) {
+    const uint32_t res = (uint32_t)(((uint64_t)t * mulhi32(y, y)) >> 28);
+    y -= (uint32_t)(mulhi32s((int32_t)y, (int32_t)res) >> 1);
+  }
+  return y < 0x7fffffffu ? y : 0x7fffffffu;
+}
+// 2^86 / sqrt(xn) for xn in [2^62, 2^64), in (2^54, 2^55], within (-2, +0.1]: y = rsqrt_q46s of xn's
+// high word is 2^62 / sqrt(xn) (1 + d), |d| < 2^-28; one Newton step y (1 + E / 2) on E =
+// 1 - y^2 xn / 2^124 leaves -1.5 d^2 (at most 0.75 of the result's units), the products' floors in
+// E (3 units of 2^-60, then its top 31 bits) less than 0.1 and the last floor 1.
+FBS_HD uint64_t rsqrt_q86(uint64_t xn, const uint32_t *tab) {
+  const uint32_t xt = (uint32_t)(xn >> 32), xb = (uint32_t)xn;
+  const uint32_t y = rsqrt_q46s(xt, tab);
+  const uint64_t y2 = (uint64_t)y * y;
+  const uint32_t yh = (uint32_t)(y2 >> 32), yl = (uint32_t)y2;
+  const uint64_t p = (uint64_t)yh * xt + ((uint64_t)mulhi32(yh, xb) + mulhi32(yl, xt));  // y^2 xn / 2^64
+  const int32_t e = (int32_t)((int64_t)((1ull << 60) - p) >> 2);
+  return ((uint64_t)y << 24) + (uint64_t)(((int64_t)e * (int32_t)y) >> 35);
+}
 
 // w ~ 2^63 / d for d in [2^31, 2^32); w in (2^31, 2^32), relative error below 2^-30. w stays
 // below 2^32 and (2^63 - d w) / 2^31 inside +-2^23.1 at every step (checked over every input),
@@ -594,11 +628,8 @@ FBS_HD NormFactor norm_factor_wave(uint64_t sum, uint32_t log2n, int64_t eps_int
 
 // norm_factor_pow2 where the factor's real value decides its floor: with m = ms in [2^30, 2^59],
 // r = floor(2^96 / s) for s = floor(2^34 sqrt(m)), and 2^96 / s exceeds R = 2^62 / sqrt(m) by less
-// than 2^28 / m. R 2^w comes from the 32-bit reciprocal square root y ~ 2^62 / sqrt(mn)
-// (mn = m 2^(4 + z) in [2^62, 2^64), relative error below 2^-28.6 with mn's truncation to mt) by one
-// Newton step, y (1 + E / 2) with E = 1 - y^2 mn / 2^124: rq = 2^86 / sqrt(mn) = R 2^(22 - z / 2)
-// within (-1.4, +0.1] (the step's own error is below 1.5 2^-57.2 of it, that of E's top 31 bits
-// below 2^-59). Its integer part is r unless its fraction lies within 1 of 0, or within 2 and the
+// than 2^28 / m. rq = rsqrt_q86(mn) of mn = m 2^(4 + z) is R 2^w, w = 22 - z / 2, within
+// (-2, +0.1]. Its integer part is r unless its fraction lies within 1 of 0, or within 2 and the
 // 2^28 / m (at most 2^(z / 2 - 8) of its units) of the next integer: then, or for another m, false
 // and the caller takes norm_factor_wave (0.7 % of the inputs near m = 2^36, 27 % just above 2^30).
 FBS_HD bool norm_factor_direct(uint64_t sum, uint32_t log2n, int64_t eps_int, const Seeds &sd,
@@ -608,13 +639,7 @@ FBS_HD bool norm_factor_direct(uint64_t sum, uint32_t log2n, int64_t eps_int, co
   const uint64_t M = ms << 4;
   const int z = clz64(M) & ~1;                        // [0, 28]
   const uint64_t mn = M << z;
-  const uint32_t mt = (uint32_t)(mn >> 32), ml = (uint32_t)mn;
-  const uint32_t y = rsqrt_q46(mt, sd.rsq_seed);
-  const uint64_t y2 = (uint64_t)y * y;
-  const uint32_t yh = (uint32_t)(y2 >> 32), yl = (uint32_t)y2;
-  const uint64_t p = (uint64_t)yh * mt + ((uint64_t)mulhi32(yh, ml) + mulhi32(yl, mt));  // y^2 mn / 2^64
-  const int32_t e = (int32_t)((int64_t)((1ull << 60) - p) >> 2);
-  const uint64_t rq = ((uint64_t)y << 24) + (uint64_t)(((int64_t)e * (int64_t)(uint64_t)y) >> 35);
+  const uint64_t rq = rsqrt_q86(mn, sd.rsq_seed);
   const int w = 22 - (z >> 1);                        // [8, 22]
   r = rq >> w;
   const uint32_t frac = (uint32_t)rq & ((1u << w) - 1), slack = 3 + ((1u << (z >> 1)) >> 8);
@@ -681,11 +706,22 @@ FBS_HD int32_t quantize_elem(int64_t v, int32_t s) {
   return (int32_t)(y > 32767 ? 32767 : y < -32767 ? -32767 : y);
 }
 
+// quantize_elem where the largest magnitude has bl <= 62 bits and s = max(bl - 15, 0): no sum
+// saturates and the shifted value fits 16 bits but for its rounding. half = 2^s / 2.
+FBS_HD int32_t quantize_elem_fast(int64_t v, uint64_t half, int32_t s) {
+  const int32_t y = (int32_t)((v + (int64_t)half) >> s);
+  const int32_t t = y > -32767 ? y : -32767;
+  return t < 32767 ? t : 32767;
+}
+
 // to_exp_i32 of a and of -a (|a| <= 32767) from exponent `exp` to -16: a << -k clamped to the
 // i32 range, or rounded half up by k = -16 - exp (zero once k >= 17, as |a| + 2^(k-1) < 2^k).
 FBS_HD void publish16_pair(int32_t a, int32_t exp, int32_t *p, int32_t *n) {
   const int32_t k = kResidualExp - exp;
-  if (k <= 0) {
+  if (k <= 0 && k >= -16) {  // |a| 2^16 < 2^31: nothing clamps
+    *p = (int32_t)((uint32_t)a << -k);
+    *n = -*p;
+  } else if (k <= 0) {
     const int32_t l = -k > 40 ? 40 : -k;
     *p = clamp_i32((int64_t)a << l);
     *n = clamp_i32(-(int64_t)a << l);
@@ -756,6 +792,27 @@ FBS_HD void hamilton32_hl(const int32_t a[4], const int64_t b[4], int64_t Ho[4],
     Lo[k] = L;
   }
 }
+// The same sums with b's halves split once: b = hi 2^32 + lo, lo signed, for b below 2^63 - 2^31
+// (split_ok), where hi fits 32 bits.
+FBS_HD bool split_ok(int64_t b) { return (int32_t)(b >> 32) != INT32_MAX; }
+FBS_HD void hamilton32_split(const int32_t a[4], const int64_t b[4], int64_t Ho[4], int64_t Lo[4]) {
+  int32_t hi[4], lo[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    hi[j] = (int32_t)(uint32_t)(((uint64_t)b[j] + (1ull << 31)) >> 32);
+    lo[j] = (int32_t)(uint32_t)b[j];
+  }
+#define FBS_R(x, i, j) ((int64_t)a[i] * (int64_t)x[j])
+#define FBS_S(o, x)                                                                \
+  o[0] = FBS_R(x, 0, 0) - FBS_R(x, 1, 1) - FBS_R(x, 2, 2) - FBS_R(x, 3, 3);       \
+  o[1] = FBS_R(x, 0, 1) + FBS_R(x, 1, 0) + FBS_R(x, 2, 3) - FBS_R(x, 3, 2);       \
+  o[2] = FBS_R(x, 0, 2) - FBS_R(x, 1, 3) + FBS_R(x, 2, 0) + FBS_R(x, 3, 1);       \
+  o[3] = FBS_R(x, 0, 3) + FBS_R(x, 1, 2) - FBS_R(x, 2, 1) + FBS_R(x, 3, 0);
+  FBS_S(Ho, hi)
+  FBS_S(Lo, lo)
+#undef FBS_S
+#undef FBS_R
+}
 FBS_HD void hamilton32(const int32_t a[4], const int64_t b[4], i128 o[4]) {
   int64_t H[4], L[4];
   hamilton32_hl(a, b, H, L);
@@ -800,8 +857,8 @@ FBS_HD void hamilton32x32(const int32_t a[4], const int32_t b[4], int64_t o[4]) 
 #undef FBS_Q
 }
 
-// shift_wide of an i64 value (round half up, no clamp needed): s in [1, 62].
-FBS_HD int64_t shift_i64(int64_t v, uint32_t s) { return (v >> s) + ((v >> (s - 1)) & 1); }
+// shift_wide of an i64 value below 2^63 - 2^(s-1) (round half up, no clamp needed): s in [1, 62].
+FBS_HD int64_t shift_i64(int64_t v, uint32_t s) { return (v + (1ll << (s - 1))) >> s; }
 
 // Sign of da + db phi, exactly (RS stack/kernels.rs:1180-1215, TW 393-408).
 FBS_HD bool diff_positive(int64_t da, int64_t db) {
@@ -867,73 +924,59 @@ FBS_HD void unit_q30_wide(const int32_t raw[4], uint64_t eps, int32_t u[4]) {
 }
 
 // unit_q30 in 64-bit arithmetic without data-dependent branches (the kernels' form; equal to
-// unit_q30_wide for every input). With X = sum v^2 + eps < 2^65 + 2^13 and Y = X 2^32:
-//  1. Xn = X 4^k in [2^62, 2^64) (k = -1: Xn = floor(X / 4)); y = rsqrt_q46(Xn / 2^32) ~
-//     2^62 / sqrt(Xn) (relative error within 2^-28.9, checked over every input); r = Xn/2^32
-//     y / 2^30 and one Newton step on the exact remainder give r within 1 of isqrt(Xn).
-//  2. s0 = r 2^j + floor((Xn - r^2) (y / 4) / 2^(61 - j)) for j = 16 - k > 0, or r >> -j, is
-//     within 1 of s = isqrt(Y); the remainder Y - s0^2 is below 2^63 in magnitude, so its
-//     value modulo 2^64 is exact, and one step down and one up give s.
-//  3. w = recip_q63 of the top 32 bits of s normalised (relative error in [-2^-30.4, 0],
-//     checked over every input; truncating s adds at most 2^-31) puts (a 2^46 w) / s within
-//     0.76 of a 2^46 / s <= 2^30 + 2^14, so q0 is within 1 of the floor; one step each way on
-//     the exact remainder a 2^46 - q0 s (small, exact modulo 2^64) gives q.
-FBS_HD void unit_q30(const int32_t raw[4], uint64_t eps, int32_t u[4], const Seeds &sd = Seeds()) {
-  uint32_t a[4];
-  uint64_t xl = eps;
-  uint32_t xh = 0;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    a[c] = uabs32(raw[c]);
-    const uint64_t t = xl + (uint64_t)a[c] * a[c];
-    xh += t < xl;
-    xl = t;
-  }
+// unit_q30_wide), for X = sum v^2 + eps < 2^64. With Y = X 2^32:
+//  1. Xn = X 2^z in [2^62, 2^64), z even; rq = rsqrt_q86(Xn) - 1 lies below 2^86 / sqrt(Xn), by
+//     less than 3.
+//  2. Xn rq / 2^64 is sqrt(Xn) 2^22 less at most 7, so s0 = that >> (6 + z / 2) is s = isqrt(Y) or
+//     s - 1; the remainder Y - s0^2 (below 2^51, exact modulo 2^64) decides.
+//  3. s 2^(16 + z / 2) lies in [2^63, 2^64); d is its top 32 bits and w0 = rq / 2^23 ~ 2^63 / d
+//     within 2^-15 (s's floor moves it by at most 1 / s <= 2^-16). One Newton step for d + 1 stays at
+//     or below 2^95 / (s 2^zs) and within 2^-29.6 of it (the step's error 2^-30, d + 1 and the floor
+//     2^-31 each, relative), so with a 2^46 / s <= 2^30 + 2^14 each quotient q0 is within
+//     [q - 2, q]; the exact remainder a 2^46 - q0 s (below 2^51) gives the steps up.
+FBS_HD void unit_q30_64(const int32_t raw[4], uint64_t x, int32_t u[4], const Seeds &sd) {
   // X = 0 (all zero, eps 0) gives u = 0 by the same steps on X = 1.
-  xl = (xh == 0 && xl == 0) ? 1 : xl;
-  // Both normalisations are formed and one is kept by masks (one basic block, so that the
-  // scheduler can interleave independent rotations).
-  // z is taken mod 64 so that the unused form stays a defined shift when xl = 0 (then xh != 0
-  // and the mask keeps the other form).
-  const int z = clz64(xl) & 62;
-  const uint64_t big = 0ull - (uint64_t)(xh != 0);
-  const uint64_t xn = ((((uint64_t)xh << 62) | (xl >> 2)) & big) | ((xl << z) & ~big);
-  const int j = xh ? 17 : 16 - (z >> 1);              // [-15, 17]
-  // As in norm_factor_pow2, every product but the fraction's has 32-bit factors.
-  const uint32_t xt = (uint32_t)(xn >> 32);
-  const uint32_t y = rsqrt_q46(xt, sd.rsq_seed);
-  uint64_t r = ((uint64_t)xt * y) >> 30;
-  r = r > 0xffffffffull ? 0xffffffffull : r;
-  const int64_t diff = (int64_t)(xn - (uint64_t)(uint32_t)r * (uint32_t)r);
-  r = (uint64_t)((int64_t)r + (((int64_t)(int32_t)(diff >> 16) * (int64_t)(uint64_t)y) >> 47));
-  r = r > 0xffffffffull ? 0xffffffffull : r < (1ull << 31) ? (1ull << 31) : r;
-  const int64_t rem = (int64_t)(xn - (uint64_t)(uint32_t)r * (uint32_t)r);  // [-2^33, 2^34]
-  const int jp = j > 0 ? j : 0, jn = j > 0 ? 0 : -j;
-  const int64_t f = (rem * (int64_t)(y >> 2)) >> (61 - jp);
-  const uint64_t frac = 0ull - (uint64_t)(j > 0);
-  uint64_t s = (((r << jp) + (uint64_t)f) & frac) | ((r >> jn) & ~frac);
-  // Y - s^2 modulo 2^64: s < 2^50, so s^2 mod 2^64 = sl^2 + (2 sh sl mod 2^32) 2^32.
-  const uint32_t sl = (uint32_t)s, shi = (uint32_t)(s >> 32);
-  int64_t dy = (int64_t)((xl << 32) - ((uint64_t)sl * sl + ((uint64_t)(2u * shi * sl) << 32)));
-  const bool down = dy < 0;
-  dy = down ? dy + (int64_t)(2 * s - 1) : dy;
-  s = down ? s - 1 : s;
-  const bool up = dy >= (int64_t)(2 * s + 1);
-  s = up ? s + 1 : s;
-  // u_c = floor(a_c 2^46 / s), s in [2^16, 2^49].
-  const int zs = clz64(s);
-  const uint32_t w = recip_q63((uint32_t)((s << zs) >> 32), sd.rcp_seed);  // ~ 2^95 / (s << zs)
-  const int sh = 49 - zs;
+  x = x ? x : 1;
+  const int z = clz64(x) & 62;
+  const uint64_t xn = x << z;
+  const uint32_t xt = (uint32_t)(xn >> 32), xb = (uint32_t)xn;
+  const uint64_t rq = rsqrt_q86(xn, sd.rsq_seed) - 1;
+  const uint32_t rh = (uint32_t)(rq >> 32), rl = (uint32_t)rq;
+  const uint64_t root = (uint64_t)rh * xt + ((uint64_t)mulhi32(rh, xb) + mulhi32(rl, xt));
+  const int half = z >> 1;
+  uint64_t s = root >> (6 + half);
+  const uint32_t sl0 = (uint32_t)s, sh0 = (uint32_t)(s >> 32);
+  const uint64_t dy = (x << 32) - ((uint64_t)sl0 * sl0 + ((uint64_t)(2u * sh0 * sl0) << 32));
+  s += dy > 2 * s;                                    // (s + 1)^2 <= Y
+  const uint32_t sl = (uint32_t)s, sh = (uint32_t)(s >> 32);
+  const uint32_t d = (uint32_t)((s << (16 + half)) >> 32);
+  const uint32_t w0 = (uint32_t)(rq >> 23);
+  const int32_t es = (int32_t)((int64_t)((1ull << 63) - w0 - (uint64_t)d * w0) >> 31);
+  const uint32_t w = w0 + (uint32_t)(((int64_t)es * (int32_t)(w0 >> 1)) >> 31);
+  const int qsh = 33 - half;
+  const uint64_t s2 = 2 * s;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    uint64_t q = ((uint64_t)a[c] * w) >> sh;        // below 2^31
-    int64_t rq = (int64_t)(((uint64_t)a[c] << 46) - (uint64_t)(uint32_t)q * s);
-    const bool qd = rq < 0;
-    rq = qd ? rq + (int64_t)s : rq;
-    q = qd ? q - 1 : q;
-    q = rq >= (int64_t)s ? q + 1 : q;
-    u[c] = raw[c] < 0 ? -(int32_t)q : (int32_t)q;
+    const uint32_t a = uabs32(raw[c]);
+    const uint32_t q0 = (uint32_t)(((uint64_t)a * w) >> qsh);
+    const uint64_t rem = ((uint64_t)(a << 14) << 32) - ((uint64_t)q0 * sl + ((uint64_t)(q0 * sh) << 32));
+    const int32_t q = (int32_t)(q0 + (rem >= s) + (rem >= s2));
+    u[c] = raw[c] < 0 ? -q : q;
   }
+}
+FBS_HD uint64_t unit_square(const int32_t raw[4], uint64_t eps, bool &wide) {
+  const uint64_t a = (uint64_t)((int64_t)raw[0] * raw[0]) + (uint64_t)((int64_t)raw[1] * raw[1]) ;
+  const uint64_t b = (uint64_t)((int64_t)raw[2] * raw[2]) + (uint64_t)((int64_t)raw[3] * raw[3]) + eps;
+  wide = ((uint32_t)(a >> 32) | (uint32_t)(b >> 32)) >> 31;  // each at most 2^63 + eps
+  return a + b;
+}
+FBS_HD void unit_q30(const int32_t raw[4], uint64_t eps, int32_t u[4], const Seeds &sd = Seeds()) {
+  bool wide;
+  const uint64_t x = unit_square(raw, eps, wide);
+  if (wide)
+    unit_q30_wide(raw, eps, u);
+  else
+    unit_q30_64(raw, x, u, sd);
 }
 
 // (lambda u) >> 30 for lambda = 2^p (p <= 31): u << (p - 30) or floor(u / 2^(30 - p)).

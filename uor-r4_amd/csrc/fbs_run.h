@@ -99,8 +99,9 @@ __device__ __forceinline__ uint64_t wave_reduce64(uint64_t v, Op op) {
   v = op(v, dpp64<kDppMirror>(v));
   return op(op(lane64(v, 0), lane64(v, 16)), op(lane64(v, 32), lane64(v, 48)));
 }
-// The bit length of the wave's largest magnitude from each lane's largest: the bit length of a
-// maximum is the maximum of the bit lengths, so a 32-bit reduction takes the place of a 64-bit one.
+// The bit length of the wave's largest magnitude from each lane's magnitudes or-ed together: the bit
+// length of a maximum is the maximum of the bit lengths, and that of the or, so a 32-bit reduction
+// takes the place of a 64-bit one.
 __device__ __forceinline__ int32_t wave_bitlen_max(uint64_t v) {
   return (int32_t)wave_reduce32((uint32_t)bitlen64(v), OpMax());
 }
@@ -341,6 +342,9 @@ __device__ __forceinline__ uint32_t prog_word(const uint16_t *prog, uint32_t slo
 // The snapped transition or gate (RS stack/kernels.rs:1474-1557), out of line: the 120-root
 // scan is long and served only by snapped artifacts. The quaternion comes back by value (in
 // registers), so no caller array lives in private memory.
+struct Wide4 {
+  int64_t hi[4], lo[4];
+};
 struct Quat64 {
   int64_t v[4];
   uint32_t root;  // the chosen root's index
@@ -365,9 +369,6 @@ __device__ __noinline__ Quat64 hamilton64_shift(int64_t q0, int64_t q1, int64_t 
   o.root = 0;
   return o;
 }
-struct Wide4 {
-  int64_t hi[4], lo[4];
-};
 __device__ __noinline__ Wide4 hamilton64_wide(int64_t q0, int64_t q1, int64_t q2, int64_t q3,
                                               int64_t r0, int64_t r1, int64_t r2, int64_t r3) {
   const int64_t q[4] = {q0, q1, q2, q3}, r[4] = {r0, r1, r2, r3};
@@ -396,6 +397,49 @@ __device__ __forceinline__ uint32_t snap_rotation_to(const int8_t *ico, int4 raw
   return q.root;
 }
 
+// unit_q30 on the wave: every lane's 64-bit form, or, where some lane's square passes 64 bits (its
+// raw values at the ends of their range), the 128-bit one, out of line.
+struct Quat32 {
+  int32_t v[4];
+};
+__device__ __noinline__ Quat32 unit_q30_slow(int4 raw, uint64_t eps) {
+  const int32_t r[4] = {raw.x, raw.y, raw.z, raw.w};
+  Quat32 q;
+  unit_q30_wide(r, eps, q.v);
+  return q;
+}
+__device__ __forceinline__ void wave_unit_q30(const int32_t (&raw)[4], uint64_t eps, int32_t (&u)[4],
+                                              const Seeds &sd) {
+  bool wide;
+  const uint64_t x = unit_square(raw, eps, wide);
+  if (__any(wide)) {
+    const Quat32 q = unit_q30_slow(make_int4(raw[0], raw[1], raw[2], raw[3]), eps);
+#pragma unroll
+    for (int c = 0; c < 4; c++) u[c] = q.v[c];
+  } else {
+    unit_q30_64(raw, x, u, sd);
+  }
+}
+// a (x) b as hamilton32_hl's sums, or its out of line form where some lane's b lies at the very top
+// of 64 bits (a saturated state).
+__device__ __noinline__ Wide4 hamilton32_slow(int4 a, int64_t b0, int64_t b1, int64_t b2, int64_t b3) {
+  const int32_t q[4] = {a.x, a.y, a.z, a.w};
+  const int64_t b[4] = {b0, b1, b2, b3};
+  Wide4 o;
+  hamilton32_hl(q, b, o.hi, o.lo);
+  return o;
+}
+__device__ __forceinline__ void wave_hamilton32(const int32_t (&a)[4], const int64_t (&b)[4], int64_t (&H)[4],
+                                                int64_t (&L)[4]) {
+  if (__all(split_ok(b[0]) & split_ok(b[1]) & split_ok(b[2]) & split_ok(b[3]))) {
+    hamilton32_split(a, b, H, L);
+  } else {
+    const Wide4 o = hamilton32_slow(make_int4(a[0], a[1], a[2], a[3]), b[0], b[1], b[2], b[3]);
+#pragma unroll
+    for (int c = 0; c < 4; c++) H[c] = o.hi[c], L[c] = o.lo[c];
+  }
+}
+
 // The Hamilton gate on rhs (session.rs:4951-4968, :4005-4025): shift_wide(q (x) rhs, 15) with
 // q the gate's unit quaternion (lambda 2^31, epsilon 0) or its icosian. Raw gates use q = 2 u
 // exactly, so the product is formed from u and shifted by 14.
@@ -406,7 +450,7 @@ __device__ __forceinline__ uint32_t gate_apply(const DevModel &M, const Seeds &s
   i128 prod[4];
   if (M.raw_gates) {
     int32_t u[4];
-    unit_q30(raw, kGateEps, u, sd);
+    wave_unit_q30(raw, kGateEps, u, sd);
     hamilton32(u, rhs, prod);
 #pragma unroll
     for (int c = 0; c < 4; c++) out[c] = shift_wide(prod[c], 14);
@@ -429,7 +473,7 @@ __device__ __forceinline__ uint32_t mlp_gate(const DevModel &M, const Seeds &sd,
   if (M.raw_gates) {
     int32_t u[4];
     int64_t prod[4];
-    unit_q30(gq, kGateEps, u, sd);
+    wave_unit_q30(gq, kGateEps, u, sd);
     hamilton32x32(u, up, prod);
 #pragma unroll
     for (int c = 0; c < 4; c++) mo[c] = shift_i64(prod[c], 14);
@@ -439,32 +483,11 @@ __device__ __forceinline__ uint32_t mlp_gate(const DevModel &M, const Seeds &sd,
   return gate_apply(M, sd, gq, up64, mo);
 }
 
-// gate_apply split in two for paired blocks: gate_quat forms the gate's quaternion (the unit
-// quaternion u of a raw gate, or the snapped gate at lambda 2^31), gate_mul applies it.
-__device__ __forceinline__ void gate_quat(const DevModel &M, const Seeds &sd, const int32_t (&raw)[4],
-                                          int64_t (&g)[4]) {
-  if (M.raw_gates) {
-    int32_t u[4];
-    unit_q30(raw, kGateEps, u, sd);
+// A snapped gate's quaternion g (paired blocks) applied to rhs.
+__device__ __forceinline__ void gate_mul(const int64_t (&g)[4], const int64_t (&rhs)[4], int64_t (&out)[4]) {
+  const Quat64 p = hamilton64_shift(g[0], g[1], g[2], g[3], rhs[0], rhs[1], rhs[2], rhs[3], 15);
 #pragma unroll
-    for (int c = 0; c < 4; c++) g[c] = u[c];
-  } else {
-    snap_rotation_to(M.icosian, make_int4(raw[0], raw[1], raw[2], raw[3]), 1ull << 31, g);
-  }
-}
-__device__ __forceinline__ void gate_mul(const DevModel &M, const int64_t (&g)[4],
-                                         const int64_t (&rhs)[4], int64_t (&out)[4]) {
-  i128 prod[4];
-  if (M.raw_gates) {
-    const int32_t u[4] = {(int32_t)g[0], (int32_t)g[1], (int32_t)g[2], (int32_t)g[3]};
-    hamilton32(u, rhs, prod);
-#pragma unroll
-    for (int c = 0; c < 4; c++) out[c] = shift_wide(prod[c], 14);
-  } else {
-    const Quat64 p = hamilton64_shift(g[0], g[1], g[2], g[3], rhs[0], rhs[1], rhs[2], rhs[3], 15);
-#pragma unroll
-    for (int c = 0; c < 4; c++) out[c] = p.v[c];
-  }
+  for (int c = 0; c < 4; c++) out[c] = p.v[c];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1088,7 +1111,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       uint32_t root = kTraceNone;
       if (M.raw_transition) {
         int32_t u[4];
-        unit_q30(rot[k], kRotationEps, u, S.seeds);
+        wave_unit_q30(rot[k], kRotationEps, u, S.seeds);
 #pragma unroll
         for (int c = 0; c < 4; c++) T[c] = u[c] >> idx;  // (lambda u) >> 30, lambda = 2^(30-idx)
       } else {
@@ -1364,21 +1387,39 @@ __device__ __forceinline__ void clip_ranges(uint32_t P, uint32_t lane, uint32_t 
   my_end = ne;
 }
 
-// The MLP's requantize (quantize16, kernels.rs:545-553) for groups j0, j0 + 2, ...: S.mlp_out
-// at the shared shift of both waves' maxima, published for the mlp_down gathers.
-__device__ __forceinline__ void pair_requant(const DevModel &M, const Lds &S, uint32_t lane,
-                                             uint32_t j0) {
-  const uint64_t bl = S.pair[0] > S.pair[1] ? S.pair[0] : S.pair[1];  // bit lengths
-  int32_t qs = (int32_t)bl - 15;
+// quantize16 (kernels.rs:545-553) of four channels at the shared shift of magnitudes of `bl` bits,
+// published at crossbar channel `channel0`: the fast element form where no sum can saturate (one
+// uniform branch).
+__device__ __forceinline__ void requant_publish(int32_t *xbar, uint32_t channel0, const int64_t (&v)[4],
+                                                int32_t bl) {
+  int32_t qs = bl - 15;
   if (qs < 0) qs = 0;
+  int32_t a[4];
+  if (bl <= 62) {
+    const uint64_t half = (1ull << qs) >> 1;
+#pragma unroll
+    for (int c = 0; c < 4; c++) a[c] = quantize_elem_fast(v[c], half, qs);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; c++) a[c] = quantize_elem(v[c], qs);
+  }
+  publish16(xbar, channel0, a, kProductExp + qs);
+}
+
+// The MLP's requantize for groups j0, j0 + 2, ... at the shared shift of both waves' magnitudes,
+// published for the mlp_down gathers: group j0 from `mo` (this lane formed it), the later ones from
+// S.mlp_out.
+__device__ __forceinline__ void pair_requant(const DevModel &M, const Lds &S, uint32_t lane,
+                                             uint32_t j0, const int64_t (&mo)[4]) {
+  const uint32_t bits = S.pair[0] > S.pair[1] ? (uint32_t)S.pair[0] : (uint32_t)S.pair[1];
+  const int32_t bl = (int32_t)uniform32(bits);
+  if (lane + kWave * j0 < M.nm) requant_publish(S.xbar, 4 * (lane + kWave * j0), mo, bl);
 #pragma unroll 1
-  for (uint32_t j = j0; j < M.mpl; j += 2) {
+  for (uint32_t j = j0 + 2; j < M.mpl; j += 2) {
     const uint32_t mq = lane + kWave * j;
     if (mq < M.nm) {
-      int32_t a[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) a[c] = quantize_elem(S.mlp_out[4 * mq + c], qs);
-      publish16(S.xbar, 4 * mq, a, kProductExp + qs);
+      const int64_t v[4] = {S.mlp_out[4 * mq], S.mlp_out[4 * mq + 1], S.mlp_out[4 * mq + 2], S.mlp_out[4 * mq + 3]};
+      requant_publish(S.xbar, 4 * mq, v, bl);
     }
   }
 }
@@ -1396,13 +1437,15 @@ __device__ __forceinline__ void pair_mlp_words(const DevModel &M, const DevLayer
   }
 }
 
-// MLP quaternion groups j0, j0 + 2, ... of the feed-forward gate (session.rs:4005-4025) into
-// S.mlp_out; pg/pu hold group j0's gather words. Returns the bit length of the groups' largest
-// magnitude.
+// MLP quaternion groups j0, j0 + 2, ... of the feed-forward gate (session.rs:4005-4025): group j0
+// into `mo`, the later ones into S.mlp_out; pg/pu hold group j0's gather words. Returns the bit
+// length of the groups' largest magnitude.
 __device__ __forceinline__ uint64_t pair_mlp(const DevModel &M, const Lds &S, const DevLayer &ly,
                                              uint32_t lane, uint32_t j0, uint32_t (&pg)[4],
-                                             uint32_t (&pu)[4]) {
+                                             uint32_t (&pu)[4], int64_t (&mo)[4]) {
   uint64_t mmx = 0;
+#pragma unroll
+  for (int c = 0; c < 4; c++) mo[c] = 0;
 #pragma unroll 1
   for (uint32_t j = j0; j < M.mpl; j += 2) {
     const uint32_t mq = lane + kWave * j;
@@ -1414,13 +1457,15 @@ __device__ __forceinline__ uint64_t pair_mlp(const DevModel &M, const Lds &S, co
     }
     pair_mlp_words(M, ly, lane, j + 2, pg, pu);  // the next group's (none past the last)
     if (mq < M.nm) {
-      int64_t mo[4];
-      mlp_gate(M, S.seeds, gq, up, mo);
+      int64_t o[4];
+      mlp_gate(M, S.seeds, gq, up, o);
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        S.mlp_out[4 * mq + c] = mo[c];
-        uint64_t a = uabs64(mo[c]);
-        mmx = a > mmx ? a : mmx;
+        mmx |= uabs64(o[c]);
+        if (j == j0)
+          mo[c] = o[c];
+        else
+          S.mlp_out[4 * mq + c] = o[c];
       }
     }
   }
@@ -1598,10 +1643,10 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
       }
       if (M.raw_transition) {
         int32_t u[4], T[4];
-        unit_q30(rot[k], kRotationEps, u, S.seeds);
+        wave_unit_q30(rot[k], kRotationEps, u, S.seeds);
 #pragma unroll
         for (int c = 0; c < 4; c++) T[c] = u[c] >> idx;  // (lambda u) >> 30, lambda = 2^(30-idx)
-        hamilton32_hl(T, h, mh[k], ml[k]);
+        wave_hamilton32(T, h, mh[k], ml[k]);
       } else {
         int64_t T64[4];
         snap_rotation_to(M.icosian, make_int4(rot[k][0], rot[k][1], rot[k][2], rot[k][3]),
@@ -1617,7 +1662,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     clk.sync(kPartTransition, kPartSync2);  // 2: the window sums and the output gates' quaternions
     // Transport: h <- shift_wide(T (x) h + (keep wide) << 16, 31). A raw transition whose sums
     // lie in transport_fast's ranges on every lane takes its 64-bit form (one uniform branch).
-    int64_t h[Q][4];
+    int64_t h[Q][4], rhs[Q][4];  // rhs: the moved state at exponent -16 (shift by 16)
     {
       bool fast = M.raw_transition != 0;
       int64_t wide[Q][4];
@@ -1634,13 +1679,18 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
 #pragma unroll
         for (int k = 0; k < Q; k++)
 #pragma unroll
-          for (int c = 0; c < 4; c++) h[k][c] = transport_fast(mh[k][c], ml[k][c], keep[k], wide[k][c]);
+          for (int c = 0; c < 4; c++) {
+            h[k][c] = transport_fast(mh[k][c], ml[k][c], keep[k], wide[k][c]);
+            rhs[k][c] = (h[k][c] + (1ll << 15)) >> 16;  // |h| < 2^62: the sum does not saturate
+          }
       } else {
 #pragma unroll
         for (int k = 0; k < Q; k++)
 #pragma unroll
-          for (int c = 0; c < 4; c++)
+          for (int c = 0; c < 4; c++) {
             h[k][c] = transport_wide(mh[k][c], ml[k][c], keep[k], wide[k][c], M.raw_transition);
+            rhs[k][c] = shift(h[k][c], kResidualExp - kStateExp);
+          }
       }
     }
     // Output gate on the moved state (session.rs:4951-4968): a raw gate's product in its 64-bit
@@ -1664,18 +1714,15 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
             for (int c = 0; c < 4; c++) hp[c] = h[k][c];
           }
         }
-        int64_t rhs[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) rhs[c] = shift(h[k][c], kResidualExp - kStateExp);
         if (M.raw_gates) {
-          const int32_t u[4] = {(int32_t)S.gq[ch], (int32_t)S.gq[ch + 1], (int32_t)S.gq[ch + 2],
-                                (int32_t)S.gq[ch + 3]};
-          hamilton32_hl(u, rhs, gh[k], gl[k]);
+          const int4 g = ((const int4 *)S.gq)[qv[k] ? qi[k] : 0];
+          const int32_t u[4] = {g.x, g.y, g.z, g.w};
+          hamilton32_split(u, rhs[k], gh[k], gl[k]);  // |rhs| <= 2^47
 #pragma unroll
           for (int c = 0; c < 4; c++) fast = fast && (!qv[k] || gate_fast_ok(gh[k][c]));
         } else {
           const int64_t g[4] = {S.gq[ch], S.gq[ch + 1], S.gq[ch + 2], S.gq[ch + 3]};
-          gate_mul(M, g, rhs, sc[k]);
+          gate_mul(g, rhs[k], sc[k]);
         }
       }
       if (M.raw_gates) {
@@ -1696,8 +1743,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
 #pragma unroll
         for (int c = 0; c < 4; c++) {
           if (!qv[k]) sc[k][c] = 0;
-          const uint64_t a = uabs64(sc[k][c]);
-          mx = a > mx ? a : mx;
+          mx |= uabs64(sc[k][c]);
         }
     }
     clk.lap(kPartTransport);
@@ -1707,16 +1753,10 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     uint32_t pg[4], pu[4];
     pair_mlp_words(M, ly, lane, 0, pg, pu);
     // quantize16 over the d outputs (kernels.rs:545-553), then gather16 of rec_out.
-    int32_t qs = wave_bitlen_max(mx) - 15;
-    if (qs < 0) qs = 0;
+    const int32_t bl = wave_bitlen_max(mx);
 #pragma unroll
     for (int k = 0; k < Q; k++)
-      if (qv[k]) {
-        int32_t a[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) a[c] = quantize_elem(sc[k][c], qs);
-        publish16(S.xbar, 4 * qi[k], a, kProductExp + qs);
-      }
+      if (qv[k]) requant_publish(S.xbar, 4 * qi[k], sc[k], bl);
     wave_sync();
     clk.lap(kPartRequantRec);
 #pragma unroll
@@ -1730,10 +1770,11 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     if constexpr (Q != 1) load_ffn();
     norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     clk.sync(kPartNormMlp, kPartSync3);  // 3: the normed activations
-    const uint64_t mbl = pair_mlp(M, S, ly, lane, 0, pg, pu);
+    int64_t mo[4];
+    const uint64_t mbl = pair_mlp(M, S, ly, lane, 0, pg, pu, mo);
     if (lane == 0) S.pair[0] = mbl;
     clk.sync(kPartMlp, kPartSync4);  // 4: both waves' MLP outputs and maxima
-    pair_requant(M, S, lane, 0);
+    pair_requant(M, S, lane, 0, mo);
     clk.sync(kPartRequantMlp, kPartSync5);  // 5: the requantized MLP outputs
 #pragma unroll
     for (int k = 0; k < Q; k++)
@@ -1959,10 +2000,17 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
 #pragma unroll
       for (int c = 0; c < 4; c++) S.wide[ch + c] = wadd64(wide[c], sum[k][c]);
       *(int4 *)(ring_l + (uint64_t)base * d + ch) = drive[k];
-      int64_t gate[4];
-      gate_quat(M, S.seeds, gv, gate);
+      // A raw gate's unit quaternion as four 32-bit words, a snapped gate's as 64-bit ones.
+      if (M.raw_gates) {
+        int32_t u[4];
+        wave_unit_q30(gv, kGateEps, u, S.seeds);
+        ((int4 *)S.gq)[qi[k]] = make_int4(u[0], u[1], u[2], u[3]);
+      } else {
+        int64_t gate[4];
+        snap_rotation_to(M.icosian, make_int4(gv[0], gv[1], gv[2], gv[3]), 1ull << 31, gate);
 #pragma unroll
-      for (int c = 0; c < 4; c++) S.gq[ch + c] = gate[c];
+        for (int c = 0; c < 4; c++) S.gq[ch + c] = gate[c];
+      }
     }
     clk.sync(kPartTransition, kPartSync2);  // 2: the window sums and the output gates' quaternions
     // One-token serving launches (defer): the next step's window sums wait for nothing on the
@@ -1986,10 +2034,11 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
     }
     clk.sync(kPartTransport, kPartSync3);  // 3: the normed activations
     if (defer) __builtin_amdgcn_s_setprio(3);  // the MLP groups, on both waves' path
-    const uint64_t mbl = pair_mlp(M, S, ly, lane, 1, pg, pu);
+    int64_t mo[4];
+    const uint64_t mbl = pair_mlp(M, S, ly, lane, 1, pg, pu, mo);
     if (lane == 0) S.pair[1] = mbl;
     clk.sync(kPartMlp, kPartSync4);  // 4: both waves' MLP outputs and maxima
-    pair_requant(M, S, lane, 1);
+    pair_requant(M, S, lane, 1, mo);
     clk.sync(kPartRequantMlp, kPartSync5);  // 5: the requantized MLP outputs
     if constexpr (HM) {  // the stream read's odd heads (ham_help), as step_main requests it
       const int32_t r = M.ham.at[l + 1];
