@@ -680,6 +680,7 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
 
   // Layers: gains, taps, biases and the gather program.
   std::vector<DevLayer> layers(L);
+  std::vector<int32_t> tap_words((size_t)L * (r.W + 1) * d);
   for (uint32_t l = 0; l < L; l++) {
     const uor_fbs_layer &ly = m->layers[l];
     DevLayer &dl = layers[l];
@@ -688,17 +689,17 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
     const int16_t *taps = (e && e->wide_taps) ? e->wide_taps[l] : ly.taps;
     if ((st = h->upload(taps, (size_t)(r.W + 1) * d, &dl.taps))) return done(st);
     {
-      std::vector<uint16_t> td((size_t)(r.W + 1) * d), rg(d), mg(d);
-      for (size_t i = 0; i < td.size(); i++) {
-        td[i] = tap_desc(taps[i]);
-        if (td[i] == kGridDescSlow) M.taps_fast = 0;
+      std::vector<uint16_t> rg(d), mg(d);
+      const size_t nt = (size_t)(r.W + 1) * d;
+      for (size_t i = 0; i < nt; i++) {
+        tap_words[l * nt + i] = tap_word(taps[i]);
+        if (tap_words[l * nt + i] == kTapWordNone) M.taps_fast = 0;
       }
       for (uint32_t i = 0; i < d; i++) {
-        rg[i] = tap_desc(ly.rec_gain[i]);
-        mg[i] = tap_desc(ly.mlp_gain[i]);
+        rg[i] = gain_desc(ly.rec_gain[i]);
+        mg[i] = gain_desc(ly.mlp_gain[i]);
         if (rg[i] == kGridDescSlow || mg[i] == kGridDescSlow) M.gains_fast = 0;
       }
-      if ((st = h->upload(td.data(), td.size(), &dl.taps_desc))) return done(st);
       if ((st = h->upload(rg.data(), rg.size(), &dl.rec_gain_desc))) return done(st);
       if ((st = h->upload(mg.data(), mg.size(), &dl.mlp_gain_desc))) return done(st);
     }
@@ -732,11 +733,12 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
     if ((st = h->upload(prog.data(), prog.size(), &dl.prog))) return done(st);
   }
   if ((st = h->upload(layers.data(), layers.size(), &M.layers))) return done(st);
+  if ((st = h->upload(tap_words.data(), tap_words.size(), &M.tap_words))) return done(st);
   if ((st = h->upload(m->final_gain, d, &M.final_gain))) return done(st);
   {
     std::vector<uint16_t> fg(d);
     for (uint32_t i = 0; i < d; i++) {
-      fg[i] = tap_desc(m->final_gain[i]);
+      fg[i] = gain_desc(m->final_gain[i]);
       if (fg[i] == kGridDescSlow) M.gains_fast = 0;
     }
     if ((st = h->upload(fg.data(), fg.size(), &M.final_gain_desc))) return done(st);

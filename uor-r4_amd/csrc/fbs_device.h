@@ -2,8 +2,8 @@
 // the kernels (fbs_run.h) and the host side that builds them (fbs_api.cpp).
 //
 // Layout in HBM (all tables uploaded once by uor_fbs_model_create, read by every sequence):
-//   per layer: gains (d i16), window taps ((W+1) x d i16, tap s = s positions back) and their
-//              descriptor forms (tap_desc; fbs_int.h),
+//   per layer: gains (d i16) and their descriptors (gain_desc; fbs_int.h), window taps ((W+1) x d
+//              i16, tap s = s positions back) and their words (tap_word, all layers together),
 //              conv_bias (d i32), gate_bias (d/4 + d i32), decay_offset (d/4 i32), and the
 //              layer's gather program: [slot][64 lanes] u16 LDS word indices that carry out the
 //              six FBS projections (stack_fbs_gather, session.rs:4037-4053) for this lane mapping;
@@ -40,7 +40,6 @@ struct DevLayer {
   const int32_t *gate_bias;     // d/4 + d
   const int32_t *decay_offset;  // d/4
   const uint16_t *prog;         // nslots * 64
-  const uint16_t *taps_desc;    // tap_desc of taps
   const uint16_t *rec_gain_desc;
   const uint16_t *mlp_gain_desc;
 };
@@ -102,14 +101,15 @@ struct DevModel {
   uint32_t nslots, s_rec_in, s_rec_gate, s_rec_out, s_mlp_gate, s_mlp_up, s_mlp_down;
   uint32_t xbar_words;      // 2 * max(d, m)
   uint32_t identity_rows;   // the nearest head: one drawer holding every token
-  uint32_t taps_fast;       // every window tap has a descriptor (tap_desc != kGridDescSlow)
-  uint32_t gains_fast;      // every norm gain (rec, mlp, final) has a descriptor (tap_desc)
+  uint32_t taps_fast;       // every window tap has a word (tap_word != kTapWordNone)
+  uint32_t gains_fast;      // every norm gain (rec, mlp, final) has a descriptor (gain_desc)
   uint32_t log2d;           // log2(d) when d is a power of two, else 0xff
   uint32_t writer_memory;   // 1: a query equal to the writer's last one takes its result
   uint64_t w_recip;         // floor(2^32 / W): the ring slot of a position without division
   const DevLayer *layers;   // L entries
   const int16_t *final_gain;
   const uint16_t *final_gain_desc;
+  const int32_t *tap_words; // L * (W + 1) * d, with taps_fast
   const uint16_t *table_b;  // vocab * d, biased
   const int16_t *keys;      // D * 16
   const uint32_t *offsets;  // D + 1

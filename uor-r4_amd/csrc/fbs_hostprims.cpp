@@ -131,21 +131,26 @@ int64_t fbs_hp_shift(int64_t v, int32_t s) { return shift(v, s); }
 int64_t fbs_hp_grid_apply(int64_t v, int16_t code) { return grid_apply(v, code); }
 
 // Every valid grid code against n inputs v[] (their low 32 bits): mismatches of the descriptor
-// form in both halves of a word, and of the gained norms' publish from its unhalved value.
+// form in both halves of a word, of the gained norms' publish from its unhalved value, and of the
+// window taps' word.
 uint64_t fbs_hp_grid_check(const int64_t *v, uint64_t n) {
   uint64_t bad = 0;
   for (int32_t code = -2047; code <= 2047; code++) {
     uint32_t field = (uint32_t)(code < 0 ? -code : code) >> 4;
     if (code != 0 && (field < 1 || field > 127)) continue;
-    uint16_t t = tap_desc((int16_t)code);
+    const int32_t tw = tap_word((int16_t)code);
+    if (tw != kTapWordNone)
+      for (uint64_t i = 0; i < n; i++)
+        bad += tap_word_apply((int32_t)v[i], tw) != grid_apply((int64_t)(int32_t)v[i], (int16_t)code);
+    uint16_t t = gain_desc((int16_t)code);
     if (t == kGridDescSlow) continue;
     const uint32_t word0 = 0xa5a50000u | t, word1 = ((uint32_t)t << 16) | 0x5a5au;
     for (uint64_t i = 0; i < n; i++) {
       int32_t v32 = (int32_t)v[i];
       const int64_t want = grid_apply((int64_t)v32, (int16_t)code);
-      bad += (tap_desc_apply(v32, word0, 0) != want) + (tap_desc_apply(v32, word1, 1) != want);
-      const int64_t h = tap_desc_half(v32, word1, 1);
-      bad += ((h + 1) >> 1 != want) + (tap_desc_half(v32, word0, 0) != h);
+      bad += (gain_desc_apply(v32, word0, 0) != want) + (gain_desc_apply(v32, word1, 1) != want);
+      const int64_t h = gain_desc_half(v32, word1, 1);
+      bad += ((h + 1) >> 1 != want) + (gain_desc_half(v32, word0, 0) != h);
       int32_t p, q;
       publish_half_pair(h, &p, &q);
       bad += p != to_exp_i32(want, kNormFineExp, kResidualExp);

@@ -112,8 +112,7 @@ FBS_HD int64_t grid_apply(int64_t v, int16_t code) {
 // The same for a 32-bit input, whose product (16 + m) v never wraps.
 FBS_HD int64_t grid_apply32(int32_t v, int16_t code) { return grid_apply((int64_t)v, code); }
 
-// A grid code prepared for the kernels (16 bits, two per word), for the window taps and the norms'
-// gains. kGridDescSlow marks a code whose right shift sh = 4 - e lies outside 1..62.
+// A norm's gain code prepared for the kernels (16 bits, two per word). kGridDescSlow marks a code whose right shift sh = 4 - e lies outside 1..62.
 constexpr uint16_t kGridDescSlow = 0xffff;
 
 // Bits 0-5 the signed multiplier
@@ -121,7 +120,7 @@ constexpr uint16_t kGridDescSlow = 0xffff;
 // p = v mul and neg = [code < 0] (the multiplier's sign bit),
 // grid_apply(v, code) = floor((p - neg + 2^(sh-1)) / 2^sh) = ((p - neg) >> (sh - 1)) + 1) >> 1.
 // Valid for the codes with 1 <= sh <= 62; |p| < 2^36.
-FBS_HD uint16_t tap_desc(int16_t code) {
+FBS_HD uint16_t gain_desc(int16_t code) {
   if (code == 0) return 0;  // multiplier 0, shift 1: ((0 >> 0) + 1) >> 1 = 0
   const uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
   const int32_t sh = 4 - ((int32_t)(c >> 4) - kGridExpBias);
@@ -130,16 +129,34 @@ FBS_HD uint16_t tap_desc(int16_t code) {
   return (uint16_t)(((uint32_t)mul & 63u) | ((uint32_t)(sh - 1) << 6));
 }
 
+// A window tap as one word M = +-(16 + m) 2^(28 - sh), for 2 <= sh <= 28 (and 0 for the zero code and
+// for sh >= 38, where every term of a 32-bit v is 0): v M + 2^27 - [M < 0] holds v's gained value
+// before its floor by 2^28, because grid_apply(v, code) = floor((v (+-(16 + m)) + 2^(sh-1) - [code <
+// 0]) / 2^sh) and the products are multiples of 2^(28 - sh). |v M| <= 2^62. kTapWordNone: no word.
+constexpr int32_t kTapWordNone = INT32_MIN;
+FBS_HD int32_t tap_word(int16_t code) {
+  if (code == 0) return 0;
+  const uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
+  const int32_t sh = 4 - ((int32_t)(c >> 4) - kGridExpBias);
+  if (sh >= 38) return 0;
+  if (sh < 2 || sh > 28) return kTapWordNone;
+  const int32_t mag = (int32_t)(16 + (c & 15)) << (28 - sh);
+  return code < 0 ? -mag : mag;
+}
+FBS_HD int64_t tap_word_apply(int32_t v, int32_t word) {
+  return ((int64_t)v * word + (int64_t)(uint32_t)((1 << 27) + (word >> 31))) >> 28;
+}
+
 // grid_apply(v, code) for the tap descriptor in bits 16 h .. 16 h + 11 of `word`.
-FBS_HD int64_t tap_desc_apply(int32_t v, uint32_t word, int h) {
+FBS_HD int64_t gain_desc_apply(int32_t v, uint32_t word, int h) {
   const int32_t mul = (int32_t)(word << (26 - 16 * h)) >> 26;  // sign-extended 6 bits
   const uint32_t shm1 = (word >> (16 * h + 6)) & 63u;
   const int64_t p = (int64_t)v * mul + (mul >> 31);            // v mul - neg
   return ((p >> shm1) + 1) >> 1;
 }
 
-// The floor before the last halving of tap_desc_apply: grid_apply(v, code) = (h + 1) >> 1.
-FBS_HD int64_t tap_desc_half(int32_t v, uint32_t word, int h) {
+// The floor before the last halving of gain_desc_apply: grid_apply(v, code) = (h + 1) >> 1.
+FBS_HD int64_t gain_desc_half(int32_t v, uint32_t word, int h) {
   const int32_t mul = (int32_t)(word << (26 - 16 * h)) >> 26;
   const uint32_t shm1 = (word >> (16 * h + 6)) & 63u;
   return ((int64_t)v * mul + (mul >> 31)) >> shm1;

@@ -276,7 +276,7 @@ __device__ __forceinline__ void norm_gain(const DevModel &M, const Seeds &sd,
     for (int k = 0; k < Q; k++)
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        out[k][c] = tap_desc_apply(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1);
+        out[k][c] = gain_desc_apply(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1);
     return;
   }
 #pragma unroll
@@ -305,7 +305,7 @@ __device__ __forceinline__ void norm_publish(const DevModel &M, const Seeds &sd,
     for (int k = 0; k < Q; k++)
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        publish_half_pair(tap_desc_half(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1),
+        publish_half_pair(gain_desc_half(norm_apply32(lo, hi, y[k][c]), c < 2 ? gdesc[k].x : gdesc[k].y, c & 1),
                           &p[k][c], &n[k][c]);
   } else {
 #pragma unroll
@@ -931,6 +931,15 @@ __device__ __forceinline__ uint32_t writer(const DevModel &M, const int32_t *q, 
   return (uint32_t)best;
 }
 
+// One window tap's terms (its words t) on the lane's four channels of a drive, added to the sums.
+// Half of the ring wave's work: 5 instructions a term (the 16-bit descriptors took 10).
+__device__ __forceinline__ void add_tap(const int4 &x, const int4 &t, int64_t (&acc)[4]) {
+  acc[0] = wadd64(acc[0], tap_word_apply(x.x, t.x));
+  acc[1] = wadd64(acc[1], tap_word_apply(x.y, t.y));
+  acc[2] = wadd64(acc[2], tap_word_apply(x.z, t.z));
+  acc[3] = wadd64(acc[3], tap_word_apply(x.w, t.w));
+}
+
 // ---------------------------------------------------------------------------------------------
 // One step of the session (RS stack/session.rs:4129-4403, TW 635-675) at ring slot `base`.
 // Returns 0 or the reference's status code; the chosen token goes to *chosen when the writer
@@ -1019,9 +1028,10 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     const DevLayer ly = M.layers[l];
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     // The layer's loads first: gains, biases and the gather program.
+    const int32_t *tw = M.tap_words + (uint64_t)l * (W + 1) * d;
     short4 g_rec[Q], g_mlp[Q], tap0[Q];
     uint2 gd_rec[Q], gd_mlp[Q];
-    uint2 td0[Q];
+    int4 tw0[Q];
     int4 cbias[Q], rbias[Q];
     int32_t dbias[Q], doff[Q];
     uint32_t pw_drive[Q][4], pw_gate[Q][4], pw_rot[Q][4], pw_dec[Q], pw_out[Q][4], pw_down[Q][4];
@@ -1033,7 +1043,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       tap0[k] = *(const short4 *)(ly.taps + ch);
       gd_rec[k] = *(const uint2 *)(ly.rec_gain_desc + ch);
       gd_mlp[k] = *(const uint2 *)(ly.mlp_gain_desc + ch);
-      td0[k] = *(const uint2 *)(ly.taps_desc + ch);
+      tw0[k] = *(const int4 *)(tw + ch);
       cbias[k] = *(const int4 *)(ly.conv_bias + ch);
       rbias[k] = *(const int4 *)(ly.gate_bias + nq + ch);
       dbias[k] = ly.gate_bias[qq];
@@ -1092,7 +1102,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       // positions back (ring slot base - s), then the drive enters slot base. Rows and taps
       // load kWindowChunk at a time; the first chunk is in flight during the rotation.
       int4 hb[kWindowChunk];
-      uint2 tb[kWindowChunk];  // tap_desc pairs: channels 0, 1 in .x, 2, 3 in .y
+      int4 tb[kWindowChunk];  // the taps' words
       auto load_chunk = [&](uint32_t s0) {
 #pragma unroll
         for (uint32_t i = 0; i < kWindowChunk; i++) {
@@ -1100,7 +1110,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
           if (s <= W) {
             const uint32_t sl = base >= s ? base - s : base + W - s;
             hb[i] = *(const int4 *)(ring_l + (uint64_t)sl * d + ch);
-            tb[i] = *(const uint2 *)(ly.taps_desc + (uint64_t)s * d + ch);
+            tb[i] = *(const int4 *)(tw + (uint64_t)s * d + ch);
           }
         }
       };
@@ -1123,24 +1133,19 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       if (lt) lt[qi[k]] = (uint8_t)root;
       int64_t wide[4];
       if (M.taps_fast) {
-        const uint2 t0 = td0[k];
-        wide[0] = wadd64(cbias[k].x, tap_desc_apply(drive[k][0], t0.x, 0));
-        wide[1] = wadd64(cbias[k].y, tap_desc_apply(drive[k][1], t0.x, 1));
-        wide[2] = wadd64(cbias[k].z, tap_desc_apply(drive[k][2], t0.y, 0));
-        wide[3] = wadd64(cbias[k].w, tap_desc_apply(drive[k][3], t0.y, 1));
+        wide[0] = cbias[k].x;
+        wide[1] = cbias[k].y;
+        wide[2] = cbias[k].z;
+        wide[3] = cbias[k].w;
+        add_tap(make_int4(drive[k][0], drive[k][1], drive[k][2], drive[k][3]), tw0[k], wide);
         for (uint32_t s0 = 1; s0 <= W; s0 += kWindowChunk) {
           if (s0 > 1) load_chunk(s0);
 #pragma unroll
           for (uint32_t i = 0; i < kWindowChunk; i++)
-            if (s0 + i <= W) {
-              wide[0] = wadd64(wide[0], tap_desc_apply(hb[i].x, tb[i].x, 0));
-              wide[1] = wadd64(wide[1], tap_desc_apply(hb[i].y, tb[i].x, 1));
-              wide[2] = wadd64(wide[2], tap_desc_apply(hb[i].z, tb[i].y, 0));
-              wide[3] = wadd64(wide[3], tap_desc_apply(hb[i].w, tb[i].y, 1));
-            }
+            if (s0 + i <= W) add_tap(hb[i], tb[i], wide);
         }
       } else {
-        // A tap outside the descriptor form somewhere in the model: the reference routine.
+        // A tap without a word somewhere in the model: the reference routine.
         const short4 t0 = tap0[k];
         wide[0] = wadd64(cbias[k].x, grid_apply(drive[k][0], t0.x));
         wide[1] = wadd64(cbias[k].y, grid_apply(drive[k][1], t0.y));
@@ -1866,15 +1871,11 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
   return 0;
 }
 
-// Tap k on the lane's four channels of x: tap_desc words (fast taps) or grid codes.
-__device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint32_t k, uint32_t ch,
-                                     const int4 &x, int64_t (&acc)[4]) {
+// Tap k of layer l on the lane's four channels of x: tap words or grid codes.
+__device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint32_t l, uint32_t k,
+                                     uint32_t ch, const int4 &x, int64_t (&acc)[4]) {
   if (M.taps_fast) {
-    const uint2 t = *(const uint2 *)(ly.taps_desc + (uint64_t)k * M.d + ch);
-    acc[0] = wadd64(acc[0], tap_desc_apply(x.x, t.x, 0));
-    acc[1] = wadd64(acc[1], tap_desc_apply(x.y, t.x, 1));
-    acc[2] = wadd64(acc[2], tap_desc_apply(x.z, t.y, 0));
-    acc[3] = wadd64(acc[3], tap_desc_apply(x.w, t.y, 1));
+    add_tap(x, *(const int4 *)(M.tap_words + ((uint64_t)l * (M.W + 1) + k) * M.d + ch), acc);
   } else {
     const short4 t = *(const short4 *)(ly.taps + (uint64_t)k * M.d + ch);
     acc[0] = wadd64(acc[0], grid_apply(x.x, t.x));
@@ -1888,37 +1889,32 @@ __device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint
 // s positions back (ring slot base - s), for s = s1..W, added to acc (session.rs:4842-4868;
 // wrapping sums, so the order of the terms does not matter). Rows and taps load kWindowChunk at
 // a time.
-__device__ __forceinline__ void window_sum(const DevModel &M, const DevLayer &ly,
+__device__ __forceinline__ void window_sum(const DevModel &M, const DevLayer &ly, uint32_t l,
                                            const int32_t *ring_l, uint32_t base, uint32_t s1,
                                            uint32_t ch, int64_t (&acc)[4], uint32_t s2 = 0) {
   const uint32_t d = M.d, W = s2 ? s2 : M.W;  // taps s1..W (the last tap s2 when given)
   if (M.taps_fast) {
+    const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * d + ch;
     for (uint32_t s0 = s1; s0 <= W; s0 += kWindowChunk) {
-      int4 hb[kWindowChunk];
-      uint2 tb[kWindowChunk];  // tap_desc pairs: channels 0, 1 in .x, 2, 3 in .y
+      int4 hb[kWindowChunk], tb[kWindowChunk];  // the rows and the taps' words
 #pragma unroll
       for (uint32_t i = 0; i < kWindowChunk; i++) {
         const uint32_t s = s0 + i;
         if (s <= W) {
           const uint32_t sl = base >= s ? base - s : base + M.W - s;
           hb[i] = *(const int4 *)(ring_l + (uint64_t)sl * d + ch);
-          tb[i] = *(const uint2 *)(ly.taps_desc + (uint64_t)s * d + ch);
+          tb[i] = *(const int4 *)(tw + (uint64_t)s * d);
         }
       }
 #pragma unroll
       for (uint32_t i = 0; i < kWindowChunk; i++)
-        if (s0 + i <= W) {
-          acc[0] = wadd64(acc[0], tap_desc_apply(hb[i].x, tb[i].x, 0));
-          acc[1] = wadd64(acc[1], tap_desc_apply(hb[i].y, tb[i].x, 1));
-          acc[2] = wadd64(acc[2], tap_desc_apply(hb[i].z, tb[i].y, 0));
-          acc[3] = wadd64(acc[3], tap_desc_apply(hb[i].w, tb[i].y, 1));
-        }
+        if (s0 + i <= W) add_tap(hb[i], tb[i], acc);
     }
   } else {
-    // A tap outside the descriptor form somewhere in the model: the reference routine.
+    // A tap without a word somewhere in the model: the reference routine.
     for (uint32_t s = s1; s <= W; s++) {
       const uint32_t sl = base >= s ? base - s : base + M.W - s;
-      tap4(M, ly, s, ch, *(const int4 *)(ring_l + (uint64_t)sl * d + ch), acc);
+      tap4(M, ly, l, s, ch, *(const int4 *)(ring_l + (uint64_t)sl * d + ch), acc);
     }
   }
 }
@@ -1964,7 +1960,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       if (fresh) {
 #pragma unroll
         for (int c = 0; c < 4; c++) sum[k][c] = 0;
-        if (qv[k]) window_sum(M, ly, ring_l, base, 1, ch, sum[k]);
+        if (qv[k]) window_sum(M, ly, l, ring_l, base, 1, ch, sum[k]);
       } else {
         const longlong2 *hp = (const longlong2 *)(hist_l + ch);
         const longlong2 a = hp[0], b = hp[1];
@@ -1978,7 +1974,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
     for (int k = 0; k < Q; k++) {
 #pragma unroll
       for (int c = 0; c < 4; c++) part[k][c] = 0;
-      if (qv[k]) window_sum(M, ly, ring_l, next, 2, 4 * qi[k], part[k], split);
+      if (qv[k]) window_sum(M, ly, l, ring_l, next, 2, 4 * qi[k], part[k], split);
     }
     // The first MLP group's gather words, for after barrier 3.
     uint32_t pg[4], pu[4];
@@ -1996,7 +1992,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
                            S.xbar[pw_drive[k][3]]);
       // Tap 0 on the drive and the conv bias, then the drive enters ring slot base.
       int64_t wide[4] = {cbias[k].x, cbias[k].y, cbias[k].z, cbias[k].w};
-      tap4(M, ly, 0, ch, drive[k], wide);
+      tap4(M, ly, l, 0, ch, drive[k], wide);
 #pragma unroll
       for (int c = 0; c < 4; c++) S.wide[ch + c] = wadd64(wide[c], sum[k][c]);
       *(int4 *)(ring_l + (uint64_t)base * d + ch) = drive[k];
@@ -2026,8 +2022,8 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       if (!qv[k]) continue;
       const uint32_t ch = 4 * qi[k];
       int64_t acc[4] = {part[k][0], part[k][1], part[k][2], part[k][3]};
-      tap4(M, ly, 1, ch, drive[k], acc);
-      if (split < W) window_sum(M, ly, ring_l, next, split + 1, ch, acc);
+      tap4(M, ly, l, 1, ch, drive[k], acc);
+      if (split < W) window_sum(M, ly, l, ring_l, next, split + 1, ch, acc);
       longlong2 *hp = (longlong2 *)(hist_l + ch);
       hp[0] = make_longlong2(acc[0], acc[1]);
       hp[1] = make_longlong2(acc[2], acc[3]);
