@@ -97,26 +97,6 @@ FBS_HD uint32_t ham_nibble(const int64_t *unit, const int64_t (&p)[4]) {
          (uint32_t)(o[3] >= 0) << 3;
 }
 
-// A load made a global load: the read's tables are reached through pointers read from memory
-// (DevHamRead), which the compiler would otherwise load with flat instructions, and a flat load
-// counts against the LDS counter as well, so every later wait for an LDS read would wait for it.
-// 8- and 16-byte types load as plain integers and vectors (no constructor of a vector type takes
-// a global-space reference).
-template <class T>
-__device__ __forceinline__ T gload(const T *p) {
-  if constexpr (sizeof(T) == 8) {
-    typedef __attribute__((address_space(1))) const unsigned long long *G8;
-    return __builtin_bit_cast(T, *(G8)p);
-  } else if constexpr (sizeof(T) == 16) {
-    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(1))) const v4u *G16;
-    return __builtin_bit_cast(T, *(G16)p);
-  } else {
-    typedef __attribute__((address_space(1))) const T *GP;
-    return *(GP)p;
-  }
-}
-
 // ham_nibble with the unit's words read by global loads (the read's tables are reached through
 // pointers read from memory, which the compiler would otherwise load as flat).
 __device__ __forceinline__ uint32_t ham_nibble_g(const int64_t *unit, const int64_t (&p)[4]) {

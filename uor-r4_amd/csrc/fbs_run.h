@@ -38,6 +38,55 @@ static_assert(kRsqrtSeedWords + kRecipSeedWords == kSeedWords, "seed table size"
 template <int Q, bool HM = false>
 constexpr bool kPairStateGlobal = Q >= 2 || HM;
 
+// A load made a global load: the layers' and the reads' tables are reached through pointers read
+// from memory (DevLayer, DevHamRead), which the compiler would otherwise load with flat
+// instructions, and a flat load counts against the LDS counter as well, so every later wait for an
+// LDS read would wait for it. 8- and 16-byte types load as plain integers and vectors (no
+// constructor of a vector type takes a global-space reference).
+template <class T>
+__device__ __forceinline__ T gload(const T *p) {
+  if constexpr (sizeof(T) == 8) {
+    typedef __attribute__((address_space(1))) const unsigned long long *G8;
+    return __builtin_bit_cast(T, *(G8)p);
+  } else if constexpr (sizeof(T) == 16) {
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) const v4u *G16;
+    return __builtin_bit_cast(T, *(G16)p);
+  } else {
+    typedef __attribute__((address_space(1))) const T *GP;
+    return *(GP)p;
+  }
+}
+// The value `bytes` past a uniform base: a scalar base and a 32-bit offset, without a 64-bit address
+// on the vector unit.
+template <class T>
+__device__ __forceinline__ T gat(const void *base, uint32_t bytes) {
+  typedef __attribute__((address_space(1))) const char *G;
+  if constexpr (sizeof(T) == 8) {
+    typedef __attribute__((address_space(1))) const unsigned long long *G8;
+    return __builtin_bit_cast(T, *(G8)((G)base + bytes));
+  } else if constexpr (sizeof(T) == 16) {
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) const v4u *G16;
+    return __builtin_bit_cast(T, *(G16)((G)base + bytes));
+  } else {
+    typedef __attribute__((address_space(1))) const T *GP;
+    return *(GP)((G)base + bytes);
+  }
+}
+// Layer l's pointers by scalar loads.
+__device__ __forceinline__ DevLayer load_layer(const DevModel &M, uint32_t l) {
+  typedef __attribute__((address_space(4))) const uint64_t *C;
+  constexpr int n = sizeof(DevLayer) / 8;
+  C src = (C)(M.layers + l);
+  struct Words {
+    uint64_t v[n];
+  } w;
+#pragma unroll
+  for (int i = 0; i < n; i++) w.v[i] = src[i];
+  return __builtin_bit_cast(DevLayer, w);
+}
+
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -336,7 +385,7 @@ __device__ __forceinline__ void publish16(int32_t *xbar, uint32_t channel0, cons
 }
 
 __device__ __forceinline__ uint32_t prog_word(const uint16_t *prog, uint32_t slot, uint32_t lane) {
-  return prog[slot * kWave + lane];
+  return gat<uint16_t>(prog, 2 * (slot * kWave + lane));
 }
 
 // The snapped transition or gate (RS stack/kernels.rs:1474-1557), out of line: the 120-root
@@ -493,7 +542,7 @@ __device__ __forceinline__ void gate_mul(const int64_t (&g)[4], const int64_t (&
 // ---------------------------------------------------------------------------------------------
 // The writer.
 
-constexpr uint32_t kWindowChunk = 8; // window rows in flight per lane
+constexpr uint32_t kWindowChunk = 8; // window rows in flight per lane (one wavefront a sequence)
 constexpr uint32_t kPrologueLayers = 8;  // layers whose state words a lane loads all at once
 constexpr int kScanUnroll = 4;       // row groups per pipeline stage
 
@@ -1025,7 +1074,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     }
   }
   for (uint32_t l = 0; l < M.L; l++) {
-    const DevLayer ly = M.layers[l];
+    const DevLayer ly = load_layer(M, l);
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     // The layer's loads first: gains, biases and the gather program.
     const int32_t *tw = M.tap_words + (uint64_t)l * (W + 1) * d;
@@ -1038,16 +1087,16 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const uint32_t qq = qv[k] ? qi[k] : 0, ch = 4 * qq;
-      g_rec[k] = *(const short4 *)(ly.rec_gain + ch);
-      g_mlp[k] = *(const short4 *)(ly.mlp_gain + ch);
-      tap0[k] = *(const short4 *)(ly.taps + ch);
-      gd_rec[k] = *(const uint2 *)(ly.rec_gain_desc + ch);
-      gd_mlp[k] = *(const uint2 *)(ly.mlp_gain_desc + ch);
+      g_rec[k] = gat<short4>(ly.rec_gain, 2 * ch);
+      g_mlp[k] = gat<short4>(ly.mlp_gain, 2 * ch);
+      tap0[k] = gload((const short4 *)(ly.taps + ch));
+      gd_rec[k] = gat<uint2>(ly.rec_gain_desc, 2 * ch);
+      gd_mlp[k] = gat<uint2>(ly.mlp_gain_desc, 2 * ch);
       tw0[k] = *(const int4 *)(tw + ch);
-      cbias[k] = *(const int4 *)(ly.conv_bias + ch);
-      rbias[k] = *(const int4 *)(ly.gate_bias + nq + ch);
-      dbias[k] = ly.gate_bias[qq];
-      doff[k] = ly.decay_offset[qq];
+      cbias[k] = gat<int4>(ly.conv_bias, 4 * ch);
+      rbias[k] = gat<int4>(ly.gate_bias, 4 * (nq + ch));
+      dbias[k] = gat<int32_t>(ly.gate_bias, 4 * qq);
+      doff[k] = gat<int32_t>(ly.decay_offset, 4 * qq);
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         pw_drive[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * k + c, lane);
@@ -1154,7 +1203,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
         for (uint32_t s = 1; s <= W; s++) {
           const uint32_t sl = base >= s ? base - s : base + W - s;
           const int4 hh = *(const int4 *)(ring_l + (uint64_t)sl * d + ch);
-          const short4 t = *(const short4 *)(ly.taps + (uint64_t)s * d + ch);
+          const short4 t = gload((const short4 *)(ly.taps + (uint64_t)s * d + ch));
           wide[0] = wadd64(wide[0], grid_apply(hh.x, t.x));
           wide[1] = wadd64(wide[1], grid_apply(hh.y, t.y));
           wide[2] = wadd64(wide[2], grid_apply(hh.z, t.z));
@@ -1436,8 +1485,8 @@ __device__ __forceinline__ void pair_mlp_words(const DevModel &M, const DevLayer
   if (j < M.mpl) {
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      pg[c] = gload(ly.prog + (M.s_mlp_gate + 4 * j + c) * kWave + lane);
-      pu[c] = gload(ly.prog + (M.s_mlp_up + 4 * j + c) * kWave + lane);
+      pg[c] = prog_word(ly.prog, M.s_mlp_gate + 4 * j + c, lane);
+      pu[c] = prog_word(ly.prog, M.s_mlp_up + 4 * j + c, lane);
     }
   }
 }
@@ -1558,7 +1607,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
   }
   clk.lap(kPartEmbed);
   for (uint32_t l = 0; l < M.L; l++) {
-    const DevLayer ly = M.layers[l];
+    const DevLayer ly = load_layer(M, l);
     short4 g_rec[Q], g_mlp[Q];
     uint2 gd_rec[Q], gd_mlp[Q];
     int4 rbias[Q];
@@ -1571,8 +1620,8 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
 #pragma unroll
       for (int k = 0; k < Q; k++) {
         const uint32_t ch = 4 * (qv[k] ? qi[k] : 0);
-        g_mlp[k] = *(const short4 *)(ly.mlp_gain + ch);
-        gd_mlp[k] = *(const uint2 *)(ly.mlp_gain_desc + ch);
+        g_mlp[k] = gat<short4>(ly.mlp_gain, 2 * ch);
+        gd_mlp[k] = gat<uint2>(ly.mlp_gain_desc, 2 * ch);
 #pragma unroll
         for (int c = 0; c < 4; c++) pw_down[k][c] = prog_word(ly.prog, M.s_mlp_down + 4 * k + c, lane);
       }
@@ -1580,11 +1629,11 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const uint32_t qq = qv[k] ? qi[k] : 0, ch = 4 * qq;
-      g_rec[k] = *(const short4 *)(ly.rec_gain + ch);
-      gd_rec[k] = *(const uint2 *)(ly.rec_gain_desc + ch);
-      rbias[k] = *(const int4 *)(ly.gate_bias + nq + ch);
-      dbias[k] = ly.gate_bias[qq];
-      doff[k] = ly.decay_offset[qq];
+      g_rec[k] = gat<short4>(ly.rec_gain, 2 * ch);
+      gd_rec[k] = gat<uint2>(ly.rec_gain_desc, 2 * ch);
+      rbias[k] = gat<int4>(ly.gate_bias, 4 * (nq + ch));
+      dbias[k] = gat<int32_t>(ly.gate_bias, 4 * qq);
+      doff[k] = gat<int32_t>(ly.decay_offset, 4 * qq);
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         pw_rot[k][c] = prog_word(ly.prog, M.s_rec_gate + Q + 4 * k + c, lane);
@@ -1752,11 +1801,6 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
         }
     }
     clk.lap(kPartTransport);
-    // The feed-forward block's gather words, loaded a phase ahead: the norm's factor is a call,
-    // whose entry waits for every load in flight, so loads issued just before it are waited for
-    // whole (global loads, so that the LDS waits in between do not wait for them).
-    uint32_t pg[4], pu[4];
-    pair_mlp_words(M, ly, lane, 0, pg, pu);
     // quantize16 over the d outputs (kernels.rs:545-553), then gather16 of rec_out.
     const int32_t bl = wave_bitlen_max(mx);
 #pragma unroll
@@ -1771,8 +1815,11 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
         for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], S.xbar[pw_out[k][c]]);
     wave_sync();
     clk.lap(kPartResidualRec);
-    // ---- feed-forward block: wave 0 takes the even quaternion groups.
+    // ---- feed-forward block: wave 0 takes the even quaternion groups. Its first gather words land
+    // during the norm.
     if constexpr (Q != 1) load_ffn();
+    uint32_t pg[4], pu[4];
+    pair_mlp_words(M, ly, lane, 0, pg, pu);
     norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     clk.sync(kPartNormMlp, kPartSync3);  // 3: the normed activations
     int64_t mo[4];
@@ -1877,7 +1924,7 @@ __device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint
   if (M.taps_fast) {
     add_tap(x, *(const int4 *)(M.tap_words + ((uint64_t)l * (M.W + 1) + k) * M.d + ch), acc);
   } else {
-    const short4 t = *(const short4 *)(ly.taps + (uint64_t)k * M.d + ch);
+    const short4 t = gload((const short4 *)(ly.taps + (uint64_t)k * M.d + ch));
     acc[0] = wadd64(acc[0], grid_apply(x.x, t.x));
     acc[1] = wadd64(acc[1], grid_apply(x.y, t.y));
     acc[2] = wadd64(acc[2], grid_apply(x.z, t.z));
@@ -1887,27 +1934,27 @@ __device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint
 
 // The window over earlier positions for a step whose ring slot is `base`: tap s on the drive
 // s positions back (ring slot base - s), for s = s1..W, added to acc (session.rs:4842-4868;
-// wrapping sums, so the order of the terms does not matter). Rows and taps load kWindowChunk at
-// a time.
+// wrapping sums, so the order of the terms does not matter). Rows and taps load N at a time.
+template <uint32_t N>
 __device__ __forceinline__ void window_sum(const DevModel &M, const DevLayer &ly, uint32_t l,
                                            const int32_t *ring_l, uint32_t base, uint32_t s1,
                                            uint32_t ch, int64_t (&acc)[4], uint32_t s2 = 0) {
   const uint32_t d = M.d, W = s2 ? s2 : M.W;  // taps s1..W (the last tap s2 when given)
   if (M.taps_fast) {
-    const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * d + ch;
-    for (uint32_t s0 = s1; s0 <= W; s0 += kWindowChunk) {
-      int4 hb[kWindowChunk], tb[kWindowChunk];  // the rows and the taps' words
+    const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * d;
+    for (uint32_t s0 = s1; s0 <= W; s0 += N) {
+      int4 hb[N], tb[N];  // the rows and the taps' words
 #pragma unroll
-      for (uint32_t i = 0; i < kWindowChunk; i++) {
+      for (uint32_t i = 0; i < N; i++) {
         const uint32_t s = s0 + i;
         if (s <= W) {
           const uint32_t sl = base >= s ? base - s : base + M.W - s;
-          hb[i] = *(const int4 *)(ring_l + (uint64_t)sl * d + ch);
-          tb[i] = *(const int4 *)(tw + (uint64_t)s * d);
+          hb[i] = gat<int4>(ring_l, 4 * (sl * d + ch));
+          tb[i] = gat<int4>(tw, 4 * (s * d + ch));
         }
       }
 #pragma unroll
-      for (uint32_t i = 0; i < kWindowChunk; i++)
+      for (uint32_t i = 0; i < N; i++)
         if (s0 + i <= W) add_tap(hb[i], tb[i], acc);
     }
   } else {
@@ -1934,6 +1981,9 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
   if (tok >= M.vocab) return 1;
   const uint32_t d = M.d, W = M.W;
   const uint32_t next = base + 1 == W ? 0 : base + 1;  // the next step's ring slot
+  // Rows and taps in flight after barrier 2: a 16-row window's rest at once where a lane holds one
+  // quaternion (its registers allow it), so that the wait is one round trip and not two.
+  constexpr uint32_t kRows = Q == 1 ? 12 : 8;
   // Windows of 16 rows or more: the next step's taps 2..split are summed before barrier 1, where
   // this wave waits for the norm, and taps split+1..W after barrier 2 (none of their ring rows is
   // the one this step writes); shorter windows sum every tap after barrier 2. Measured: W = 32,
@@ -1941,7 +1991,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
   // 2..4 first 1.7 % faster than none (2..6 slower in one-token serving launches).
   const uint32_t split = W > 16 ? 1 + (W - 1) / 2 : W == 16 ? 1 + (W - 1) / 4 : 1;
   for (uint32_t l = 0; l < M.L; l++) {
-    const DevLayer ly = M.layers[l];
+    const DevLayer ly = load_layer(M, l);
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     int64_t *hist_l = hist + (uint64_t)l * d;
     int4 cbias[Q];
@@ -1951,7 +2001,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const uint32_t ch = 4 * (qv[k] ? qi[k] : 0);
-      cbias[k] = *(const int4 *)(ly.conv_bias + ch);
+      cbias[k] = gat<int4>(ly.conv_bias, 4 * ch);
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         pw_drive[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * k + c, lane);
@@ -1960,10 +2010,9 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       if (fresh) {
 #pragma unroll
         for (int c = 0; c < 4; c++) sum[k][c] = 0;
-        if (qv[k]) window_sum(M, ly, l, ring_l, base, 1, ch, sum[k]);
+        if (qv[k]) window_sum<kRows>(M, ly, l, ring_l, base, 1, ch, sum[k]);
       } else {
-        const longlong2 *hp = (const longlong2 *)(hist_l + ch);
-        const longlong2 a = hp[0], b = hp[1];
+        const longlong2 a = gat<longlong2>(hist_l, 8 * ch), b = gat<longlong2>(hist_l, 8 * ch + 16);
         sum[k][0] = a.x;
         sum[k][1] = a.y;
         sum[k][2] = b.x;
@@ -1974,7 +2023,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
     for (int k = 0; k < Q; k++) {
 #pragma unroll
       for (int c = 0; c < 4; c++) part[k][c] = 0;
-      if (qv[k]) window_sum(M, ly, l, ring_l, next, 2, 4 * qi[k], part[k], split);
+      if (qv[k]) window_sum<8>(M, ly, l, ring_l, next, 2, 4 * qi[k], part[k], split);
     }
     // The first MLP group's gather words, for after barrier 3.
     uint32_t pg[4], pu[4];
@@ -2023,7 +2072,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       const uint32_t ch = 4 * qi[k];
       int64_t acc[4] = {part[k][0], part[k][1], part[k][2], part[k][3]};
       tap4(M, ly, l, 1, ch, drive[k], acc);
-      if (split < W) window_sum(M, ly, l, ring_l, next, split + 1, ch, acc);
+      if (split < W) window_sum<kRows>(M, ly, l, ring_l, next, split + 1, ch, acc);
       longlong2 *hp = (longlong2 *)(hist_l + ch);
       hp[0] = make_longlong2(acc[0], acc[1]);
       hp[1] = make_longlong2(acc[2], acc[3]);
