@@ -644,13 +644,12 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
   if (M.qpl == 3) M.qpl = 4;
   M.mpl = (M.nm + kWave - 1) / kWave;
   const uint32_t Q = M.qpl, MP = M.mpl;
-  M.s_rec_in = 0;
-  M.s_rec_gate = 8 * Q;
-  M.s_rec_out = 13 * Q;
-  M.s_mlp_gate = 17 * Q;
-  M.s_mlp_up = 17 * Q + 4 * MP;
-  M.s_mlp_down = 17 * Q + 8 * MP;
-  M.nslots = 21 * Q + 8 * MP;
+  M.p_rec = 0;
+  M.p_rot = 16 * kWave * Q;
+  M.p_mlp = 2 * M.p_rot;
+  M.p_down = M.p_mlp + 16 * kWave * MP;
+  M.p_dec = M.p_down + 8 * kWave * Q;
+  M.prog_words = M.p_dec / 2 + kWave * Q;
   M.xbar_words = 2 * (d > mlp ? d : mlp);
   M.identity_rows = r.head == 1;
   M.taps_fast = 1;
@@ -706,27 +705,31 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
     if ((st = h->upload(ly.conv_bias, d, &dl.conv_bias))) return done(st);
     if ((st = h->upload(ly.gate_bias, d / 4 + d, &dl.gate_bias))) return done(st);
     if ((st = h->upload(ly.decay_offset, d / 4, &dl.decay_offset))) return done(st);
-    std::vector<uint16_t> prog((size_t)M.nslots * kWave, 0);
-    auto put = [&](uint32_t slot, uint32_t lane, uint16_t w) { prog[(size_t)slot * kWave + lane] = w; };
+    std::vector<uint16_t> prog(M.prog_words, 0);
+    // Word c of the `per` words that lane `lane` holds in group k of the part at byte offset `part`:
+    // the crossbar word's byte offset.
+    auto put = [&](uint32_t part, uint32_t per, uint32_t k, uint32_t lane, uint32_t c, uint16_t w) {
+      prog[part / 2 + (size_t)per * (k * kWave + lane) + c] = (uint16_t)(4 * w);
+    };
     for (uint32_t lane = 0; lane < kWave; lane++) {
       for (uint32_t k = 0; k < Q; k++) {
         uint32_t q = lane + kWave * k;
         if (q >= M.nq) continue;
         for (uint32_t c = 0; c < 4; c++) {
-          put(M.s_rec_in + 4 * k + c, lane, prog_word(ly.rec_in, 4 * q + c));
-          put(M.s_rec_in + 4 * Q + 4 * k + c, lane, prog_word(ly.rec_in, d + 4 * q + c));
-          put(M.s_rec_gate + Q + 4 * k + c, lane, prog_word(ly.rec_gate, M.nq + 4 * q + c));
-          put(M.s_rec_out + 4 * k + c, lane, prog_word(ly.rec_out, 4 * q + c));
-          put(M.s_mlp_down + 4 * k + c, lane, prog_word(ly.mlp_down, 4 * q + c));
+          put(M.p_rec, 8, k, lane, c, prog_word(ly.rec_in, 4 * q + c));
+          put(M.p_rec, 8, k, lane, 4 + c, prog_word(ly.rec_in, d + 4 * q + c));
+          put(M.p_rot, 8, k, lane, c, prog_word(ly.rec_gate, M.nq + 4 * q + c));
+          put(M.p_rot, 8, k, lane, 4 + c, prog_word(ly.rec_out, 4 * q + c));
+          put(M.p_down, 4, k, lane, c, prog_word(ly.mlp_down, 4 * q + c));
         }
-        put(M.s_rec_gate + k, lane, prog_word(ly.rec_gate, q));
+        put(M.p_dec, 1, k, lane, 0, prog_word(ly.rec_gate, q));
       }
       for (uint32_t j = 0; j < MP; j++) {
         uint32_t mq = lane + kWave * j;
         if (mq >= M.nm) continue;
         for (uint32_t c = 0; c < 4; c++) {
-          put(M.s_mlp_gate + 4 * j + c, lane, prog_word(ly.mlp_gate, 4 * mq + c));
-          put(M.s_mlp_up + 4 * j + c, lane, prog_word(ly.mlp_up, 4 * mq + c));
+          put(M.p_mlp, 8, j, lane, c, prog_word(ly.mlp_gate, 4 * mq + c));
+          put(M.p_mlp, 8, j, lane, 4 + c, prog_word(ly.mlp_up, 4 * mq + c));
         }
       }
     }

@@ -5,8 +5,8 @@
 //   per layer: gains (d i16) and their descriptors (gain_desc; fbs_int.h), window taps ((W+1) x d
 //              i16, tap s = s positions back) and their words (tap_word, all layers together),
 //              conv_bias (d i32), gate_bias (d/4 + d i32), decay_offset (d/4 i32), and the
-//              layer's gather program: [slot][64 lanes] u16 LDS word indices that carry out the
-//              six FBS projections (stack_fbs_gather, session.rs:4037-4053) for this lane mapping;
+//              layer's gather program: per lane, u16 LDS byte offsets that carry out the six
+//              FBS projections (stack_fbs_gather, session.rs:4037-4053) for this lane mapping;
 //   writer: the table as biased u16 rows (v ^ 0x8000, vocab x d), drawer keys (D x 16 i16:
 //           first-block key then last-block key), CSR drawer offsets (D + 1) and members;
 //   per-sequence work (the library's, sized for the resident grid): the causal window ring,
@@ -39,7 +39,7 @@ struct DevLayer {
   const int32_t *conv_bias;     // d
   const int32_t *gate_bias;     // d/4 + d
   const int32_t *decay_offset;  // d/4
-  const uint16_t *prog;         // nslots * 64
+  const uint16_t *prog;         // the gather program (DevModel::p_*), prog_words entries
   const uint16_t *rec_gain_desc;
   const uint16_t *mlp_gain_desc;
 };
@@ -98,7 +98,10 @@ struct DevHam {
 struct DevModel {
   uint32_t vocab, d, m, L, W, D, P, head, context, raw_gates, raw_transition;
   uint32_t nq, nm, mpl, qpl;
-  uint32_t nslots, s_rec_in, s_rec_gate, s_rec_out, s_mlp_gate, s_mlp_up, s_mlp_down;
+  // The gather program's byte offsets, [group][64 lanes] each: eight words a lane of drive and output
+  // gate (qpl groups), of rotation and rec_out (qpl), of MLP gate and up (mpl); four of mlp_down
+  // (qpl); one of the decay (qpl).
+  uint32_t prog_words, p_rec, p_rot, p_mlp, p_down, p_dec;
   uint32_t xbar_words;      // 2 * max(d, m)
   uint32_t identity_rows;   // the nearest head: one drawer holding every token
   uint32_t taps_fast;       // every window tap has a word (tap_word != kTapWordNone)

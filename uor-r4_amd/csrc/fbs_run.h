@@ -384,8 +384,21 @@ __device__ __forceinline__ void publish16(int32_t *xbar, uint32_t channel0, cons
   dst[1] = make_int4(p[2], n[2], p[3], n[3]);
 }
 
-__device__ __forceinline__ uint32_t prog_word(const uint16_t *prog, uint32_t slot, uint32_t lane) {
-  return gat<uint16_t>(prog, 2 * (slot * kWave + lane));
+// The crossbar word of a gather: `pair` holds two LDS byte offsets, the low half first.
+__device__ __forceinline__ int32_t gather(const int32_t *xbar, uint32_t pair, int half) {
+  return *(const int32_t *)((const char *)xbar + (half ? pair >> 16 : pair & 0xffffu));
+}
+// A lane's gather words, laid out so that one load brings what one phase needs: quaternion k's drive
+// and output gate, or its rotation and rec_out, or MLP quaternion group j's gate and up (16 bytes),
+// and its mlp_down (8 bytes); one load a word took four times the loads and twice the registers.
+__device__ __forceinline__ uint4 gather8(const DevLayer &ly, uint32_t at, uint32_t k, uint32_t lane) {
+  return gat<uint4>(ly.prog, at + 16 * (k * kWave + lane));
+}
+__device__ __forceinline__ uint2 gather4(const DevLayer &ly, uint32_t at, uint32_t k, uint32_t lane) {
+  return gat<uint2>(ly.prog, at + 8 * (k * kWave + lane));
+}
+__device__ __forceinline__ uint32_t gather1(const DevLayer &ly, uint32_t at, uint32_t k, uint32_t lane) {
+  return gat<uint16_t>(ly.prog, at + 2 * (k * kWave + lane));
 }
 
 // The snapped transition or gate (RS stack/kernels.rs:1474-1557), out of line: the 120-root
@@ -480,7 +493,7 @@ __device__ __noinline__ Wide4 hamilton32_slow(int4 a, int64_t b0, int64_t b1, in
 }
 __device__ __forceinline__ void wave_hamilton32(const int32_t (&a)[4], const int64_t (&b)[4], int64_t (&H)[4],
                                                 int64_t (&L)[4]) {
-  if (__all(split_ok(b[0]) & split_ok(b[1]) & split_ok(b[2]) & split_ok(b[3]))) {
+  if (__all(split_ok(b[0]) && split_ok(b[1]) && split_ok(b[2]) && split_ok(b[3]))) {
     hamilton32_split(a, b, H, L);
   } else {
     const Wide4 o = hamilton32_slow(make_int4(a[0], a[1], a[2], a[3]), b[0], b[1], b[2], b[3]);
@@ -1083,7 +1096,9 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     int4 tw0[Q];
     int4 cbias[Q], rbias[Q];
     int32_t dbias[Q], doff[Q];
-    uint32_t pw_drive[Q][4], pw_gate[Q][4], pw_rot[Q][4], pw_dec[Q], pw_out[Q][4], pw_down[Q][4];
+    uint4 pw_rec[Q], pw_rot[Q];
+    uint2 pw_down[Q];
+    uint32_t pw_dec[Q];
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const uint32_t qq = qv[k] ? qi[k] : 0, ch = 4 * qq;
@@ -1097,15 +1112,10 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       rbias[k] = gat<int4>(ly.gate_bias, 4 * (nq + ch));
       dbias[k] = gat<int32_t>(ly.gate_bias, 4 * qq);
       doff[k] = gat<int32_t>(ly.decay_offset, 4 * qq);
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        pw_drive[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * k + c, lane);
-        pw_gate[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * Q + 4 * k + c, lane);
-        pw_rot[k][c] = prog_word(ly.prog, M.s_rec_gate + Q + 4 * k + c, lane);
-        pw_out[k][c] = prog_word(ly.prog, M.s_rec_out + 4 * k + c, lane);
-        pw_down[k][c] = prog_word(ly.prog, M.s_mlp_down + 4 * k + c, lane);
-      }
-      pw_dec[k] = prog_word(ly.prog, M.s_rec_gate + k, lane);
+      pw_rec[k] = gather8(ly, M.p_rec, k, lane);
+      pw_rot[k] = gather8(ly, M.p_rot, k, lane);
+      pw_down[k] = gather4(ly, M.p_down, k, lane);
+      pw_dec[k] = gather1(ly, M.p_dec, k, lane);
     }
     // ---- recurrence block
     norm_publish<Q>(M, S.seeds, x, qv, qi, g_rec, gd_rec, S.xbar);
@@ -1116,11 +1126,11 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       const int32_t rb[4] = {rbias[k].x, rbias[k].y, rbias[k].z, rbias[k].w};
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        drive[k][c] = S.xbar[pw_drive[k][c]];
-        gv[k][c] = S.xbar[pw_gate[k][c]];
-        rot[k][c] = sat_add32(S.xbar[pw_rot[k][c]], rb[c]);
+        drive[k][c] = gather(S.xbar, c < 2 ? pw_rec[k].x : pw_rec[k].y, c & 1);
+        gv[k][c] = gather(S.xbar, c < 2 ? pw_rec[k].z : pw_rec[k].w, c & 1);
+        rot[k][c] = sat_add32(gather(S.xbar, c < 2 ? pw_rot[k].x : pw_rot[k].y, c & 1), rb[c]);
       }
-      dec[k] = sat_add32(S.xbar[pw_dec[k]], dbias[k]);
+      dec[k] = sat_add32(gather(S.xbar, pw_dec[k], 0), dbias[k]);
     }
     wave_sync();
     int64_t sc[Q][4];
@@ -1255,17 +1265,12 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     for (int k = 0; k < Q; k++)
       if (qv[k])
 #pragma unroll
-        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], S.xbar[pw_out[k][c]]);
+        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], gather(S.xbar, c < 2 ? pw_rot[k].z : pw_rot[k].w, c & 1));
     wave_sync();
     // ---- feed-forward block: the Hamilton gate of mlp_gate on mlp_up (session.rs:4005-4025).
     // The gather words of MLP quaternion group j load one group ahead (the first during the
     // norm), so that their latency hides behind the previous work.
-    uint32_t pg[4], pu[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      pg[c] = prog_word(ly.prog, M.s_mlp_gate + c, lane);
-      pu[c] = prog_word(ly.prog, M.s_mlp_up + c, lane);
-    }
+    uint4 pw_mlp = gather8(ly, M.p_mlp, 0, lane);
     norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     wave_sync();
     uint64_t mmx = 0;
@@ -1275,16 +1280,10 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       int32_t gq[4], up[4];
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        gq[c] = S.xbar[pg[c]];
-        up[c] = S.xbar[pu[c]];
+        gq[c] = gather(S.xbar, c < 2 ? pw_mlp.x : pw_mlp.y, c & 1);
+        up[c] = gather(S.xbar, c < 2 ? pw_mlp.z : pw_mlp.w, c & 1);
       }
-      if (j + 1 < M.mpl) {
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          pg[c] = prog_word(ly.prog, M.s_mlp_gate + 4 * (j + 1) + c, lane);
-          pu[c] = prog_word(ly.prog, M.s_mlp_up + 4 * (j + 1) + c, lane);
-        }
-      }
+      if (j + 1 < M.mpl) pw_mlp = gather8(ly, M.p_mlp, j + 1, lane);
       if (mq < M.nm) {
         int64_t mo[4];
         const uint32_t mroot = mlp_gate(M, S.seeds, gq, up, mo);
@@ -1315,7 +1314,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     for (int k = 0; k < Q; k++)
       if (qv[k])
 #pragma unroll
-        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], S.xbar[pw_down[k][c]]);
+        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], gather(S.xbar, c < 2 ? pw_down[k].x : pw_down[k].y, c & 1));
     wave_sync();
     if (HM) {  // the stream read after l + 1 layers (session.rs:4252-4276)
       const int32_t r = M.ham.at[l + 1];
@@ -1478,25 +1477,12 @@ __device__ __forceinline__ void pair_requant(const DevModel &M, const Lds &S, ui
   }
 }
 
-// MLP group j's gather words (gate and up) for this lane, nothing past the last group; read by
-// global loads, which the LDS waits before their use do not wait for (a flat load's would).
-__device__ __forceinline__ void pair_mlp_words(const DevModel &M, const DevLayer &ly, uint32_t lane,
-                                               uint32_t j, uint32_t (&pg)[4], uint32_t (&pu)[4]) {
-  if (j < M.mpl) {
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      pg[c] = prog_word(ly.prog, M.s_mlp_gate + 4 * j + c, lane);
-      pu[c] = prog_word(ly.prog, M.s_mlp_up + 4 * j + c, lane);
-    }
-  }
-}
-
 // MLP quaternion groups j0, j0 + 2, ... of the feed-forward gate (session.rs:4005-4025): group j0
-// into `mo`, the later ones into S.mlp_out; pg/pu hold group j0's gather words. Returns the bit
+// into `mo`, the later ones into S.mlp_out; pw holds group j0's gather words. Returns the bit
 // length of the groups' largest magnitude.
 __device__ __forceinline__ uint64_t pair_mlp(const DevModel &M, const Lds &S, const DevLayer &ly,
-                                             uint32_t lane, uint32_t j0, uint32_t (&pg)[4],
-                                             uint32_t (&pu)[4], int64_t (&mo)[4]) {
+                                             uint32_t lane, uint32_t j0, uint4 pw,
+                                             int64_t (&mo)[4]) {
   uint64_t mmx = 0;
 #pragma unroll
   for (int c = 0; c < 4; c++) mo[c] = 0;
@@ -1506,10 +1492,10 @@ __device__ __forceinline__ uint64_t pair_mlp(const DevModel &M, const Lds &S, co
     int32_t gq[4], up[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      gq[c] = S.xbar[pg[c]];
-      up[c] = S.xbar[pu[c]];
+      gq[c] = gather(S.xbar, c < 2 ? pw.x : pw.y, c & 1);
+      up[c] = gather(S.xbar, c < 2 ? pw.z : pw.w, c & 1);
     }
-    pair_mlp_words(M, ly, lane, j + 2, pg, pu);  // the next group's (none past the last)
+    if (j + 2 < M.mpl) pw = gather8(ly, M.p_mlp, j + 2, lane);
     if (mq < M.nm) {
       int64_t o[4];
       mlp_gate(M, S.seeds, gq, up, o);
@@ -1612,7 +1598,9 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     uint2 gd_rec[Q], gd_mlp[Q];
     int4 rbias[Q];
     int32_t dbias[Q], doff[Q];
-    uint32_t pw_rot[Q][4], pw_dec[Q], pw_out[Q][4], pw_down[Q][4];
+    uint4 pw_rot[Q];
+    uint2 pw_down[Q];
+    uint32_t pw_dec[Q];
     // The feed-forward block's gains and gather words: loaded here for one quaternion a lane,
     // where registers allow their latency to hide behind the recurrence block, and at the
     // feed-forward block for more (their registers would spill to scratch across the block).
@@ -1622,8 +1610,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
         const uint32_t ch = 4 * (qv[k] ? qi[k] : 0);
         g_mlp[k] = gat<short4>(ly.mlp_gain, 2 * ch);
         gd_mlp[k] = gat<uint2>(ly.mlp_gain_desc, 2 * ch);
-#pragma unroll
-        for (int c = 0; c < 4; c++) pw_down[k][c] = prog_word(ly.prog, M.s_mlp_down + 4 * k + c, lane);
+        pw_down[k] = gather4(ly, M.p_down, k, lane);
       }
     };
 #pragma unroll
@@ -1634,12 +1621,8 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
       rbias[k] = gat<int4>(ly.gate_bias, 4 * (nq + ch));
       dbias[k] = gat<int32_t>(ly.gate_bias, 4 * qq);
       doff[k] = gat<int32_t>(ly.decay_offset, 4 * qq);
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        pw_rot[k][c] = prog_word(ly.prog, M.s_rec_gate + Q + 4 * k + c, lane);
-        pw_out[k][c] = prog_word(ly.prog, M.s_rec_out + 4 * k + c, lane);
-      }
-      pw_dec[k] = prog_word(ly.prog, M.s_rec_gate + k, lane);
+      pw_rot[k] = gather8(ly, M.p_rot, k, lane);
+      pw_dec[k] = gather1(ly, M.p_dec, k, lane);
     }
     if constexpr (Q == 1) load_ffn();
     clk.lap(kPartLoads);
@@ -1664,8 +1647,9 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     for (int k = 0; k < Q; k++) {
       const int32_t rb[4] = {rbias[k].x, rbias[k].y, rbias[k].z, rbias[k].w};
 #pragma unroll
-      for (int c = 0; c < 4; c++) rot[k][c] = sat_add32(S.xbar[pw_rot[k][c]], rb[c]);
-      dec[k] = sat_add32(S.xbar[pw_dec[k]], dbias[k]);
+      for (int c = 0; c < 4; c++)
+        rot[k][c] = sat_add32(gather(S.xbar, c < 2 ? pw_rot[k].x : pw_rot[k].y, c & 1), rb[c]);
+      dec[k] = sat_add32(gather(S.xbar, pw_dec[k], 0), dbias[k]);
     }
     // Lane weights (session.rs:4989-5026), the transition's rotation (session.rs:5097-5145)
     // and its product with the state, which do not wait for the window.
@@ -1812,18 +1796,17 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     for (int k = 0; k < Q; k++)
       if (qv[k])
 #pragma unroll
-        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], S.xbar[pw_out[k][c]]);
+        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], gather(S.xbar, c < 2 ? pw_rot[k].z : pw_rot[k].w, c & 1));
     wave_sync();
     clk.lap(kPartResidualRec);
     // ---- feed-forward block: wave 0 takes the even quaternion groups. Its first gather words land
     // during the norm.
     if constexpr (Q != 1) load_ffn();
-    uint32_t pg[4], pu[4];
-    pair_mlp_words(M, ly, lane, 0, pg, pu);
+    const uint4 pw_mlp = gather8(ly, M.p_mlp, 0, lane);
     norm_publish<Q>(M, S.seeds, x, qv, qi, g_mlp, gd_mlp, S.xbar);
     clk.sync(kPartNormMlp, kPartSync3);  // 3: the normed activations
     int64_t mo[4];
-    const uint64_t mbl = pair_mlp(M, S, ly, lane, 0, pg, pu, mo);
+    const uint64_t mbl = pair_mlp(M, S, ly, lane, 0, pw_mlp, mo);
     if (lane == 0) S.pair[0] = mbl;
     clk.sync(kPartMlp, kPartSync4);  // 4: both waves' MLP outputs and maxima
     pair_requant(M, S, lane, 0, mo);
@@ -1832,7 +1815,7 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
     for (int k = 0; k < Q; k++)
       if (qv[k])
 #pragma unroll
-        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], S.xbar[pw_down[k][c]]);
+        for (int c = 0; c < 4; c++) x[k][c] = sat_add32(x[k][c], gather(S.xbar, c < 2 ? pw_down[k].x : pw_down[k].y, c & 1));
     wave_sync();
     clk.lap(kPartResidualMlp);
     if constexpr (HM) {  // the stream read after l + 1 layers (session.rs:4252-4276)
@@ -1995,18 +1978,14 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     int64_t *hist_l = hist + (uint64_t)l * d;
     int4 cbias[Q];
-    uint32_t pw_drive[Q][4], pw_gate[Q][4];
+    uint4 pw_rec[Q];
     int64_t sum[Q][4];   // taps 1..W over the earlier positions
     int64_t part[Q][4];  // the next step's taps 2..split
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const uint32_t ch = 4 * (qv[k] ? qi[k] : 0);
       cbias[k] = gat<int4>(ly.conv_bias, 4 * ch);
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        pw_drive[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * k + c, lane);
-        pw_gate[k][c] = prog_word(ly.prog, M.s_rec_in + 4 * Q + 4 * k + c, lane);
-      }
+      pw_rec[k] = gather8(ly, M.p_rec, k, lane);
       if (fresh) {
 #pragma unroll
         for (int c = 0; c < 4; c++) sum[k][c] = 0;
@@ -2026,8 +2005,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       if (qv[k]) window_sum<8>(M, ly, l, ring_l, next, 2, 4 * qi[k], part[k], split);
     }
     // The first MLP group's gather words, for after barrier 3.
-    uint32_t pg[4], pu[4];
-    pair_mlp_words(M, ly, lane, 1, pg, pu);
+    const uint4 pw_mlp = M.mpl > 1 ? gather8(ly, M.p_mlp, 1, lane) : make_uint4(0, 0, 0, 0);
     clk.sync(kPartLoads, kPartSync1);  // 1: the normed activations
     int4 drive[Q];
 #pragma unroll
@@ -2036,9 +2014,9 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
       const uint32_t ch = 4 * qi[k];
       int32_t gv[4];
 #pragma unroll
-      for (int c = 0; c < 4; c++) gv[c] = S.xbar[pw_gate[k][c]];
-      drive[k] = make_int4(S.xbar[pw_drive[k][0]], S.xbar[pw_drive[k][1]], S.xbar[pw_drive[k][2]],
-                           S.xbar[pw_drive[k][3]]);
+      for (int c = 0; c < 4; c++) gv[c] = gather(S.xbar, c < 2 ? pw_rec[k].z : pw_rec[k].w, c & 1);
+      drive[k] = make_int4(gather(S.xbar, pw_rec[k].x, 0), gather(S.xbar, pw_rec[k].x, 1),
+                           gather(S.xbar, pw_rec[k].y, 0), gather(S.xbar, pw_rec[k].y, 1));
       // Tap 0 on the drive and the conv bias, then the drive enters ring slot base.
       int64_t wide[4] = {cbias[k].x, cbias[k].y, cbias[k].z, cbias[k].w};
       tap4(M, ly, l, 0, ch, drive[k], wide);
@@ -2080,7 +2058,7 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
     clk.sync(kPartTransport, kPartSync3);  // 3: the normed activations
     if (defer) __builtin_amdgcn_s_setprio(3);  // the MLP groups, on both waves' path
     int64_t mo[4];
-    const uint64_t mbl = pair_mlp(M, S, ly, lane, 1, pg, pu, mo);
+    const uint64_t mbl = pair_mlp(M, S, ly, lane, 1, pw_mlp, mo);
     if (lane == 0) S.pair[1] = mbl;
     clk.sync(kPartMlp, kPartSync4);  // 4: both waves' MLP outputs and maxima
     pair_requant(M, S, lane, 1, mo);
