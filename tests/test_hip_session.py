@@ -409,3 +409,24 @@ def test_a_slot_rewritten_in_place_sums_its_window_afresh(art):
     end = [a.download() for a in (st, hi, po)]
     for r in end:                                     # the whole session, not only its tokens
         np.testing.assert_array_equal(r[A], r[B])
+
+
+@pytest.mark.parametrize("n", [1, 9])
+def test_in_place_and_staged_launches_agree(art, n, monkeypatch):
+    # The launch's inputs and outputs in the pool's pinned buffer and in a device block: same
+    # outputs, of served and of refused sequences (a token outside the vocabulary).
+    from uor_fbs import session as session_module
+    model = hip.Model(art)
+    tokens = synth.uniform_prompts(SPEC.vocab, n, 5, 91).copy()
+    tokens[-1, 3] = SPEC.vocab
+    slots = np.arange(n, dtype=np.uint32)[::-1]
+    outs = []
+    for limit in (session_module.IN_PLACE_BYTES, 0):
+        monkeypatch.setattr(session_module, "IN_PLACE_BYTES", limit)
+        pool = SessionPool(model, capacity=12)
+        first = pool.run(slots, tokens, gen=2, native=True)
+        pool.run(slots, tokens[:, :2], gen=1)  # the buffer is used again: the first outputs stand
+        outs.append(first)
+    assert outs[0].keys() == outs[1].keys() and outs[0]["status"][-1] != 0
+    for name in outs[0]:
+        np.testing.assert_array_equal(outs[0][name], outs[1][name], err_msg=name)

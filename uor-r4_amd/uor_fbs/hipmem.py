@@ -1,6 +1,7 @@
 """Device arrays for the host side: hipMalloc'd buffers through the HIP runtime the library
 itself links (libamdhip64.so.7), so that buffers, copies and launches share one runtime in the
-process. Plain memory only: allocate, fill with zeros, copy in and out, free."""
+process. Plain memory only: allocate, fill with zeros, copy in and out, free; and pinned host
+memory that kernels reach in place."""
 
 from __future__ import annotations
 
@@ -23,6 +24,10 @@ def runtime():
         rt.hipFree.argtypes = [C.c_void_p]
         rt.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
         rt.hipMemset.argtypes = [C.c_void_p, C.c_int, C.c_size_t]
+        rt.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+        rt.hipHostFree.argtypes = [C.c_void_p]
+        rt.hipHostGetDevicePointer.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_uint]
+        rt.hipStreamSynchronize.argtypes = [C.c_void_p]
         rt.hipSetDevice.argtypes = [C.c_int]
         rt.hipGetDevice.argtypes = [C.POINTER(C.c_int)]
         _rt = rt
@@ -101,10 +106,72 @@ class DeviceArray:
             _check(runtime().hipMemcpy(out.ctypes.data_as(C.c_void_p), src, out.nbytes, _D2H), "hipMemcpy")
         return out
 
+    def upload_at(self, offset: int, a):
+        """Copy host bytes in at a byte offset (checked against the allocation)."""
+        a = np.ascontiguousarray(a, np.uint8)
+        if offset < 0 or offset + a.nbytes > self.nbytes:
+            raise IndexError(f"bytes {offset}..{offset + a.nbytes} outside the array's {self.nbytes}")
+        with _OnDevice(self.device):
+            _check(runtime().hipMemcpy(C.c_void_p(self._p.value + offset), a.ctypes.data_as(C.c_void_p),
+                                       a.nbytes, _H2D), "hipMemcpy")
+
+    def download_from(self, offset: int) -> np.ndarray:
+        """The bytes from an offset to the end; waits for the device."""
+        if not 0 <= offset <= self.nbytes:
+            raise IndexError(f"byte {offset} outside the array's {self.nbytes}")
+        out = np.empty(self.nbytes - offset, np.uint8)
+        with _OnDevice(self.device):
+            _check(runtime().hipMemcpy(out.ctypes.data_as(C.c_void_p), C.c_void_p(self._p.value + offset),
+                                       out.nbytes, _D2H), "hipMemcpy")
+        return out
+
     def free(self):
         if self._p.value:
             with _OnDevice(self.device):
                 runtime().hipFree(self._p)
+            self._p = C.c_void_p()
+
+    def __del__(self):
+        try:
+            self.free()
+        except Exception:
+            pass
+
+
+class HostBuffer:
+    """`nbytes` of pinned host memory that kernels on HIP device `device` read and write in place
+    (small inputs and outputs of a launch: no copy command of their own)."""
+
+    def __init__(self, nbytes: int, device: int = 0):
+        self.device = device
+        self.nbytes = nbytes
+        self._p, dp = C.c_void_p(), C.c_void_p()
+        with _OnDevice(device):
+            _check(runtime().hipHostMalloc(C.byref(self._p), nbytes, 0), "hipHostMalloc")
+            _check(runtime().hipHostGetDevicePointer(C.byref(dp), self._p, 0), "hipHostGetDevicePointer")
+        self._dev = dp.value
+        self._bytes = np.frombuffer((C.c_uint8 * nbytes).from_address(self._p.value), np.uint8)
+
+    def view(self, offset: int, shape, dtype) -> np.ndarray:
+        """The array at a byte offset (checked against the allocation)."""
+        n = int(np.prod(shape)) * np.dtype(dtype).itemsize
+        if offset < 0 or offset + n > self.nbytes:
+            raise IndexError(f"bytes {offset}..{offset + n} outside the buffer's {self.nbytes}")
+        return self._bytes[offset:offset + n].view(dtype).reshape(shape)
+
+    def ptr(self, offset: int) -> C.c_void_p:
+        return C.c_void_p(self._dev + offset)
+
+    def wait(self):
+        """Waits for the device's null stream, after which its kernels' writes are visible here."""
+        with _OnDevice(self.device):
+            _check(runtime().hipStreamSynchronize(None), "hipStreamSynchronize")
+
+    def free(self):
+        if self._p.value:
+            self._bytes = None
+            with _OnDevice(self.device):
+                runtime().hipHostFree(self._p)
             self._p = C.c_void_p()
 
     def __del__(self):

@@ -22,19 +22,23 @@ than continuing differently): read-layer caches (the FBS trunk has none).
 
 from __future__ import annotations
 
+import ctypes as C
 import hashlib
 import os
+import threading
 from dataclasses import dataclass
 
 import numpy as np
 
 from . import hip
-from .hipmem import DeviceArray
+from .hipmem import DeviceArray, HostBuffer
 from .session_codec import (STACK_SESSION_SCHEMA, CodecError, RecurrenceLayer, SerializedStackSession,
                             from_json, to_json)
 
 NO_CHOICE = 0xFFFFFFFF  # session.rs:4406: a nearest-head read step chose no token
 TRACE_UNSET = 0xFFFFFFFF  # a snap trace entry no step has written (session.rs:2580-2584)
+# Launches whose inputs and outputs fit this many bytes pass them in the pool's own pinned buffer.
+IN_PLACE_BYTES = 1 << 20
 TRACE_ZERO = 255  # the launch's trace byte for a zero raw quaternion, whose selection is root 0
 
 
@@ -261,6 +265,9 @@ class SessionPool:
             if a is not None:
                 a.zero()
         self._free = list(range(capacity - 1, -1, -1))
+        # The launches' inputs and outputs where they are small (one launch at a time uses it).
+        self._host: HostBuffer | None = None
+        self._lock = threading.Lock()
 
     def acquire(self, slot: int | None = None) -> int:
         """A free slot holding a fresh session: the next free one, or `slot` if it is free."""
@@ -341,7 +348,7 @@ class SessionPool:
         """One launch: the sessions in `slots` take tokens [n, len] and `gen` greedy steps.
         Returns dict(reply [n, gen+1], status [n], kept [n, P], query [n, d], trace [n, len + gen,
         trace stride]) (kept and query when `native`, trace when `trace`)."""
-        slots = np.asarray(slots, dtype=np.uint32).reshape(-1)
+        slots = np.ascontiguousarray(slots, dtype=np.uint32).reshape(-1)
         tokens = np.ascontiguousarray(tokens, dtype=np.uint32)
         n = len(slots)
         if tokens.ndim != 2 or tokens.shape[0] != n or tokens.shape[1] == 0:
@@ -351,36 +358,67 @@ class SessionPool:
         if np.any(slots >= self.capacity):
             raise ValueError("a slot outside the pool")
         dev = self.model.device
-        d_slots, d_tok = DeviceArray(n, np.uint32, dev), DeviceArray(tokens.size, np.uint32, dev)
-        d_slots.upload(slots)
-        d_tok.upload(tokens.reshape(-1))
-        reply = DeviceArray((n, gen + 1), np.uint32, dev)
-        status = DeviceArray(n, np.int32, dev)
-        kept = DeviceArray((n, self.model.probes), np.uint32, dev) if native else None
-        query = DeviceArray((n, self.model.width), np.int32, dev) if native else None
         steps = tokens.shape[1] + gen
-        stride = int(hip.lib().uor_fbs_trace_stride(self.model.handle))
-        snap = DeviceArray((n, steps, stride), np.uint8, dev) if trace else None
-        ptr = lambda x: None if x is None else x.ptr  # noqa: E731
-        # The null stream: the runtime's blocking copies below wait for the launch.
-        if self.stream is not None:
-            if trace:
-                raise SessionError("Shape", "the snap trace is not served with Hamming reads")
-            hip._check(hip.lib().uor_fbs_serve_slots_stream_async(
-                self.model.handle, d_slots.ptr, n, self.capacity, d_tok.ptr, tokens.shape[1], gen,
-                reply.ptr, self.state.ptr, self.history.ptr, self.position.ptr, self.stream.ptr,
-                ptr(self.payloads), self.cache.ptr, ptr(kept), ptr(query), status.ptr, None))
-        else:
-            hip._check(hip.lib().uor_fbs_serve_slots_async(
-                self.model.handle, d_slots.ptr, n, self.capacity, d_tok.ptr, tokens.shape[1], gen,
-                reply.ptr, self.state.ptr, self.history.ptr, self.position.ptr, self.cache.ptr,
-                self.slide.ptr, ptr(kept), ptr(query), ptr(snap), status.ptr, None))
-        out = dict(reply=reply.download(), status=status.download())
+        # What the launch reads and writes beside the slots, laid out in one buffer: (name, shape,
+        # dtype) at 16-byte offsets.
+        parts = [("slots", (n,), np.uint32), ("tokens", tokens.shape, np.uint32),
+                 ("reply", (n, gen + 1), np.uint32), ("status", (n,), np.int32)]
         if native:
-            out["kept"] = kept.download()
-            out["query"] = query.download()
+            parts += [("kept", (n, self.model.probes), np.uint32), ("query", (n, self.model.width), np.int32)]
         if trace:
-            out["trace"] = snap.download()
+            if self.stream is not None:
+                raise SessionError("Shape", "the snap trace is not served with Hamming reads")
+            stride = int(hip.lib().uor_fbs_trace_stride(self.model.handle))
+            parts.append(("trace", (n, steps, stride), np.uint8))
+        at, total = {}, 0
+        for name, shape, dtype in parts:
+            at[name] = total
+            total += (int(np.prod(shape)) * np.dtype(dtype).itemsize + 15) // 16 * 16
+        ptr = lambda x: None if x is None else x.ptr  # noqa: E731
+
+        def launch(where):
+            opt = lambda name: where(at[name]) if name in at else None  # noqa: E731
+            # The null stream: the wait (or the runtime's blocking copies) below waits for it.
+            if self.stream is not None:
+                hip._check(hip.lib().uor_fbs_serve_slots_stream_async(
+                    self.model.handle, where(at["slots"]), n, self.capacity, where(at["tokens"]),
+                    tokens.shape[1], gen, where(at["reply"]), self.state.ptr, self.history.ptr,
+                    self.position.ptr, self.stream.ptr, ptr(self.payloads), self.cache.ptr, opt("kept"),
+                    opt("query"), where(at["status"]), None))
+            else:
+                hip._check(hip.lib().uor_fbs_serve_slots_async(
+                    self.model.handle, where(at["slots"]), n, self.capacity, where(at["tokens"]),
+                    tokens.shape[1], gen, where(at["reply"]), self.state.ptr, self.history.ptr,
+                    self.position.ptr, self.cache.ptr, self.slide.ptr, opt("kept"), opt("query"),
+                    opt("trace"), where(at["status"]), None))
+
+        outs = parts[2:]
+        if total <= IN_PLACE_BYTES:
+            # A step of a few sessions takes some 50 us; allocating, copying and freeing a buffer for
+            # each of its arguments took five times that (8 sessions of width 128: 311 us a call, 129 in place).
+            with self._lock:
+                if self._host is None:
+                    self._host = HostBuffer(IN_PLACE_BYTES, dev)
+                buf = self._host
+                buf.view(at["slots"], (n,), np.uint32)[:] = slots
+                buf.view(at["tokens"], tokens.shape, np.uint32)[:] = tokens
+                for name, shape, dtype in outs:  # what a refused sequence does not write is zero
+                    buf.view(at[name], shape, dtype)[:] = 0
+                launch(buf.ptr)
+                buf.wait()
+                return {name: buf.view(at[name], shape, dtype).copy() for name, shape, dtype in outs}
+        block = DeviceArray(total, np.uint8, dev)
+        base = block.ptr.value
+        host = np.zeros(at["reply"], np.uint8)
+        host[:4 * n] = slots.view(np.uint8)
+        host[at["tokens"]:at["tokens"] + tokens.nbytes] = tokens.reshape(-1).view(np.uint8)
+        block.upload_at(0, host)
+        launch(lambda offset: C.c_void_p(base + offset))
+        raw = block.download_from(at["reply"])
+        out = {}
+        for name, shape, dtype in outs:
+            o = at[name] - at["reply"]
+            out[name] = raw[o:o + int(np.prod(shape)) * np.dtype(dtype).itemsize].view(dtype).reshape(shape)
         return out
 
 
