@@ -130,15 +130,16 @@ FBS_HD uint16_t gain_desc(int16_t code) {
 }
 
 // A window tap as one word M = +-(16 + m) 2^(28 - sh), for 2 <= sh <= 28 (and 0 for the zero code and
-// for sh >= 38, where every term of a 32-bit v is 0): v M + 2^27 - [M < 0] holds v's gained value
-// before its floor by 2^28, because grid_apply(v, code) = floor((v (+-(16 + m)) + 2^(sh-1) - [code <
-// 0]) / 2^sh) and the products are multiples of 2^(28 - sh). |v M| <= 2^62. kTapWordNone: no word.
+// for 38 <= sh <= 62, where every term of a 32-bit v is 0; a shift past 63 leaves the sign, so those
+// codes have no word): v M + 2^27 - [M < 0] holds v's gained value before its floor by 2^28, because
+// grid_apply(v, code) = floor((v (+-(16 + m)) + 2^(sh-1) - [code < 0]) / 2^sh) and the products are
+// multiples of 2^(28 - sh). |v M| <= 2^62. kTapWordNone: no word.
 constexpr int32_t kTapWordNone = INT32_MIN;
 FBS_HD int32_t tap_word(int16_t code) {
   if (code == 0) return 0;
   const uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
   const int32_t sh = 4 - ((int32_t)(c >> 4) - kGridExpBias);
-  if (sh >= 38) return 0;
+  if (sh >= 38 && sh <= 62) return 0;
   if (sh < 2 || sh > 28) return kTapWordNone;
   const int32_t mag = (int32_t)(16 + (c & 15)) << (28 - sh);
   return code < 0 ? -mag : mag;
