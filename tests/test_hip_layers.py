@@ -1,0 +1,190 @@
+"""Teacher-forced tokens layer by layer (fbs_layers.hip) against the step kernels (a model created with
+one wavefront a sequence, which takes no layer by layer launch) and the oracle: prompts and scored rows at
+the edges of the stretches, widths and windows, fresh and resumed sessions, refused tokens and full
+contexts. Every output is an integer and equal."""
+
+from dataclasses import replace
+
+import numpy as np
+import pytest
+
+import oracle
+from uor_fbs import hip, synth
+from uor_fbs.hipmem import DeviceArray, runtime
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    # One quaternion a lane: half the lanes, a ragged width (24 quaternions; its norm is no power of
+    # two's), the full wavefront with a window of 16.
+    "w128": replace(synth.CONFIGS["c2"], context=96, layers=3),
+    "w96": synth.Spec(vocab=2048, width=96, mlp=160, layers=2, context=96, kept=4, window=5, drawers=40, probes=4),
+    "w256": replace(synth.CONFIGS["c3"], context=96, layers=3),
+    # Two and four a lane, int8 codes, windows whose tap words take two positions a round and one.
+    "w512i8": replace(synth.CONFIGS["c5"], context=224, layers=2),
+    "w320": synth.Spec(vocab=2048, width=320, mlp=512, layers=2, context=96, kept=4, window=40, drawers=33, probes=3),
+    "w768": synth.Spec(vocab=2048, width=768, mlp=1024, layers=2, context=96, kept=4, window=24, drawers=64, probes=4),
+    # The shortest window over the reference's cells, and the whole-table head.
+    "w64": synth.Spec(vocab=4096, width=64, mlp=96, layers=2, context=96, kept=8, window=1),
+}
+
+
+@pytest.fixture(scope="module")
+def models():
+    made = {}
+
+    def get(name, monkeypatch):
+        if name not in made:
+            art = synth.make_artifact(SHAPES[name], 31)
+            monkeypatch.setenv("UOR_FBS_BLOCK_WAVES", "1")
+            steps = hip.Model(art)
+            monkeypatch.delenv("UOR_FBS_BLOCK_WAVES")
+            made[name] = art, hip.Model(art), steps
+        return made[name]
+
+    return get
+
+
+def _up(a, t):
+    d = DeviceArray(np.shape(a), t)
+    d.upload(np.ascontiguousarray(a, t))
+    return d
+
+
+def decode(model, prompts, gen, resume=None):
+    n, length = prompts.shape
+    tok = _up(prompts, np.uint32)
+    ins = [None] * 3 if resume is None else [_up(a, t) for a, t in zip(resume, (np.int64, np.int32, np.uint32))]
+    out = [DeviceArray((n, gen + 1), np.uint32), DeviceArray((n, model.state_words), np.int64),
+           DeviceArray((n, model.history_words), np.int32), DeviceArray(n, np.uint32), DeviceArray(n, np.int32)]
+    p = lambda d: None if d is None else d.ptr  # noqa: E731
+    hip._check(hip.lib().uor_fbs_decode_async(model.handle, tok.ptr, n, length, gen, out[0].ptr, *map(p, ins),
+                                              *[o.ptr for o in out[1:]], None))
+    assert runtime().hipDeviceSynchronize() == 0
+    return [o.download() for o in out]
+
+
+def rows(model, tokens):
+    """The rows' choices, kept drawers, queries and statuses, and their next-token matches, without and
+    with the choices written out."""
+    n, length = tokens.shape
+    tok = _up(tokens, np.uint32)
+    out = [DeviceArray((n, length), np.uint32), DeviceArray((n, length, model.probes), np.uint32),
+           DeviceArray((n, length, model.width), np.int32), DeviceArray(n, np.int32)]
+    hip._check(hip.lib().uor_fbs_sequences_async(model.handle, tok.ptr, n, length, *[o.ptr for o in out], None))
+    assert runtime().hipDeviceSynchronize() == 0
+    got = [o.download() for o in out]
+    for argmin in (False, True):
+        matches, status = DeviceArray(1, np.uint64), DeviceArray(n, np.int32)
+        best = DeviceArray((n, length), np.uint32) if argmin else None
+        hip._check(hip.lib().uor_fbs_score_async(model.handle, tok.ptr, n, length,
+                                                 best.ptr if argmin else None, matches.ptr, status.ptr, None))
+        assert runtime().hipDeviceSynchronize() == 0
+        got += [matches.download(), status.download()] + ([best.download()] if argmin else [])
+    return got
+
+
+def tokens_for(name, n, length, seed):
+    spec = SHAPES[name]
+    make = synth.zipf_prompts if spec.zipf_drawers else synth.uniform_prompts
+    return make(spec.vocab, n, length, seed).copy()
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+@pytest.mark.parametrize("n,length", [(1, 9), (3, 10), (2, 40), (5, 64)])
+def test_prompts_equal_the_step_kernels(models, monkeypatch, name, n, length):
+    art, layers, steps = models(name, monkeypatch)
+    print(f"prompts {name}: {n} of {length}", flush=True)
+    a = tokens_for(name, n, length, 5)
+    first = decode(layers, a, 3)
+    for got, want in zip(first, decode(steps, a, 3)):
+        np.testing.assert_array_equal(got, want)
+    # The sessions resumed by a second prompt, whose choices the oracle makes in one pass.
+    b = tokens_for(name, n, 12, 6)
+    second = decode(layers, b, 0, first[1:4])
+    for got, want in zip(second, decode(steps, b, 0, first[1:4])):
+        np.testing.assert_array_equal(got, want)
+    if name in ("w128", "w96"):
+        fed = np.concatenate([a, first[0][:, :3], b], axis=1)
+        st, want_tok, _, _ = oracle.sequences(art, fed, threads=2)
+        assert st == 0
+        np.testing.assert_array_equal(second[0][:, 0], want_tok[:, -1])
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+@pytest.mark.parametrize("n,length", [(1, 8), (7, 31), (3, 96)])
+def test_rows_equal_the_step_kernels(models, monkeypatch, name, n, length):
+    art, layers, steps = models(name, monkeypatch)
+    print(f"rows {name}: {n} of {length}", flush=True)
+    t = tokens_for(name, n, length, 7)
+    got = rows(layers, t)
+    for g, w in zip(got, rows(steps, t)):
+        np.testing.assert_array_equal(g, w)
+    if name in ("w128", "w96"):
+        st, want_tok, want_kept, want_query = oracle.sequences(art, t, threads=2)
+        assert st == 0
+        for g, w in zip(got, (want_tok, want_kept, want_query)):
+            np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("name", ["w128", "w512i8"])
+def test_refused_sequences(models, monkeypatch, name):
+    # A token outside the vocabulary at the first, a middle and the last position, a context that ends
+    # within the prompt (and under a bad token): the others are served, the refused export nothing.
+    art, layers, steps = models(name, monkeypatch)
+    vocab, context = SHAPES[name].vocab, SHAPES[name].context
+    t = tokens_for(name, 8, 24, 8)
+    for r, at in ((0, 0), (2, 11), (3, 23), (4, 22), (6, 20)):
+        t[r, at] = vocab + r
+    for g, w in zip(rows(layers, t), rows(steps, t)):
+        np.testing.assert_array_equal(g, w)
+    fresh = decode(layers, t, 2)
+    for g, w in zip(fresh, decode(steps, t, 2)):
+        np.testing.assert_array_equal(g, w)
+    assert [int(s) for s in fresh[4]] == [1, 0, 1, 1, 1, 0, 1, 0]
+    warm = decode(steps, tokens_for(name, 8, 10, 9), 0)
+    position = np.array([10, context - 24, context - 24, context, context - 20, context - 12, context - 3, context - 26],
+                        np.uint32)
+    resume = (warm[1], warm[2], position)
+    held = decode(layers, t, 2, resume)
+    for g, w in zip(held, decode(steps, t, 2, resume)):
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("name", ["w128", "w96", "w320", "w512i8"])
+def test_sessions_at_the_ends_of_their_range(models, monkeypatch, name):
+    # States and window rows over all of their types' values: the transport leaves its fast form's ranges
+    # (at the first positions, in some quaternions only) and comes back to them.
+    art, layers, steps = models(name, monkeypatch)
+    n, rng = 6, np.random.default_rng(12)
+    state = rng.integers(-2**63, 2**63 - 1, (n, layers.state_words), dtype=np.int64)
+    state >>= rng.integers(0, 63, state.shape)
+    state[0], state[1, ::7], state[2, 5] = 2**63 - 1, -2**63, 2**62 + 9
+    state[3:5] >>= 40
+    history = rng.integers(-2**31, 2**31 - 1, (n, layers.history_words), dtype=np.int32)
+    history[3] = 2**31 - 1
+    history[4] >>= 12
+    resume = (state, history, np.arange(n, dtype=np.uint32))
+    t = tokens_for(name, n, 43, 13)
+    for g, w in zip(decode(layers, t, 1, resume), decode(steps, t, 1, resume)):
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("n,length", [(2600, 72), (1000, 200)])
+def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
+    # More positions than the workspace holds at once: the sequences run in parts, or in stretches.
+    art, layers, steps = models("w512i8", monkeypatch)
+    t = tokens_for("w512i8", n, length, 10)
+    t[n - 100, 3] = t[n - 5, length - 7] = SHAPES["w512i8"].vocab
+    print(f"rows {n} of {length}", flush=True)
+    got = rows(layers, t)
+    print("prompts", flush=True)
+    fed = decode(layers, t, 1)
+    pick = [0, 700, n - 577, n - 576, n - 101, n - 100, n - 5, n - 1]
+    for i, w in enumerate(rows(steps, t[pick])[:4]):
+        np.testing.assert_array_equal(got[i][pick], w)
+    for g, w in zip(fed, decode(steps, t[pick], 1)):
+        np.testing.assert_array_equal(g[pick], w)
+    # The matches of all rows: the choices against the next tokens of the positions served.
+    served = np.cumsum(t >= SHAPES["w512i8"].vocab, axis=1) == 0
+    assert got[4][0] == ((got[0][:, :-1] == t[:, 1:]) & served[:, :-1]).sum() == got[6][0]

@@ -19,6 +19,7 @@
 
 #include "../../include/uor_fbs.h"
 #include "fbs_device.h"
+#include "fbs_layers.h"
 #include "fbs_int.h"
 
 namespace fbs {
@@ -114,11 +115,54 @@ struct uor_fbs_handle {
   // whatever the sizes.
   bool serve_drawer_major = true;
   uint32_t serve_nchunks = 0, serve_max_chunks = 0;
-  uint32_t jobs_cap = 0, item_cap = 0;
-  uint32_t *job_query = nullptr, *job_flag = nullptr, *drawer_count = nullptr,
-           *drawer_list = nullptr, *item_count = nullptr;
-  uint4 *items = nullptr;
-  unsigned long long *job_best = nullptr;
+  struct Jobs {
+    uint32_t cap = 0, item_cap = 0;
+    uint32_t *query = nullptr, *flag = nullptr, *drawer_count = nullptr, *drawer_list = nullptr,
+             *item_count = nullptr;
+    uint4 *items = nullptr;
+    unsigned long long *best = nullptr;
+
+    void free() {
+      for (void *p : {(void *)query, (void *)flag, (void *)drawer_count, (void *)drawer_list, (void *)best,
+                      (void *)items, (void *)item_count})
+        if (p) (void)hipFree(p);
+      *this = Jobs();
+    }
+    void hand(RunArgs &A) const {
+      A.job_query = query;
+      A.job_flag = flag;
+      A.job_best = best;
+      A.drawer_count = drawer_count;
+      A.drawer_list = drawer_list;
+      A.list_stride = cap;
+      A.items = items;
+      A.item_count = item_count;
+      A.item_cap = item_cap;
+    }
+    ServeScan scan(uint32_t n, uint32_t *out_tokens) const {
+      ServeScan J{};
+      J.items = items;
+      J.item_count = item_count;
+      J.item_cap = item_cap;
+      J.n = n;
+      J.job_query = query;
+      J.job_flag = flag;
+      J.job_best = best;
+      J.drawer_count = drawer_count;
+      J.drawer_list = drawer_list;
+      J.list_stride = cap;
+      J.out_tokens = out_tokens;
+      return J;
+    }
+  };
+  Jobs jobs;
+  // The layer by layer launches (fbs_layers.hip): their workspace (grown, at most kLayerBytes) and,
+  // for scored rows, job buffers of their own, so that a row launch never moves the buffers that a
+  // captured serving launch holds.
+  bool keep_small = true;  // every keep_q31 is below 2^31: the kernels take it as 32 bits
+  unsigned char *layers = nullptr;
+  size_t layers_bytes = 0;
+  Jobs row_jobs;
 
   ~uor_fbs_handle() {
     int prev = 0;
@@ -128,51 +172,69 @@ struct uor_fbs_handle {
     if (ring) (void)hipFree(ring);
     if (hist) (void)hipFree(hist);
     if (pay) (void)hipFree(pay);
-    free_jobs();
+    if (layers) (void)hipFree(layers);
+    jobs.free();
+    row_jobs.free();
     (void)hipSetDevice(prev);
   }
 
-  void free_jobs() {
-    for (void *p : {(void *)job_query, (void *)job_flag, (void *)drawer_count, (void *)drawer_list,
-                    (void *)job_best, (void *)items, (void *)item_count})
-      if (p) (void)hipFree(p);
-    job_query = job_flag = drawer_count = drawer_list = item_count = nullptr;
-    items = nullptr;
-    job_best = nullptr;
-    jobs_cap = item_cap = 0;
+  // Work items of n jobs at most: a chunk's slices are at most its drawer's sessions / 16 + 1, and the
+  // sessions of all drawers together n P.
+  uint64_t job_items(uint32_t n) const {
+    return serve_nchunks +
+           (uint64_t)serve_max_chunks * (((uint64_t)n * M.P + kServeSessions - 1) / kServeSessions);
   }
 
   // The deferred writer's job buffers for n sequences: flags and drawer counts start at zero
   // (a fill kernel on `stream`; the hand-out kernel clears what a launch set).
-  int ensure_jobs(uint32_t n, hipStream_t stream) {
-    if (n <= jobs_cap) return 0;
-    free_jobs();
+  int ensure_jobs(Jobs &b, uint32_t n, hipStream_t stream) {
+    if (n <= b.cap) return 0;
+    b.free();
     const size_t words = M.d / 2;
-    // Items: a chunk's slices are at most its drawer's sessions / 16 + 1, and the sessions of all
-    // drawers together n P.
-    const uint64_t cap = serve_nchunks + (uint64_t)serve_max_chunks *
-                                             (((uint64_t)n * M.P + kServeSessions - 1) / kServeSessions);
+    const uint64_t cap = job_items(n);
     if (cap > 0xffffffffull) return fail(UOR_FBS_ERR_UNSUPPORTED, "too many serving sessions");
-    hipError_t e = hipMalloc((void **)&job_query, (size_t)n * words * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&job_flag, (size_t)n * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&job_best, (size_t)n * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc((void **)&drawer_count, (size_t)M.D * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&drawer_list, (size_t)M.D * n * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&items, (size_t)cap * sizeof(uint4));
-    if (e == hipSuccess) e = hipMalloc((void **)&item_count, sizeof(uint32_t));
+    hipError_t e = hipMalloc((void **)&b.query, (size_t)n * words * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.flag, (size_t)n * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.best, (size_t)n * sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.drawer_count, (size_t)M.D * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.drawer_list, (size_t)M.D * n * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.items, (size_t)cap * sizeof(uint4));
+    if (e == hipSuccess) e = hipMalloc((void **)&b.item_count, sizeof(uint32_t));
     if (e != hipSuccess) {
-      free_jobs();
+      b.free();
       return hip_fail(e, "hipMalloc(serving jobs)");
     }
-    if ((e = launch_fbs_fill_u32(job_flag, n, 0, stream)) != hipSuccess ||
-        (e = launch_fbs_fill_u32(drawer_count, M.D, 0, stream)) != hipSuccess ||
-        (e = launch_fbs_fill_u32(item_count, 1, 0, stream)) != hipSuccess) {
-      free_jobs();
+    if ((e = launch_fbs_fill_u32(b.flag, n, 0, stream)) != hipSuccess ||
+        (e = launch_fbs_fill_u32(b.drawer_count, M.D, 0, stream)) != hipSuccess ||
+        (e = launch_fbs_fill_u32(b.item_count, 1, 0, stream)) != hipSuccess) {
+      b.free();
       return hip_fail(e, "kernel launch");
     }
-    jobs_cap = n;
-    item_cap = (uint32_t)cap;
+    b.cap = n;
+    b.item_cap = (uint32_t)cap;
     return 0;
+  }
+
+  // The layer by layer launches' workspace; false where the device has no room for it (the launch then
+  // takes the step kernels, which need none).
+  bool ensure_layers(size_t bytes) {
+    if (bytes <= layers_bytes) return true;
+    if (layers) (void)hipFree(layers);
+    layers = nullptr;
+    layers_bytes = 0;
+    if (hipMalloc((void **)&layers, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      layers = nullptr;
+      return false;
+    }
+    layers_bytes = bytes;
+    return true;
+  }
+
+  // The scan's wavefronts take the items in turn: two a SIMD, or one an item.
+  uint32_t scan_blocks(uint32_t item_cap) const {
+    const uint32_t blocks = item_cap < 8 * cus ? item_cap : 8 * cus;
+    return blocks ? blocks : 1;
   }
 
   // Payload words (i64) one session keeps: slots x context x d.
@@ -822,6 +884,7 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
   }
   if ((st = h->upload(m->icosian, 120 * 8, &M.icosian))) return done(st);
   if ((st = h->upload(m->keep_q31, 16, &M.keep_q31))) return done(st);
+  for (uint32_t i = 0; i < 16; i++) h->keep_small = h->keep_small && m->keep_q31[i] < (1ull << 31);
   if ((st = h->upload(eps_int, 9, &M.eps_int))) return done(st);
   M.eps0 = eps_int[0];
 
@@ -865,12 +928,194 @@ extern "C" uint32_t uor_fbs_block_waves(const uor_fbs_handle *h, uint32_t n) {
 
 namespace {
 
+// The layer by layer path (fbs_layers.hip) takes the tokens that are known before any choice: a
+// prompt's but its last, whose step (the choice, the generated steps) the step kernels then run from
+// the sessions left in the workspace, and every position of teacher-forced rows, whose choices the
+// drawer-major scan makes. The step kernels take what is left: short inputs, models with reads or
+// snapped rotations, session slots, traces, the nearest head's rows, and launches under capture (a
+// graph must not hold a workspace that a later launch may grow).
+// Measured at width 256 (6 layers, window 16): 300 prompts of 509 tokens 19.2 ms by the step kernels,
+// whose 509 steps run one after another, 4.8 ms by layers; 8,192 rows of 128 76 against 54 ms.
+constexpr size_t kLayerBytes = (size_t)2 << 30;  // the workspace: under 1 % of the card's memory
+constexpr uint32_t kLayerMin = 8;        // tokens a sequence
+constexpr uint32_t kLayerStretch = 64;   // tokens at once of a sequence that runs in several stretches
+constexpr uint32_t kLayerJobs = 32768;   // positions a scan
+constexpr size_t kLayerLists = 1 << 24;  // drawer-list entries a scan
+
+bool layer_model(const uor_fbs_handle *h, bool rows) {
+  const DevModel &M = h->M;
+  return h->pair && h->keep_small && !M.ham.heads && M.raw_gates && M.raw_transition && M.taps_fast && fbs_layers_fit(M) &&
+         (!rows || (M.head != 1 && M.d % 32 == 0));
+}
+
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return stream && (hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone);
+}
+
+// Positions a scan of scored rows: the job buffers stay within kLayerJobs queries, kLayerLists list
+// entries and as many work items (0: a drawer alone exceeds them).
+uint32_t layer_jobs(const uor_fbs_handle *h) {
+  uint32_t n = kLayerJobs;
+  while (n && ((uint64_t)n * h->M.D > kLayerLists || h->job_items(n) > kLayerLists)) n /= 2;
+  return n;
+}
+
+int launch(uor_fbs_handle *h, RunArgs &A, hipStream_t stream, bool noalloc = false,
+           bool one_wave = false);
+
+// The workspace of n sequences of len tokens from `base`, its parts 256-byte aligned: their positions'
+// arrays, with `sessions` the sessions after them, with `rows` their choices. Returns its bytes.
+size_t carve_layers(const DevModel &M, unsigned char *base, uint32_t n, uint32_t len, bool sessions, bool rows,
+                    LayerArgs &P) {
+  size_t at = 0;
+  auto take = [&](auto *&p, size_t count) {
+    p = (std::remove_reference_t<decltype(p)>)(base + at);
+    at += (count * sizeof(*p) + 255) & ~(size_t)255;
+  };
+  const size_t p = (size_t)n * len, ld = (size_t)M.L * M.d;
+  take(P.x, p * M.d);
+  take(P.drive, p * M.d);
+  take(P.turn, p * M.d);
+  take(P.gate, p * M.d);
+  take(P.rhs, p * M.d);
+  take(P.keep, p * M.nq);
+  take(P.steps, n);
+  if (rows) take(P.chosen, p);
+  if (sessions) {
+    take(P.out_state, n * ld);
+    take(P.out_history, n * ld * M.W);
+    take(P.out_position, n);
+  }
+  return at;
+}
+
+// A launch of the layer by layer path; *taken = false: not a call it serves (the step kernels run it).
+int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool *taken) {
+  const DevModel &M = h->M;
+  *taken = false;
+  const bool rows = A.mode != kModeDecode;
+  const uint32_t len = rows ? A.len : A.len - 1;
+  if (len < kLayerMin || A.slots || A.out_trace || A.out_dtrace || A.out_parts || !layer_model(h, rows) ||
+      capturing(stream))
+    return 0;
+  const uint32_t jobs = rows ? layer_jobs(h) : 0;
+  if (rows && jobs == 0) return 0;
+  // The sequences run together (`part` of them where the workspace does not hold them all: the grids'
+  // second dimension, and for a decode whole turns of the step kernels' resident blocks), over all
+  // their tokens or, where the workspace does not hold those, in stretches of `run` tokens, the
+  // sessions kept between them.
+  LayerArgs P{};
+  uint32_t part = A.n < 65535u ? A.n : 65535u, run = len;
+  const auto bytes = [&](uint32_t n, uint32_t t) { return carve_layers(M, nullptr, n, t, !rows || t < len, rows, P); };
+  if (bytes(part, run) > kLayerBytes) {
+    const uint32_t least = len < kLayerStretch ? len : kLayerStretch;
+    if (bytes(part, least) > kLayerBytes) {
+      uint32_t fit = 0;
+      for (uint32_t bit = 1u << 15; bit; bit >>= 1)
+        if (fit + bit < part && bytes(fit + bit, least) <= kLayerBytes) fit += bit;
+      if (fit == 0) return 0;
+      part = !rows && fit > h->pair_grid ? fit - fit % h->pair_grid : fit;
+    }
+    uint32_t most = least;
+    for (uint32_t bit = 1u << 30; bit; bit >>= 1)
+      if (bit < len - most && bytes(part, most + bit) <= kLayerBytes) most += bit;
+    const uint32_t stretches = (len + most - 1) / most;
+    run = (len + stretches - 1) / stretches;
+  }
+  const bool sessions = !rows || run < len;
+  if (!h->ensure_layers(bytes(part, run))) return 0;
+  *taken = true;
+  int st = 0;
+  if (rows) {
+    const uint64_t all = (uint64_t)part * run;
+    if ((st = h->ensure_jobs(h->row_jobs, all < jobs ? (uint32_t)all : jobs, stream))) return st;
+  }
+  const size_t ld = (size_t)M.L * M.d;
+  for (uint32_t s0 = 0; s0 < A.n; s0 += part) {
+    const uint32_t n = A.n - s0 < part ? A.n - s0 : part;
+    P = LayerArgs{};
+    P.n = n;
+    P.row = A.len;
+    P.tokens = A.tokens + (size_t)s0 * A.len;
+    P.in_state = A.in_state ? A.in_state + s0 * ld : nullptr;
+    P.in_history = A.in_history ? A.in_history + s0 * ld * M.W : nullptr;
+    P.in_position = A.in_position ? A.in_position + s0 : nullptr;
+    P.status = A.status + s0;
+    P.out_tokens = rows && A.out_tokens ? A.out_tokens + (size_t)s0 * A.len : nullptr;
+    P.out_kept = rows && A.out_kept ? A.out_kept + (size_t)s0 * A.len * M.P : nullptr;
+    P.out_query = rows && A.out_query ? A.out_query + (size_t)s0 * A.len * M.d : nullptr;
+    P.matches = A.mode == kModeScore ? A.matches : nullptr;
+    for (uint32_t t0 = 0; t0 < len; t0 += run) {
+      P.start = t0;
+      P.len = len - t0 < run ? len - t0 : run;
+      carve_layers(M, h->layers, n, P.len, false, rows, P);
+      if (sessions) {  // at one place in every stretch, after the longest one's arrays
+        LayerArgs Q{};
+        carve_layers(M, h->layers, n, run, true, rows, Q);
+        P.out_state = Q.out_state;
+        P.out_history = Q.out_history;
+        P.out_position = Q.out_position;
+        if (t0) {
+          P.in_state = P.out_state;
+          P.in_history = P.out_history;
+          P.in_position = P.out_position;
+        }
+      }
+      P.len_recip = (1ull << 32) / P.len;
+      // Eight positions a wavefront, or fewer that the chip's SIMDs get eight wavefronts each.
+      const uint64_t turns = (uint64_t)n * P.len / (32ull * h->cus);
+      P.turns = turns < 1 ? 1 : turns > 8 ? 8 : (uint32_t)turns;
+      hipError_t e = launch_fbs_layers(M, P, rows, stream);
+      if (e != hipSuccess) return hip_fail(e, "kernel launch");
+      if (!rows) continue;
+      const uint32_t all = n * P.len;
+      for (P.first = 0; P.first < all; P.first += jobs) {
+        RunArgs B{};
+        B.n = all - P.first < jobs ? all - P.first : jobs;
+        h->row_jobs.hand(B);
+        e = launch_fbs_layer_query(M, P, B, stream);
+        if (e == hipSuccess)
+          e = launch_fbs_serve_scan(M, h->row_jobs.scan(B.n, P.chosen + P.first),
+                                    h->scan_blocks(h->row_jobs.item_cap), stream);
+        if (e != hipSuccess) return hip_fail(e, "kernel launch");
+      }
+      e = launch_fbs_layer_choices(P, stream);
+      if (e != hipSuccess) return hip_fail(e, "kernel launch");
+    }
+    if (rows) continue;
+    RunArgs B = A;  // the prompts' last tokens and the generated steps
+    B.n = n;
+    B.len = 1;
+    B.row = A.len;
+    B.tokens = P.tokens + len;
+    B.out_tokens = A.out_tokens + (size_t)s0 * (A.gen + 1);
+    B.in_state = P.out_state;
+    B.in_history = P.out_history;
+    B.in_position = P.out_position;
+    B.out_kept = A.out_kept ? A.out_kept + (size_t)s0 * M.P : nullptr;
+    B.out_query = A.out_query ? A.out_query + (size_t)s0 * M.d : nullptr;
+    B.out_state = A.out_state ? A.out_state + s0 * ld : nullptr;
+    B.out_history = A.out_history ? A.out_history + s0 * ld * M.W : nullptr;
+    B.out_position = A.out_position ? A.out_position + s0 : nullptr;
+    B.status = P.status;
+    B.in_status = P.status;  // a sequence refused in its prompt stays so
+    if ((st = launch(h, B, stream))) return st;
+  }
+  return 0;
+}
+
 // `noalloc`: the window rings and sums come from the device's scratch array, whose size bounds
 // the grid (sequences loop within the blocks), and nothing is allocated. `one_wave`: the
 // one-wavefront kernels whatever the model's default (the snap trace is recorded there).
-int launch(uor_fbs_handle *h, RunArgs &A, hipStream_t stream, bool noalloc = false,
-           bool one_wave = false) {
+int launch(uor_fbs_handle *h, RunArgs &A, hipStream_t stream, bool noalloc, bool one_wave) {
   if (A.n == 0) return 0;
+  if (!A.row) A.row = A.len;
+  if (!noalloc && !one_wave) {
+    bool taken = false;
+    const int st = launch_layers(h, A, stream, &taken);
+    if (st || taken) return st;
+  }
   const bool clocks = A.out_parts != nullptr;
   if (clocks && (!h->pair || one_wave || noalloc || h->M.ham.heads || A.mode != kModeDecode ||
                  A.gen == 0 || A.slots))
@@ -1374,40 +1619,18 @@ extern "C" int uor_fbs_serve_slots_async(uor_fbs_handle *h, const uint32_t *slot
                         (uint64_t)h->M.D * sequences < (1ull << 32);  // drawer-list indices
   hipStream_t st = (hipStream_t)stream;
   if (deferred) {
-    int e = h->ensure_jobs(sequences, st);
+    int e = h->ensure_jobs(h->jobs, sequences, st);
     if (e) return e;
-    A.job_query = h->job_query;
-    A.job_flag = h->job_flag;
-    A.job_best = h->job_best;
-    A.drawer_count = h->drawer_count;
-    A.drawer_list = h->drawer_list;
-    A.list_stride = h->jobs_cap;
-    A.items = h->items;
-    A.item_count = h->item_count;
-    A.item_cap = h->item_cap;
+    h->jobs.hand(A);
   }
   // The trace is recorded by the one-wavefront kernels.
   int rc = launch(h, A, st, false, out_trace != nullptr);
   if (rc || !deferred) return rc;
-  ServeScan J{};
-  J.items = h->items;
-  J.item_count = h->item_count;
-  J.item_cap = h->item_cap;
-  J.n = sequences;
-  J.gen = gen;
-  J.job_query = h->job_query;
-  J.job_flag = h->job_flag;
-  J.job_best = h->job_best;
-  J.drawer_count = h->drawer_count;
-  J.drawer_list = h->drawer_list;
-  J.list_stride = h->jobs_cap;
-  J.out_tokens = out_reply;
+  ServeScan J = h->jobs.scan(sequences, out_reply);
   J.slots = slots;
   J.cache = (uint8_t *)cache;
   J.cache_stride = A.cache_stride;
-  // The scan's wavefronts take the items in turn: two a SIMD, or one an item.
-  uint32_t blocks = h->item_cap < 8 * h->cus ? h->item_cap : 8 * h->cus;
-  blocks = blocks ? blocks : 1;
+  const uint32_t blocks = h->scan_blocks(h->jobs.item_cap);
   const hipError_t e = launch_fbs_serve_scan(h->M, J, blocks, st);
   return e != hipSuccess ? hip_fail(e, "kernel launch") : 0;
 }

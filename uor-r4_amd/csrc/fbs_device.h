@@ -274,6 +274,9 @@ struct RunArgs {
   uint4 *items;
   uint32_t *item_count;
   uint32_t item_cap;
+  uint32_t row;               // a sequence's tokens in `tokens` (len, or more where the first were
+                              // taken in by the layer kernels)
+  const int32_t *in_status;   // nullable: a sequence whose entry is not 0 is refused with it
 };
 
 // The drawer-major scan of the deferred writer's jobs (fbs_serve.hip). A work item is one

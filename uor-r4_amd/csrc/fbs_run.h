@@ -2077,6 +2077,55 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
   return 0;
 }
 
+// A deferred writer's job for sequence s (RunArgs::job_query): its query, the sequence in each kept
+// drawer's list, its best reset. The wave's query and kept drawers are in LDS.
+template <int Q, bool T8>
+__device__ __forceinline__ void push_job(const DevModel &M, const RunArgs &A, uint32_t s, const int32_t *query,
+                                         const uint32_t *kept, uint32_t lane, const bool (&qv)[Q],
+                                         const uint32_t (&qi)[Q]) {
+  uint32_t *jq = A.job_query + (uint64_t)s * (M.d / 2);
+#pragma unroll
+  for (int k = 0; k < Q; k++)
+    if (qv[k]) {
+      const int4 q = *(const int4 *)(query + 4 * qi[k]);
+      // As scan_setup packs it: biased 16-bit pairs, or for an int8 table the query clamped to the
+      // table's range and scaled to meet its widened codes.
+      uint32_t b[4];
+      const int32_t qa[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        if (T8) {
+          const int32_t lo = -(128 << M.t8_shift), hi = 127 << M.t8_shift;
+          const int32_t x = qa[c] < lo ? lo : qa[c] > hi ? hi : qa[c];
+          b[c] = (uint32_t)(x - lo) << (8 - M.t8_shift);
+        } else {
+          b[c] = (uint32_t)(qa[c] + 32768);
+        }
+      }
+      *(uint2 *)(jq + 2 * qi[k]) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+    }
+  if (lane < M.P) {
+    const uint32_t c = kept[lane];
+    const uint32_t at = atomicAdd(A.drawer_count + c, 1u);
+    if (at < A.list_stride) {
+      A.drawer_list[(uint64_t)c * A.list_stride + at] = s;
+      if (at % kServeSessions == 0) {  // this sequence opens a slice: its items
+        const uint32_t b = M.offsets[c], e = M.offsets[c + 1];
+        const uint32_t nch = (e - b + kServeRows - 1) / kServeRows;
+        const uint32_t i0 = nch ? atomicAdd(A.item_count, nch) : 0u;
+        for (uint32_t k = 0; k < nch && i0 + k < A.item_cap; k++) {
+          const uint32_t m0 = b + kServeRows * k;
+          A.items[i0 + k] = make_uint4(m0, e - m0 < kServeRows ? e - m0 : kServeRows, c * A.list_stride + at, c);
+        }
+      }
+    }
+  }
+  if (lane == 0) {
+    A.job_best[s] = ~0ull;
+    A.job_flag[s] = 1u;
+  }
+}
+
 // The phase a kernel is compiled for. Prefill: decode launches with no generated step (the
 // prompt, its last choice, the state out). Decode: decode launches that generate. Rows: the
 // teacher-forced modes, sequences and score.
@@ -2353,11 +2402,11 @@ __device__ __forceinline__ void run(const DevModel &M, const RunArgs &A) {
       wave_sync();
     clk.start();
     if (NW == 2 && ce) fresh = fresh || S.wmeta[3] != fp_tag;
-    int status = bad_stream ? 1 : 0;
+    int status = bad_stream ? 1 : A.in_status ? A.in_status[s] : 0;
     uint32_t chosen = 0;
     constexpr bool decode = PH != kPhaseRows;
-    const uint32_t *toks = A.tokens + (uint64_t)s * A.len;
-    const uint32_t steps = bad_stream ? 0u : PH == kPhaseDecode ? A.len + A.gen : A.len;
+    const uint32_t *toks = A.tokens + (uint64_t)s * A.row;
+    const uint32_t steps = status ? 0u : PH == kPhaseDecode ? A.len + A.gen : A.len;
     unsigned long long hits = 0;
     uint32_t done = 0;  // steps run
     for (uint32_t t = 0; t < steps; t++) {
@@ -2425,50 +2474,7 @@ __device__ __forceinline__ void run(const DevModel &M, const RunArgs &A) {
           // drawer's list, its best reset (the scan kernel's atomic minimum starts there).
           if (defer && wave == 0 && status == 0) {
             wave_sync();
-            if (S.wmeta[2] == 2) {
-              uint32_t *jq = A.job_query + (uint64_t)s * (d / 2);
-#pragma unroll
-              for (int k = 0; k < Q; k++)
-                if (qv[k]) {
-                  const int4 q = *(const int4 *)(S.xbar + 4 * qi[k]);
-                  // As scan_setup packs it: biased 16-bit pairs, or for an int8 table the query
-                  // clamped to the table's range and scaled to meet its widened codes.
-                  uint32_t b[4];
-                  const int32_t qa[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-                  for (int c = 0; c < 4; c++) {
-                    if (T8) {
-                      const int32_t lo = -(128 << M.t8_shift), hi = 127 << M.t8_shift;
-                      const int32_t x = qa[c] < lo ? lo : qa[c] > hi ? hi : qa[c];
-                      b[c] = (uint32_t)(x - lo) << (8 - M.t8_shift);
-                    } else {
-                      b[c] = (uint32_t)(qa[c] + 32768);
-                    }
-                  }
-                  *(uint2 *)(jq + 2 * qi[k]) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
-                }
-              if (lane < M.P) {
-                const uint32_t c = S.kept[lane];
-                const uint32_t at = atomicAdd(A.drawer_count + c, 1u);
-                if (at < A.list_stride) {
-                  A.drawer_list[(uint64_t)c * A.list_stride + at] = s;
-                  if (at % kServeSessions == 0) {  // this session opens a slice: its items
-                    const uint32_t b = M.offsets[c], e = M.offsets[c + 1];
-                    const uint32_t nch = (e - b + kServeRows - 1) / kServeRows;
-                    const uint32_t i0 = nch ? atomicAdd(A.item_count, nch) : 0u;
-                    for (uint32_t k = 0; k < nch && i0 + k < A.item_cap; k++) {
-                      const uint32_t m0 = b + kServeRows * k;
-                      A.items[i0 + k] = make_uint4(m0, e - m0 < kServeRows ? e - m0 : kServeRows,
-                                                   c * A.list_stride + at, c);
-                    }
-                  }
-                }
-              }
-              if (lane == 0) {
-                A.job_best[s] = ~0ull;
-                A.job_flag[s] = 1u;
-              }
-            }
+            if (S.wmeta[2] == 2) push_job<Q, T8>(M, A, s, S.xbar, S.kept, lane, qv, qi);
           }
         }
       }
