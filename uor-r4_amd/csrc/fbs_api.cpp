@@ -48,9 +48,6 @@ FBS_LAUNCHER(fbs_prefill_pair_ham)
 FBS_LAUNCHER(fbs_decode_pair_ham)
 FBS_LAUNCHER(fbs_rows_pair_ham)
 #undef FBS_LAUNCHER
-// The deferred writer's drawer-major scan and hand-out (fbs_serve.hip).
-hipError_t launch_fbs_serve_scan(const DevModel &M, const ServeScan &J, uint32_t blocks,
-                                 hipStream_t stream);
 hipError_t launch_fbs_fill_u32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t stream);
 }
 
@@ -159,6 +156,7 @@ struct uor_fbs_handle {
   // The layer by layer launches (fbs_layers.hip): their workspace (grown, at most kLayerBytes) and,
   // for scored rows, job buffers of their own, so that a row launch never moves the buffers that a
   // captured serving launch holds.
+  bool taps_high = true;   // every tap word lies within +-2^27
   bool keep_small = true;  // every keep_q31 is below 2^31: the kernels take it as 32 bits
   unsigned char *layers = nullptr;
   size_t layers_bytes = 0;
@@ -755,6 +753,7 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
       for (size_t i = 0; i < nt; i++) {
         tap_words[l * nt + i] = tap_word(taps[i]);
         if (tap_words[l * nt + i] == kTapWordNone) M.taps_fast = 0;
+        h->taps_high = h->taps_high && tap_words[l * nt + i] < (1 << 27) && tap_words[l * nt + i] > -(1 << 27);
       }
       for (uint32_t i = 0; i < d; i++) {
         rg[i] = gain_desc(ly.rec_gain[i]);
@@ -935,9 +934,8 @@ namespace {
 // snapped rotations, session slots, traces, the nearest head's rows, and launches under capture (a
 // graph must not hold a workspace that a later launch may grow).
 // Measured at width 256 (6 layers, window 16): 300 prompts of 509 tokens 19.2 ms by the step kernels,
-// whose 509 steps run one after another, 4.8 ms by layers; 8,192 rows of 128 76 against 54 ms.
+// whose 509 steps run one after another, 3.8 ms by layers; 8,192 rows of 128 76 against 40 ms.
 constexpr size_t kLayerBytes = (size_t)2 << 30;  // the workspace: under 1 % of the card's memory
-constexpr uint32_t kLayerMin = 8;        // tokens a sequence
 constexpr uint32_t kLayerStretch = 64;   // tokens at once of a sequence that runs in several stretches
 constexpr uint32_t kLayerJobs = 32768;   // positions a scan
 constexpr size_t kLayerLists = 1 << 24;  // drawer-list entries a scan
@@ -945,7 +943,19 @@ constexpr size_t kLayerLists = 1 << 24;  // drawer-list entries a scan
 bool layer_model(const uor_fbs_handle *h, bool rows) {
   const DevModel &M = h->M;
   return h->pair && h->keep_small && !M.ham.heads && M.raw_gates && M.raw_transition && M.taps_fast && fbs_layers_fit(M) &&
-         (!rows || (M.head != 1 && M.d % 32 == 0));
+         M.d % 32 == 0 && (!rows || M.head != 1);
+}
+
+// Whether `len` known tokens of n sequences take less time by layers than by steps. In units of a tenth of
+// a step of a full grid (G sequences): a token costs the steps 10 a turn of the grid, and the layers 7
+// for G prompts (4 for rows, whose steps run the writer as well) and less for fewer, whose steps cost no
+// less; against that stand the layers' launches, 40 (30). Microseconds by layers and by steps, widths
+// 128 / 256 / 512: one prompt of 5 tokens 148 and 180 / 193 and 203 / 395 and 473, of 4 148 and 150 / 193
+// and 184 / 395 and 389; 1,024 prompts of 12 379 and 429 / 645 and 621 / 1,649 and 1,681, of 16 438 and 555
+// / 714 and 780 / 1,808 and 2,149; 1,024 rows of 8 296 and 361 / 464 and 679 / 966 and 1,637.
+bool layers_pay(const uor_fbs_handle *h, uint64_t n, uint32_t len, bool rows) {
+  const uint64_t G = h->pair_grid, turns = (n + G - 1) / G, t = len < 64 ? len : 64;
+  return t * (10 * turns * G - (rows ? 4 : 7) * n) >= (rows ? 30 : 40) * G;
 }
 
 bool capturing(hipStream_t stream) {
@@ -981,7 +991,10 @@ size_t carve_layers(const DevModel &M, unsigned char *base, uint32_t n, uint32_t
   take(P.rhs, p * M.d);
   take(P.keep, p * M.nq);
   take(P.steps, n);
-  if (rows) take(P.chosen, p);
+  if (rows) {
+    take(P.chosen, p);
+    take(P.kept, (p < kLayerJobs ? p : (size_t)kLayerJobs) * M.P);
+  }
   if (sessions) {
     take(P.out_state, n * ld);
     take(P.out_history, n * ld * M.W);
@@ -996,8 +1009,8 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
   *taken = false;
   const bool rows = A.mode != kModeDecode;
   const uint32_t len = rows ? A.len : A.len - 1;
-  if (len < kLayerMin || A.slots || A.out_trace || A.out_dtrace || A.out_parts || !layer_model(h, rows) ||
-      capturing(stream))
+  if (A.slots || A.out_trace || A.out_dtrace || A.out_parts || !layer_model(h, rows) ||
+      !layers_pay(h, A.n, len, rows) || capturing(stream))
     return 0;
   const uint32_t jobs = rows ? layer_jobs(h) : 0;
   if (rows && jobs == 0) return 0;
@@ -1025,18 +1038,21 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
   }
   const bool sessions = !rows || run < len;
   if (!h->ensure_layers(bytes(part, run))) return 0;
-  *taken = true;
-  int st = 0;
   if (rows) {
     const uint64_t all = (uint64_t)part * run;
-    if ((st = h->ensure_jobs(h->row_jobs, all < jobs ? (uint32_t)all : jobs, stream))) return st;
+    if (h->ensure_jobs(h->row_jobs, all < jobs ? (uint32_t)all : jobs, stream)) {
+      (void)hipGetLastError();  // no room: the step kernels, which need none
+      return 0;
+    }
   }
+  *taken = true;
   const size_t ld = (size_t)M.L * M.d;
   for (uint32_t s0 = 0; s0 < A.n; s0 += part) {
     const uint32_t n = A.n - s0 < part ? A.n - s0 : part;
     P = LayerArgs{};
     P.n = n;
     P.row = A.len;
+    P.taps_high = h->taps_high;
     P.tokens = A.tokens + (size_t)s0 * A.len;
     P.in_state = A.in_state ? A.in_state + s0 * ld : nullptr;
     P.in_history = A.in_history ? A.in_history + s0 * ld * M.W : nullptr;
@@ -1074,10 +1090,7 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
         RunArgs B{};
         B.n = all - P.first < jobs ? all - P.first : jobs;
         h->row_jobs.hand(B);
-        e = launch_fbs_layer_query(M, P, B, stream);
-        if (e == hipSuccess)
-          e = launch_fbs_serve_scan(M, h->row_jobs.scan(B.n, P.chosen + P.first),
-                                    h->scan_blocks(h->row_jobs.item_cap), stream);
+        e = launch_fbs_layer_query(M, P, B, h->row_jobs.scan(B.n, P.chosen + P.first), h->cus, stream);
         if (e != hipSuccess) return hip_fail(e, "kernel launch");
       }
       e = launch_fbs_layer_choices(P, stream);
@@ -1100,7 +1113,8 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
     B.out_position = A.out_position ? A.out_position + s0 : nullptr;
     B.status = P.status;
     B.in_status = P.status;  // a sequence refused in its prompt stays so
-    if ((st = launch(h, B, stream))) return st;
+    const int st = launch(h, B, stream);
+    if (st) return st;
   }
   return 0;
 }

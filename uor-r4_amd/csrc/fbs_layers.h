@@ -13,6 +13,7 @@ namespace fbs {
 struct LayerArgs {
   uint32_t n, len;
   uint32_t row, start;        // a row's tokens, the stretch's first
+  uint32_t taps_high;         // every tap word lies within +-2^27
   uint32_t turns;             // positions a wavefront of the front kernel takes in turn
   uint64_t len_recip;         // floor(2^32 / len): a position's sequence without a division
   const uint32_t *tokens;     // n * row
@@ -34,6 +35,7 @@ struct LayerArgs {
   // each position's query, kept drawers and choice at its place in the rows, and the rows' next-token
   // matches (all nullable; without out_tokens a row's last choice is not made).
   uint32_t first;
+  uint32_t *kept;             // a scan's positions * probes
   uint32_t *chosen;
   int32_t *out_query;
   uint32_t *out_kept;
@@ -41,12 +43,17 @@ struct LayerArgs {
   unsigned long long *matches;
 };
 
+// fbs_serve.hip
+hipError_t launch_fbs_serve_scan(const DevModel &M, const ServeScan &J, uint32_t blocks, hipStream_t stream);
+hipError_t launch_fbs_serve_finish(const DevModel &M, const ServeScan &J, hipStream_t stream);
+
 // Whether the kernels' LDS serves the model's shapes.
 bool fbs_layers_fit(const DevModel &M);
 // Every layer over the positions; `rows`: also the end of the last one (the query kernel's input).
 hipError_t launch_fbs_layers(const DevModel &M, const LayerArgs &P, bool rows, hipStream_t stream);
-// A.n positions' queries and drawers, their jobs for the drawer-major scan (RunArgs::job_query ...).
-hipError_t launch_fbs_layer_query(const DevModel &M, const LayerArgs &P, const RunArgs &A, hipStream_t stream);
+// A.n positions' queries, drawers and choices (S.out_tokens); `cus`: the device's compute units.
+hipError_t launch_fbs_layer_query(const DevModel &M, const LayerArgs &P, const RunArgs &A, const ServeScan &S,
+                                  uint32_t cus, hipStream_t stream);
 // The stretch's choices to out_tokens, and those equal to their row's next token added to *matches.
 hipError_t launch_fbs_layer_choices(const LayerArgs &P, hipStream_t stream);
 

@@ -148,6 +148,14 @@ __device__ __forceinline__ uint64_t wave_reduce64(uint64_t v, Op op) {
   v = op(v, dpp64<kDppMirror>(v));
   return op(op(lane64(v, 0), lane64(v, 16)), op(lane64(v, 32), lane64(v, 48)));
 }
+// The minimum over each row of 16 lanes, in all of them.
+__device__ __forceinline__ uint64_t row16_min(uint64_t v) {
+  const OpMin op;
+  v = op(v, dpp64<kDppXor1>(v));
+  v = op(v, dpp64<kDppXor2>(v));
+  v = op(v, dpp64<kDppHalfMirror>(v));
+  return op(v, dpp64<kDppMirror>(v));
+}
 // The bit length of the wave's largest magnitude from each lane's magnitudes or-ed together: the bit
 // length of a maximum is the maximum of the bit lengths, and that of the or, so a 32-bit reduction
 // takes the place of a 64-bit one.
@@ -2077,12 +2085,10 @@ __device__ __forceinline__ int step_window(const DevModel &M, const Lds &S, int3
   return 0;
 }
 
-// A deferred writer's job for sequence s (RunArgs::job_query): its query, the sequence in each kept
-// drawer's list, its best reset. The wave's query and kept drawers are in LDS.
+// A deferred writer's query (`query` in LDS) as the drawer-major scan reads it.
 template <int Q, bool T8>
-__device__ __forceinline__ void push_job(const DevModel &M, const RunArgs &A, uint32_t s, const int32_t *query,
-                                         const uint32_t *kept, uint32_t lane, const bool (&qv)[Q],
-                                         const uint32_t (&qi)[Q]) {
+__device__ __forceinline__ void job_words(const DevModel &M, const RunArgs &A, uint32_t s, const int32_t *query,
+                                          const bool (&qv)[Q], const uint32_t (&qi)[Q]) {
   uint32_t *jq = A.job_query + (uint64_t)s * (M.d / 2);
 #pragma unroll
   for (int k = 0; k < Q; k++)
@@ -2104,6 +2110,15 @@ __device__ __forceinline__ void push_job(const DevModel &M, const RunArgs &A, ui
       }
       *(uint2 *)(jq + 2 * qi[k]) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
     }
+}
+
+// A deferred writer's job for sequence s (RunArgs::job_query): its query, the sequence in each kept
+// drawer's list, its best reset. The wave's query and kept drawers are in LDS.
+template <int Q, bool T8>
+__device__ __forceinline__ void push_job(const DevModel &M, const RunArgs &A, uint32_t s, const int32_t *query,
+                                         const uint32_t *kept, uint32_t lane, const bool (&qv)[Q],
+                                         const uint32_t (&qi)[Q]) {
+  job_words<Q, T8>(M, A, s, query, qv, qi);
   if (lane < M.P) {
     const uint32_t c = kept[lane];
     const uint32_t at = atomicAdd(A.drawer_count + c, 1u);

@@ -174,6 +174,15 @@ __global__ __launch_bounds__(256) void fbs_fill_u32(uint32_t *p, uint64_t n, uin
     p[i] = v;
 }
 
+hipError_t launch_fbs_serve_finish(const DevModel &M, const ServeScan &J, hipStream_t stream) {
+  DevModel m = M;
+  ServeScan j = J;
+  void *args[] = {&m, &j};
+  const uint32_t fin = (J.n + 255) / 256;
+  const hipError_t e = hipLaunchKernel((const void *)fbs_serve_finish, dim3(fin ? fin : 1), dim3(256), args, 0, stream);
+  return e != hipSuccess ? e : hipGetLastError();
+}
+
 // The scan over `blocks` wavefronts, then the hand-out.
 hipError_t launch_fbs_serve_scan(const DevModel &M, const ServeScan &J, uint32_t blocks,
                                  hipStream_t stream) {
@@ -191,10 +200,7 @@ hipError_t launch_fbs_serve_scan(const DevModel &M, const ServeScan &J, uint32_t
                                           : (const void *)fbs_serve_scan<16, false>);
   hipError_t e = hipLaunchKernel(f, dim3(blocks), dim3(kWave), args, 0, stream);
   if (e == hipSuccess) e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const uint32_t fin = (J.n + 255) / 256;
-  e = hipLaunchKernel((const void *)fbs_serve_finish, dim3(fin ? fin : 1), dim3(256), args, 0, stream);
-  return e != hipSuccess ? e : hipGetLastError();
+  return e != hipSuccess ? e : launch_fbs_serve_finish(M, J, stream);
 }
 
 hipError_t launch_fbs_fill_u32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t stream) {
