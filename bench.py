@@ -443,9 +443,10 @@ def score_main(a, torch, oracle, art, model, rows, dev, stream, sp) -> dict:
     S = 1
     while S < spec.width // 32:
         S *= 2
-    family = "fbs_rows_pair" if model.block_waves(R) == 2 else "fbs_rows"
-    if spec.table == "i8":  # the int8 table's own kernels (fbs_rows_pair8, fbs_rows_8)
-        family += "8" if family.endswith("pair") else "_8"
+    # Paired models score rows layer by layer, the others by steps.
+    family = "fbs_rows_8" if spec.table == "i8" else "fbs_rows"
+    kernel = ("fbs_layer_front, fbs_layer_chain, fbs_layer_query, fbs_layer_scan" if model.block_waves(R) == 2
+              else f"{family}<{(spec.width // 4 + 63) // 64}, {S}>")
     out = {
         "metric": f"teacher-forced scored positions/sec, {R} rows x {n}, width {spec.width} (1 GPU)",
         "value": round(positions / (ms_per_step / 1e3), 1), "unit": "positions/s", "n_gpus": 1,
@@ -460,9 +461,9 @@ def score_main(a, torch, oracle, art, model, rows, dev, stream, sp) -> dict:
         "matches": int(matches.item()),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic(a, f"{family}<{(spec.width // 4 + 63) // 64}, {S}>"),
+                     "traffic": measured_traffic(a, kernel),
                      "bytes_per_position": round(bpt, 1), "mean_candidate_rows": round(mean_cand, 1),
-                     "kernel": f"{family}<{(spec.width // 4 + 63) // 64}, {S}>",
+                     "kernel": kernel,
                      "launch_ms": [round(x, 3) for x in launch_ms]},
     }
     if not a.no_cpu:
