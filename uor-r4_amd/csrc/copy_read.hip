@@ -487,7 +487,7 @@ extern "C" int uor_copy_mean_rows_async(void *handle, const uint32_t *d_tokens,
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(h->device);
   // Four streams a block, or two where their distances would pass 64 KB of LDS (strides above
-  // 3,840). The vector form wants rows of whole 8-byte pieces.
+  // 3,776). The vector form wants rows of whole 8-byte pieces.
   const uint32_t pitch = (stride + 63u) & ~63u;
   const uint32_t waves = kWaves * wave_lds_bytes(stride) <= (64u << 10) ? kWaves : kWaves / 2;
   const uint32_t w = h->d.width;
