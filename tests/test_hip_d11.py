@@ -174,3 +174,21 @@ def test_traced_evaluation_api():
     finally:
         ko.close()
         model.close()
+
+
+@pytest.mark.parametrize("mode,kept,sweeps", [("flock", 1, 0), ("flock", 8, 0), ("relation", 1, 1),
+                                              ("relation", 7, 5), ("relation", 8, 2)])
+@pytest.mark.parametrize("vocab", [3, 400])
+def test_kept_nodes_at_the_edges_of_the_lanes(mode, kept, sweeps, vocab):
+    # Levels of as many nodes as lanes and one more or less, and of a few tokens: most nodes tie in score
+    # and frame, and the last positions decide which are kept. Every gate is set.
+    art = d11.synthetic(vocabulary=vocab, blocks=3, context=243, kept_cells=3, read_mode=mode, read_kept=kept,
+                        read_sweeps=sweeps, seed=40 + kept, trunk=False, gate_density=1.0)
+    edges = [1, 2, 3, 8, 9, 10, 26, 27, 28, 63, 64, 65, 66, 80, 81, 127, 128, 129, 130, 191, 192, 193, 194, 195, 196,
+             242, 243]
+    pre, lens, tg = d11.panel_rows(art, 4 * len(edges), 41)
+    lens[:] = np.repeat(edges, 4)
+    got = gpu_rows(art, pre, lens, tg)
+    want = oracle.d11_score_rows(art, pre, lens, tg, threads=8)
+    assert (want["status"] == 0).all()
+    assert_same(got, want)

@@ -37,7 +37,7 @@ constexpr int kWaves = 8;  // rows per block
 constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxNodes = 512;
 constexpr int kMaxLevels = 8;
-constexpr int kPerLane = kMaxNodes / 64;  // a level's nodes per lane
+constexpr int kPerLane = (UOR_D11_MAX_CONTEXT + 63) / 64;  // a level's nodes per lane (no level exceeds its atoms)
 constexpr uint32_t kNone = 0x1ff;
 constexpr int kRecWords = sizeof(uor_d11_row_out) / 4;
 static_assert(sizeof(uor_d11_row_out) == 656, "record layout");
@@ -63,7 +63,7 @@ struct Geo {
   uint8_t bfs[256];
   uint8_t branch[16][4];
   uint8_t compose[64][64];  // state a after state b
-  int8_t roots[16][8];
+  alignas(8) int8_t roots[16][8];  // coordinates -2, 0 and 2
 };
 static_assert(sizeof(Geo) % 4 == 0, "staged in words");
 
@@ -286,6 +286,89 @@ __device__ int route_block(const DevModel &M, const Geo &g, const Plan &P, const
   return -1;
 }
 
+// The kept nodes of one level (discrete_d11.rs:1646-1712): the `kept` eligible ones with the largest
+// (relation score, nearness and Hamming nearness of the frame, last position), carried into the query's
+// frame; the sum of their roots to `sum`, their number returned. `n` nodes at order[begin], a node a
+// lane and slot, at most 64 N; `none`: every node scores 0 (the Flock read).
+// A score is at most 72 * 10^4 in magnitude (a first sweep sums 9 neighbours of 0..8, each further one adds
+// 9 of the last), so that a key of 32 bits holds it beside the two nearnesses. Only the set enters
+// the sum, not its order: the loop goes down the distinct keys, taking all nodes of one at a time,
+// and where a key has more than are still wanted, the later ones go first (a level's nodes lie in the
+// order of their last positions), which a ballot ranks at once. The kept nodes' roots are then looked
+// up by their own lanes together and summed as bytes. Bound by vector instructions; `kept` successive maxima of
+// 64-bit keys over eight slots a lane, with a chain of lookups each, took 608 us for 14,287 rows of
+// 186-192 tokens, this form 519.
+template <int N>
+__device__ __forceinline__ int kept_sum(const Geo &g, const Plan &P, const WaveLds &w, int begin, int n, int len,
+                                        int qf, int kept, bool none, int lane, int32_t (&sum)[8]) {
+  static_assert(UOR_D11_MAX_SWEEPS <= 5 && UOR_D11_MAX_KEPT <= 8, "the key's and the byte sums' ranges");
+  uint32_t key[N];
+  int node[N];
+  uint64_t all[N];
+  int eligible = 0;
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    key[j] = 0;
+    node[j] = 0;
+    const int k = lane + 64 * j;
+    if (k < n) {
+      const int i = P.order[begin + k];
+      const int last = P.link[i] >> 8 & 0xff;
+      if (last + 1 < len) {
+        const int fr = w.frame[i];
+        node[j] = i;
+        key[j] = (uint32_t)((none ? 0 : w.rel[i]) + (1 << 23)) << 8 | (uint32_t)(15 - g.dist[qf][fr]) << 4 |
+                 (uint32_t)(15 - g.ham[qf][fr]);
+      }
+    }
+    all[j] = __ballot(key[j] != 0);
+    eligible += __popcll(all[j]);
+  }
+  // What is taken: the keys above `m` and, of those equal to it, the latest `need`.
+  uint32_t m = 0;
+  int need = 0;
+  if (eligible > kept) {
+    m = 0xffffffffu;
+    need = kept;
+    for (;;) {
+      uint32_t top = 0;
+#pragma unroll
+      for (int j = 0; j < N; j++) top = max(top, key[j] < m ? key[j] : 0u);
+      m = wave_max32(top);
+      int count = 0;
+#pragma unroll
+      for (int j = 0; j < N; j++) count += __popcll(__ballot(key[j] == m));
+      if (count >= need) break;  // eligible > kept: some key gets here
+      need -= count;
+    }
+  }
+  // Sums of coordinates + 2 as bytes: at most 8 * 4.
+  uint32_t lo = 0, hi = 0;
+  int later = 0;
+#pragma unroll
+  for (int j = N - 1; j >= 0; j--) {
+    const uint64_t same = __ballot(key[j] == m);
+    const int rank = later + __popcll(same >> lane) - 1;
+    later += __popcll(same);
+    if (key[j] > m || (key[j] == m && rank < need)) {
+      const int cr = g.act[g.bfs[(w.frame[node[j]] << 4) + qf]][w.payload[node[j]]];
+      const uint2 r = *(const uint2 *)g.roots[cr];
+      // Bytes -2, 0, 2 as 0, 2, 4, without a carry between them.
+      lo += (r.x ^ 0x80808080u) - 0x7e7e7e7eu;
+      hi += (r.y ^ 0x80808080u) - 0x7e7e7e7eu;
+    }
+  }
+  lo = wave_sum32(lo);
+  hi = wave_sum32(hi);
+  const int found = eligible < kept ? eligible : kept;
+#pragma unroll
+  for (int d = 0; d < 4; d++) {
+    sum[d] = (int32_t)(lo >> (8 * d) & 0xff) - 2 * found;
+    sum[d + 4] = (int32_t)(hi >> (8 * d) & 0xff) - 2 * found;
+  }
+  return found;
+}
+
 // flock_or_relation_read (discrete_d11.rs:1453-1741) of block b. TR: the block's trace words
 // at `tw` (header, then 28 words a level, every level visited whatever its gate, :1480-1738)
 // and, for the relation read, its scores at `rw` padded to M.rel_stride (:1640-1644).
@@ -409,67 +492,58 @@ __device__ int flock_block(const DevModel &M, const Geo &g, const Plan &P, WaveL
   for (int l = 0; l < S; l++) {
     const int gate = M.gates[b * S + l];
     if (!TR && gate == 0) continue;
-    uint64_t mk[kPerLane];
-#pragma unroll
-    for (int j = 0; j < kPerLane; j++) {
-      mk[j] = 0;
-      const int k = P.level_start[l] + lane + 64 * j;
-      if (l < kMaxLevels && k < P.level_start[l + 1]) {
-        const int i = P.order[k];
-        const uint32_t lst = P.link[i] >> 8 & 0xff;
-        if ((int)lst + 1 < len) {
-          const int fr = w.frame[i];
-          const uint32_t r = relation ? (uint32_t)w.rel[i] ^ 0x80000000u : 0x80000000u;
-          mk[j] = (uint64_t)r << 32 | (uint64_t)(15 - g.dist[qf][fr]) << 28 |
-                  (uint64_t)(15 - g.ham[qf][fr]) << 24 | (uint64_t)lst << 16 |
-                  (uint64_t)(kNone - (uint32_t)i);
-        }
-      }
-    }
     int32_t sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int found = 0;
-    // Only the kept set enters the sum: when the eligible nodes fit, take them all.
-    uint32_t mine = 0;
-#pragma unroll
-    for (int j = 0; j < kPerLane; j++) mine += mk[j] != 0;
-    const uint32_t eligible = wave_sum32(mine);
-    // The level's trace word this lane writes: kept nodes at 4 + k, their route states at 12 + k,
-    // the carried roots at 20 + k, in selection order (the ordered selection always runs).
-    uint32_t tv = 0xffffffffu;
-    if (!TR && (int)eligible <= kept) {
+    if constexpr (!TR) {
+      const int begin = __builtin_amdgcn_readfirstlane(P.level_start[l]);
+      const int n = __builtin_amdgcn_readfirstlane(P.level_start[l + 1]) - begin;
+      found = n <= 64 ? kept_sum<1>(g, P, w, begin, n, len, qf, kept, !relation, lane, sum)
+                      : kept_sum<kPerLane>(g, P, w, begin, n, len, qf, kept, !relation, lane, sum);
+    } else {
+      // In selection order: the level's trace word this lane writes is node r's at 4 + r, its route
+      // state at 12 + r and its carried root at 20 + r.
+      uint64_t mk[kPerLane];
+      uint32_t mine = 0;
 #pragma unroll
       for (int j = 0; j < kPerLane; j++) {
-        if (mk[j]) {
-          const int node = (int)(kNone - (uint32_t)(mk[j] & kNone));
-          const int cr = g.act[g.bfs[(w.frame[node] << 4) + qf]][w.payload[node]];
-#pragma unroll
-          for (int d = 0; d < 8; d++) sum[d] += g.roots[cr][d];
+        mk[j] = 0;
+        const int k = P.level_start[l] + lane + 64 * j;
+        if (k < P.level_start[l + 1]) {
+          const int i = P.order[k];
+          const uint32_t lst = P.link[i] >> 8 & 0xff;
+          if ((int)lst + 1 < len) {
+            const int fr = w.frame[i];
+            const uint32_t r = relation ? (uint32_t)w.rel[i] ^ 0x80000000u : 0x80000000u;
+            mk[j] = (uint64_t)r << 32 | (uint64_t)(15 - g.dist[qf][fr]) << 28 |
+                    (uint64_t)(15 - g.ham[qf][fr]) << 24 | (uint64_t)lst << 16 |
+                    (uint64_t)(kNone - (uint32_t)i);
+          }
         }
+        mine += mk[j] != 0;
       }
+      const uint32_t eligible = wave_sum32(mine);
+      uint32_t tv = 0xffffffffu;
+      for (int r = 0; r < kept; r++) {
+        uint64_t loc = 0;
 #pragma unroll
-      for (int d = 0; d < 8; d++) sum[d] = (int32_t)wave_sum32((uint32_t)sum[d]);
-      found = (int)eligible;
+        for (int j = 0; j < kPerLane; j++) loc = mk[j] > loc ? mk[j] : loc;
+        const uint64_t m = wave_max64(loc);
+        if (m == 0) break;
+#pragma unroll
+        for (int j = 0; j < kPerLane; j++)
+          if (mk[j] == m) mk[j] = 0;
+        const int node = (int)(kNone - (uint32_t)(m & kNone));
+        const int act = g.bfs[(w.frame[node] << 4) + qf];
+        const int cr = g.act[act][w.payload[node]];
+        tv = lane == 4 + r ? (uint32_t)node : lane == 12 + r ? (uint32_t)act : lane == 20 + r ? (uint32_t)cr : tv;
+#pragma unroll
+        for (int d = 0; d < 8; d++) sum[d] += g.roots[cr][d];
+        found++;
+      }
+      if (lane < 28 && lane != 2)
+        tw[4 + 28 * l + lane] = lane == 0 ? (uint32_t)(gate + 1) : lane == 1 ? (uint32_t)found
+                                : lane == 3 ? eligible : tv;
     }
-    for (int r = 0; (TR || (int)eligible > kept) && r < kept; r++) {
-      uint64_t loc = 0;
-#pragma unroll
-      for (int j = 0; j < kPerLane; j++) loc = mk[j] > loc ? mk[j] : loc;
-      const uint64_t m = wave_max64(loc);
-      if (m == 0) break;
-#pragma unroll
-      for (int j = 0; j < kPerLane; j++)
-        if (mk[j] == m) mk[j] = 0;
-      const int node = (int)(kNone - (uint32_t)(m & kNone));
-      const int act = g.bfs[(w.frame[node] << 4) + qf];
-      const int cr = g.act[act][w.payload[node]];
-      if (TR) tv = lane == 4 + r ? (uint32_t)node : lane == 12 + r ? (uint32_t)act : lane == 20 + r ? (uint32_t)cr : tv;
-#pragma unroll
-      for (int d = 0; d < 8; d++) sum[d] += g.roots[cr][d];
-      found++;
-    }
-    if (TR && lane < 28 && lane != 2)
-      tw[4 + 28 * l + lane] = lane == 0 ? (uint32_t)(gate + 1) : lane == 1 ? (uint32_t)found
-                              : lane == 3 ? eligible : tv;
     if (found == 0) {
       if (TR && lane == 2) tw[4 + 28 * l + 2] = 0xffffffffu;
       continue;
