@@ -3,6 +3,7 @@ one wavefront a sequence, which takes no layer by layer launch) and the oracle: 
 the edges of the stretches, widths and windows, fresh and resumed sessions, refused tokens and full
 contexts. Every output is an integer and equal."""
 
+import ctypes as C
 from dataclasses import replace
 
 import numpy as np
@@ -27,6 +28,7 @@ SHAPES = {
     # The shortest window over the reference's cells, and the whole-table head.
     "w64": synth.Spec(vocab=4096, width=64, mlp=96, layers=2, context=96, kept=8, window=1),
 }
+DEEP = synth.Spec(vocab=512, width=1024, mlp=1024, layers=16, context=96, kept=4, window=64, drawers=32, probes=3)
 
 
 @pytest.fixture(scope="module")
@@ -188,3 +190,60 @@ def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
     # The matches of all rows: the choices against the next tokens of the positions served.
     served = np.cumsum(t >= SHAPES["w512i8"].vocab, axis=1) == 0
     assert got[4][0] == ((got[0][:, :-1] == t[:, 1:]) & served[:, :-1]).sum() == got[6][0]
+
+
+def _capture(stream, call):
+    """`call` recorded on `stream`, as an executable graph."""
+    rt = runtime()
+    graph, run = C.c_void_p(), C.c_void_p()
+    assert rt.hipStreamBeginCapture(stream, 0) == 0  # global mode: an allocation ends the capture
+    try:
+        call()
+    finally:
+        ended = rt.hipStreamEndCapture(stream, C.byref(graph))
+    assert ended == 0
+    assert rt.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    assert rt.hipGraphDestroy(graph) == 0
+    return run
+
+
+@pytest.mark.parametrize("call", ["score", "sequences", "decode", "decode in parts"])
+def test_calls_captured_after_a_warm_up(call):
+    # The warm-up goes by layers, the captured call by the step kernels, whose buffers the warm-up left:
+    # nothing is allocated under capture, and every replay equals the direct call.
+    parts = call == "decode in parts"  # the workspace holds fewer of DEEP's sessions than run together
+    spec, n, length = (DEEP, 500, 70) if parts else (SHAPES["w128"], 40, 24)
+    model = hip.Model(synth.make_artifact(spec, 31))
+    rt, lib, h = runtime(), hip.lib(), model.handle
+    t = synth.uniform_prompts(spec.vocab, n, length, 21)
+    tok, status = _up(t, np.uint32), DeviceArray(n, np.int32)
+    if call == "score":
+        outs = [DeviceArray((n, length), np.uint32), DeviceArray(1, np.uint64), status]
+        launch = lambda st: lib.uor_fbs_score_async(h, tok.ptr, n, length, *[o.ptr for o in outs], st)  # noqa: E731
+    elif call == "sequences":
+        outs = [DeviceArray((n, length), np.uint32), DeviceArray((n, length, model.probes), np.uint32),
+                DeviceArray((n, length, model.width), np.int32), status]
+        launch = lambda st: lib.uor_fbs_sequences_async(h, tok.ptr, n, length, *[o.ptr for o in outs], st)  # noqa: E731
+    else:
+        outs = [DeviceArray((n, 2), np.uint32), status]
+        launch = lambda st: lib.uor_fbs_decode_async(h, tok.ptr, n, length, 1, outs[0].ptr, *[None] * 6,  # noqa: E731
+                                                     status.ptr, st)
+    stream = C.c_void_p()
+    assert rt.hipStreamCreate(C.byref(stream)) == 0
+    print(f"{call}: warm-up", flush=True)
+    hip._check(launch(stream))
+    assert rt.hipStreamSynchronize(stream) == 0
+    want = [o.download() for o in outs]
+    print("capture", flush=True)
+    run = _capture(stream, lambda: hip._check(launch(stream)))
+    for _ in range(3):
+        for o in outs:
+            o.zero()
+        assert rt.hipDeviceSynchronize() == 0
+        assert rt.hipGraphLaunch(run, stream) == 0
+        assert rt.hipStreamSynchronize(stream) == 0
+        for o, w in zip(outs, want):
+            np.testing.assert_array_equal(o.download(), w)
+        rows(model, t[:3])  # the program's own calls between the replays
+    assert rt.hipGraphExecDestroy(run) == 0
+    assert rt.hipStreamDestroy(stream) == 0

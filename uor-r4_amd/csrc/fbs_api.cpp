@@ -1046,6 +1046,13 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
     }
   }
   *taken = true;
+  // The same call under capture runs on the step kernels, where nothing may be allocated: the call that
+  // warms up for it leaves the ring that it needs, also where the parts (or rows, which need none) do not.
+  const std::string error = g_last_error;
+  if (h->ensure_ring(A.n < h->pair_grid ? A.n : h->pair_grid)) {
+    (void)hipGetLastError();  // no room: rows run without it, a decode's step launches report it
+    g_last_error = error;
+  }
   const size_t ld = (size_t)M.L * M.d;
   for (uint32_t s0 = 0; s0 < A.n; s0 += part) {
     const uint32_t n = A.n - s0 < part ? A.n - s0 : part;
