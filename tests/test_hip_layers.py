@@ -192,6 +192,24 @@ def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
     assert got[4][0] == ((got[0][:, :-1] == t[:, 1:]) & served[:, :-1]).sum() == got[6][0]
 
 
+@pytest.mark.parametrize("n,length", [(3, 96), (2, 600)])
+def test_scored_rows_take_their_choices_in_place(n, length):
+    # A score call whose choices go over its rows counts the matches of the rows as they came in, at
+    # the edges of wavefronts and of rounds of 256 positions.
+    model = hip.Model(synth.make_artifact(replace(SHAPES["w128"], context=600), 31))
+    t = synth.uniform_prompts(SHAPES["w128"].vocab, n, length, 22)
+    for _ in range(12):  # every other token the choice before it, as far as twelve rounds settle them
+        t[:, 1::2] = model.sequences(t)[0][:, :-1:2]
+    want_choices = model.sequences(t)[0]
+    want = int((want_choices[:, :-1] == t[:, 1:]).sum())
+    assert 0 < want < n * (length - 1)
+    tok, matches, status = _up(t, np.uint32), DeviceArray(1, np.uint64), DeviceArray(n, np.int32)
+    hip._check(hip.lib().uor_fbs_score_async(model.handle, tok.ptr, n, length, tok.ptr, matches.ptr, status.ptr, None))
+    assert runtime().hipDeviceSynchronize() == 0
+    np.testing.assert_array_equal(tok.download(), want_choices)
+    assert int(matches.download()[0]) == want and not status.download().any()
+
+
 def _capture(stream, call):
     """`call` recorded on `stream`, as an executable graph."""
     rt = runtime()

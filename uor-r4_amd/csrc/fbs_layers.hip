@@ -794,18 +794,24 @@ __global__ __launch_bounds__(64, 2) void fbs_layer_scan(DevModel M, ServeScan J)
   }
 }
 
-// The stretch's choices to the rows' place and their matches with the rows' next tokens.
+// The stretch's choices to the rows' place and their matches with the rows' next tokens. The choices may go
+// over the rows themselves, as a step's choice goes over its own token: a round's next tokens are read
+// before any of its choices is written.
 __global__ __launch_bounds__(256) void fbs_layer_choices(LayerArgs P) {
   const uint32_t s = blockIdx.x;
   const uint32_t steps = P.steps[s];
   const uint32_t *tok = P.tokens + (uint64_t)s * P.row + P.start;
   uint32_t hits = 0;
-  for (uint32_t t = threadIdx.x; t < steps; t += blockDim.x) {
-    const bool next = P.start + t + 1 < P.row;
-    if (!P.out_tokens && !next) continue;
-    const uint32_t c = P.chosen[(uint64_t)s * P.len + t];
-    if (P.out_tokens) P.out_tokens[(uint64_t)s * P.row + P.start + t] = c;
-    hits += next && c == tok[t + 1];
+  for (uint32_t t0 = 0; t0 < steps; t0 += blockDim.x) {
+    const uint32_t t = t0 + threadIdx.x;
+    const bool in = t < steps, next = in && P.start + t + 1 < P.row;
+    const uint32_t after = next ? tok[t + 1] : 0;
+    const uint32_t c = next || (in && P.out_tokens) ? P.chosen[(uint64_t)s * P.len + t] : 0;
+    if (P.out_tokens) {
+      __syncthreads();
+      if (in) P.out_tokens[(uint64_t)s * P.row + P.start + t] = c;
+    }
+    hits += next && c == after;
   }
   hits = wave_reduce32(hits, OpAdd());
   if (P.matches && threadIdx.x % kWave == 0 && hits) atomicAdd(P.matches, (unsigned long long)hits);
