@@ -188,13 +188,33 @@ void uor_fbs_model_destroy(uor_fbs_handle *handle);
 uint64_t uor_fbs_state_words(const uor_fbs_handle *handle);
 uint64_t uor_fbs_history_words(const uor_fbs_handle *handle);
 
-/* Wavefronts per sequence of the kernels a run of n sequences launches: 2 (paired blocks, at
- * most one block per SIMD, each stepping its share of the sequences) unless
+/* Wavefronts per sequence of the step kernels that a run of n sequences launches: 2 (paired blocks,
+ * at most one block per SIMD, each stepping its share of the sequences) unless
  * UOR_FBS_BLOCK_WAVES=1 was set at model creation or the model's paired LDS does not fit, then
  * 1 (one wavefront per sequence). The same for every n today; n is kept for a policy that
- * depends on the batch. No counterpart in the reference (its CPU decoder has no launch shape):
+ * depends on the batch. Tokens that are known beforehand may run by layers instead
+ * (uor_fbs_layer_calls). No counterpart in the reference (its CPU decoder has no launch shape):
  * for profilers and tests. */
 uint32_t uor_fbs_block_waves(const uor_fbs_handle *handle, uint32_t n);
+
+/* The layer by layer path: on a model whose step kernels are paired, with raw gates and transitions and
+ * no Hamming reads, a prompt's tokens but its last (uor_fbs_decode and its _async and _stream forms),
+ * and teacher-forced rows (uor_fbs_sequences, uor_fbs_score and their _async forms; not with the
+ * nearest head), run each layer over all their positions at once wherever that takes less time than
+ * step after step: from about 4 prompt tokens of one sequence and 12 of a thousand. The results
+ * are the steps'. Such a call works in device memory that the handle allocates when it first needs
+ * it, grows, and keeps until the model is destroyed: at most 2 GiB (longer or larger calls run
+ * in parts), or the environment variable UOR_FBS_LAYER_BYTES at model creation where that is
+ * smaller (0: no call runs by layers), and for rows the buffers of up to 32,768 queries beside it.
+ * Where the device has no room, the call runs in smaller parts or step after step. A call on a stream
+ * under capture runs step after step, with what the same call before it has allocated.
+ * `uor_fbs_layer_calls`: the handle's calls that ran by layers; `uor_fbs_layer_bytes`: the
+ * device bytes it holds for them. No counterpart in the reference.
+ *
+ * A handle's launches share its scratch memory (window rings, this workspace, the serving launches'
+ * job buffers): calls on one handle run one at a time, on one stream or ordered by the caller. */
+uint64_t uor_fbs_layer_calls(const uor_fbs_handle *handle);
+uint64_t uor_fbs_layer_bytes(const uor_fbs_handle *handle);
 
 /* Teacher-forced sequences from fresh sessions: every position's chosen token, kept drawers
  * (best first) and Q12 query. Same contract as fbs_host_sequences (host_kernel.cpp:16-29)

@@ -192,6 +192,40 @@ def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
     assert got[4][0] == ((got[0][:, :-1] == t[:, 1:]) & served[:, :-1]).sum() == got[6][0]
 
 
+def test_the_workspace_keeps_to_its_bound(models, monkeypatch):
+    # 2 MiB hold some 600 positions of width 128: 50 sequences of 90 run in parts or in stretches of 64.
+    art, _, steps = models("w128", monkeypatch)
+    t = tokens_for("w128", 50, 90, 23)
+    monkeypatch.setenv("UOR_FBS_LAYER_BYTES", str(2 << 20))
+    small = hip.Model(art)
+    for g, w in zip(decode(small, t, 1), decode(steps, t, 1)):
+        np.testing.assert_array_equal(g, w)
+    assert small.layer_calls == 1 and 0 < small.layer_bytes <= 2 << 20
+    for g, w in zip(rows(small, t), rows(steps, t)):
+        np.testing.assert_array_equal(g, w)
+    assert small.layer_calls == 4
+    monkeypatch.setenv("UOR_FBS_LAYER_BYTES", "0")
+    none = hip.Model(art)
+    with pytest.raises(hip.FbsError):
+        hip._check(hip.lib().uor_fbs_decode_async(none.handle, None, 1, 1, 0, *[None] * 9))
+    error = hip.lib().uor_fbs_last_error()
+    for g, w in zip(decode(none, t, 1), decode(steps, t, 1)):
+        np.testing.assert_array_equal(g, w)
+    assert none.layer_calls == none.layer_bytes == 0 and hip.lib().uor_fbs_last_error() == error
+
+
+def test_the_workspace_grows_in_few_steps(models, monkeypatch):
+    # Prompts and rows that get longer call by call (the larger sizes allocate by doubling).
+    art = models("w128", monkeypatch)[0]
+    for call in (lambda m, t: decode(m, t, 0), lambda m, t: m.score(t)):
+        model = hip.Model(art)
+        held = []
+        for length in range(16, 64):
+            call(model, tokens_for("w128", 8, length, 24))
+            held.append(model.layer_bytes)
+        assert model.layer_calls == len(held) and held == sorted(held) and len(set(held)) <= 5
+
+
 @pytest.mark.parametrize("n,length", [(3, 96), (2, 600)])
 def test_scored_rows_take_their_choices_in_place(n, length):
     # A score call whose choices go over its rows counts the matches of the rows as they came in, at

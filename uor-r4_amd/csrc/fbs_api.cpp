@@ -78,6 +78,8 @@ bool grid_valid(int16_t code) {  // kernels.rs:116-120
 
 }  // namespace
 
+constexpr size_t kLayerBytes = (size_t)2 << 30;  // the layers' workspace: under 1 % of the card's memory
+
 struct uor_fbs_handle {
   int device = 0;
   DevModel M{};
@@ -114,6 +116,7 @@ struct uor_fbs_handle {
   uint32_t serve_nchunks = 0, serve_max_chunks = 0;
   struct Jobs {
     uint32_t cap = 0, item_cap = 0;
+    size_t bytes = 0;
     uint32_t *query = nullptr, *flag = nullptr, *drawer_count = nullptr, *drawer_list = nullptr,
              *item_count = nullptr;
     uint4 *items = nullptr;
@@ -153,13 +156,14 @@ struct uor_fbs_handle {
     }
   };
   Jobs jobs;
-  // The layer by layer launches (fbs_layers.hip): their workspace (grown, at most kLayerBytes) and,
+  // The layer by layer launches (fbs_layers.hip): their workspace (grown, at most layer_budget) and,
   // for scored rows, job buffers of their own, so that a row launch never moves the buffers that a
   // captured serving launch holds.
   bool taps_high = true;   // every tap word lies within +-2^27
   bool keep_small = true;  // every keep_q31 is below 2^31: the kernels take it as 32 bits
   unsigned char *layers = nullptr;
-  size_t layers_bytes = 0;
+  size_t layers_bytes = 0, layer_budget = kLayerBytes;
+  uint64_t layer_calls = 0;
   Jobs row_jobs;
 
   ~uor_fbs_handle() {
@@ -184,20 +188,29 @@ struct uor_fbs_handle {
   }
 
   // The deferred writer's job buffers for n sequences: flags and drawer counts start at zero
-  // (a fill kernel on `stream`; the hand-out kernel clears what a launch set).
-  int ensure_jobs(Jobs &b, uint32_t n, hipStream_t stream) {
+  // (a fill kernel on `stream`; the hand-out kernel clears what a launch set). Grown to n, or to twice
+  // what they were where that is at most `most`.
+  int ensure_jobs(Jobs &b, uint32_t n, hipStream_t stream, uint32_t most = 0) {
     if (n <= b.cap) return 0;
+    const uint32_t twice = b.cap > most / 2 ? most : 2 * b.cap;
+    n = n < twice ? twice : n;
     b.free();
     const size_t words = M.d / 2;
     const uint64_t cap = job_items(n);
     if (cap > 0xffffffffull) return fail(UOR_FBS_ERR_UNSUPPORTED, "too many serving sessions");
-    hipError_t e = hipMalloc((void **)&b.query, (size_t)n * words * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.flag, (size_t)n * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.best, (size_t)n * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.drawer_count, (size_t)M.D * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.drawer_list, (size_t)M.D * n * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.items, (size_t)cap * sizeof(uint4));
-    if (e == hipSuccess) e = hipMalloc((void **)&b.item_count, sizeof(uint32_t));
+    hipError_t e = hipSuccess;
+    const auto alloc = [&](auto **p, size_t count) {
+      const size_t bytes = count * sizeof **p;
+      if (e == hipSuccess) e = hipMalloc((void **)p, bytes);
+      b.bytes += bytes;
+    };
+    alloc(&b.query, (size_t)n * words);
+    alloc(&b.flag, n);
+    alloc(&b.best, n);
+    alloc(&b.drawer_count, M.D);
+    alloc(&b.drawer_list, (size_t)M.D * n);
+    alloc(&b.items, cap);
+    alloc(&b.item_count, 1);
     if (e != hipSuccess) {
       b.free();
       return hip_fail(e, "hipMalloc(serving jobs)");
@@ -213,20 +226,27 @@ struct uor_fbs_handle {
     return 0;
   }
 
-  // The layer by layer launches' workspace; false where the device has no room for it (the launch then
-  // takes the step kernels, which need none).
+  // The layer by layer launches' workspace of at least `bytes` (at most layer_budget), grown to twice what
+  // it was, so that calls of rising sizes wait for the device and allocate a few times only. False where
+  // the device has no room: the budget is then below `bytes`, also for later calls.
   bool ensure_layers(size_t bytes) {
     if (bytes <= layers_bytes) return true;
+    size_t want = 2 * layers_bytes < layer_budget ? 2 * layers_bytes : layer_budget;
+    if (want < bytes || !layers_bytes) want = bytes;
     if (layers) (void)hipFree(layers);
     layers = nullptr;
     layers_bytes = 0;
-    if (hipMalloc((void **)&layers, bytes) != hipSuccess) {
+    for (;; want = bytes) {
+      if (hipMalloc((void **)&layers, want) == hipSuccess) {
+        layers_bytes = want;
+        return true;
+      }
       (void)hipGetLastError();
       layers = nullptr;
-      return false;
+      if (want == bytes) break;
     }
-    layers_bytes = bytes;
-    return true;
+    layer_budget = bytes / 2;
+    return false;
   }
 
   // The scan's wavefronts take the items in turn: two a SIMD, or one an item.
@@ -719,6 +739,11 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
   // every step then scans its candidates; the results are the same either way).
   const char *wm = getenv("UOR_FBS_WRITER_MEMORY");
   M.writer_memory = (wm && wm[0] == '0' && !wm[1]) ? 0u : 1u;
+  // UOR_FBS_LAYER_BYTES=n bounds the layer by layer workspace to n bytes (0: no call goes by layers).
+  if (const char *lb = getenv("UOR_FBS_LAYER_BYTES"); lb && *lb) {
+    const unsigned long long n = strtoull(lb, nullptr, 10);
+    h->layer_budget = n < kLayerBytes ? (size_t)n : kLayerBytes;
+  }
   // UOR_FBS_SERVE_SCAN=fused keeps the writer inside one-token serving launches, =drawer takes
   // the drawer-major scan; otherwise the drawers' sizes choose (below). The results are the same
   // either way.
@@ -925,6 +950,11 @@ extern "C" uint32_t uor_fbs_block_waves(const uor_fbs_handle *h, uint32_t n) {
   return h && h->pair ? 2u : 1u;
 }
 
+extern "C" uint64_t uor_fbs_layer_calls(const uor_fbs_handle *h) { return h ? h->layer_calls : 0; }
+extern "C" uint64_t uor_fbs_layer_bytes(const uor_fbs_handle *h) {
+  return h ? h->layers_bytes + h->row_jobs.bytes : 0;
+}
+
 namespace {
 
 // The layer by layer path (fbs_layers.hip) takes the tokens that are known before any choice: a
@@ -935,7 +965,6 @@ namespace {
 // graph must not hold a workspace that a later launch may grow).
 // Measured at width 256 (6 layers, window 16): 300 prompts of 509 tokens 19.2 ms by the step kernels,
 // whose 509 steps run one after another, 3.8 ms by layers; 8,192 rows of 128 76 against 40 ms.
-constexpr size_t kLayerBytes = (size_t)2 << 30;  // the workspace: under 1 % of the card's memory
 constexpr uint32_t kLayerStretch = 64;   // tokens at once of a sequence that runs in several stretches
 constexpr uint32_t kLayerJobs = 32768;   // positions a scan
 constexpr size_t kLayerLists = 1 << 24;  // drawer-list entries a scan
@@ -1017,42 +1046,50 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
   // The sequences run together (`part` of them where the workspace does not hold them all: the grids'
   // second dimension, and for a decode whole turns of the step kernels' resident blocks), over all
   // their tokens or, where the workspace does not hold those, in stretches of `run` tokens, the
-  // sessions kept between them.
+  // sessions kept between them. Planned again within a smaller budget where the device refuses one.
   LayerArgs P{};
-  uint32_t part = A.n < 65535u ? A.n : 65535u, run = len;
+  uint32_t part, run;
   const auto bytes = [&](uint32_t n, uint32_t t) { return carve_layers(M, nullptr, n, t, !rows || t < len, rows, P); };
-  if (bytes(part, run) > kLayerBytes) {
+  do {
+    const size_t room = h->layer_budget;
+    part = A.n < 65535u ? A.n : 65535u, run = len;
+    if (bytes(part, run) <= room) continue;
     const uint32_t least = len < kLayerStretch ? len : kLayerStretch;
-    if (bytes(part, least) > kLayerBytes) {
+    if (bytes(part, least) > room) {
       uint32_t fit = 0;
       for (uint32_t bit = 1u << 15; bit; bit >>= 1)
-        if (fit + bit < part && bytes(fit + bit, least) <= kLayerBytes) fit += bit;
+        if (fit + bit < part && bytes(fit + bit, least) <= room) fit += bit;
       if (fit == 0) return 0;
       part = !rows && fit > h->pair_grid ? fit - fit % h->pair_grid : fit;
     }
     uint32_t most = least;
     for (uint32_t bit = 1u << 30; bit; bit >>= 1)
-      if (bit < len - most && bytes(part, most + bit) <= kLayerBytes) most += bit;
+      if (bit < len - most && bytes(part, most + bit) <= room) most += bit;
     const uint32_t stretches = (len + most - 1) / most;
     run = (len + stretches - 1) / stretches;
-  }
+  } while (!h->ensure_layers(bytes(part, run)));
   const bool sessions = !rows || run < len;
-  if (!h->ensure_layers(bytes(part, run))) return 0;
+  // A call that finds no room for what it can do without says nothing of it.
+  const std::string error = g_last_error;
+  const auto skip = [&] {
+    (void)hipGetLastError();
+    g_last_error = error;
+  };
   if (rows) {
     const uint64_t all = (uint64_t)part * run;
-    if (h->ensure_jobs(h->row_jobs, all < jobs ? (uint32_t)all : jobs, stream)) {
-      (void)hipGetLastError();  // no room: the step kernels, which need none
+    const uint32_t most = all < jobs ? (uint32_t)all : jobs;
+    if (h->ensure_jobs(h->row_jobs, most, stream, jobs) && h->ensure_jobs(h->row_jobs, most, stream)) {
+      skip();  // the step kernels need none
       return 0;
     }
+    skip();
   }
   *taken = true;
+  h->layer_calls++;
   // The same call under capture runs on the step kernels, where nothing may be allocated: the call that
   // warms up for it leaves the ring that it needs, also where the parts (or rows, which need none) do not.
-  const std::string error = g_last_error;
-  if (h->ensure_ring(A.n < h->pair_grid ? A.n : h->pair_grid)) {
-    (void)hipGetLastError();  // no room: rows run without it, a decode's step launches report it
-    g_last_error = error;
-  }
+  if (h->ensure_ring(A.n < h->pair_grid ? A.n : h->pair_grid))
+    skip();  // rows run without it, a decode's step launches report it
   const size_t ld = (size_t)M.L * M.d;
   for (uint32_t s0 = 0; s0 < A.n; s0 += part) {
     const uint32_t n = A.n - s0 < part ? A.n - s0 : part;

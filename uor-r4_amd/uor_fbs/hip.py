@@ -29,7 +29,7 @@ SYMBOLS = (
     "uor_fbs_last_error", "uor_fbs_model_create", "uor_fbs_model_destroy", "uor_fbs_state_words",
     "uor_fbs_history_words", "uor_fbs_sequences", "uor_fbs_sequences_async", "uor_fbs_decode",
     "uor_fbs_decode_async", "uor_fbs_decode_noalloc_async", "uor_fbs_score",
-    "uor_fbs_score_async", "uor_fbs_block_waves",
+    "uor_fbs_score_async", "uor_fbs_block_waves", "uor_fbs_layer_calls", "uor_fbs_layer_bytes",
     "uor_fbs_decode_slots_async", "uor_fbs_index_workspace_bytes", "uor_fbs_index_build_async",
     "uor_fbs_index_update_async", "uor_fbs_index_remove_async", "uor_fbs_index_validate_async",
     "uor_fbs_index_probe_async", "uor_fbs_index_full_scan_async", "uor_fbs_stream_words",
@@ -68,6 +68,9 @@ def lib():
         L.uor_fbs_history_words.restype = C.c_uint64
         L.uor_fbs_block_waves.argtypes = [P, C.c_uint32]
         L.uor_fbs_block_waves.restype = C.c_uint32
+        for f in (L.uor_fbs_layer_calls, L.uor_fbs_layer_bytes):
+            f.argtypes = [P]
+            f.restype = C.c_uint64
         L.uor_fbs_sequences.argtypes = [P, P, C.c_uint32, C.c_uint32, P, P, P]
         L.uor_fbs_sequences_async.argtypes = [P, P, C.c_uint32, C.c_uint32, P, P, P, P, P]
         L.uor_fbs_decode.argtypes = [P, P, C.c_uint32, C.c_uint32, C.c_uint32, P, P, P, P, P, P, P]
@@ -169,6 +172,16 @@ class Model:
     def block_waves(self, n: int) -> int:
         """Wavefronts per sequence of the kernels a run of n sequences launches (1 or 2)."""
         return int(lib().uor_fbs_block_waves(self.handle, n))
+
+    @property
+    def layer_calls(self) -> int:
+        """The model's calls so far whose known tokens ran by layers."""
+        return int(lib().uor_fbs_layer_calls(self.handle))
+
+    @property
+    def layer_bytes(self) -> int:
+        """Device bytes that the model holds for such calls."""
+        return int(lib().uor_fbs_layer_bytes(self.handle))
 
     def sequences(self, tokens, want_kept=True, want_query=True):
         """Teacher-forced runs from fresh sessions: (tokens [S,len], kept [S,len,P], query [S,len,d])."""
