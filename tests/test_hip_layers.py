@@ -192,6 +192,45 @@ def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
     assert got[4][0] == ((got[0][:, :-1] == t[:, 1:]) & served[:, :-1]).sum() == got[6][0]
 
 
+@pytest.mark.parametrize("name,window", [("w128", 16), ("w96", 5), ("w320", 40)])
+@pytest.mark.parametrize("beyond", [False, True])
+def test_layers_with_the_smallest_and_largest_taps(monkeypatch, name, window, beyond):
+    # Codes whose shifts have no word of the common form (1 and 29 to 37) in the second layer, which alone
+    # takes the other form: the model still goes by layers, and equals the one-wavefront kernels and the oracle.
+    # Beyond: the third layer has codes without any word (shifts of 0 and 63), and no call goes by layers.
+    spec = replace(SHAPES[name], window=window, layers=3)
+    art = synth.make_artifact(spec, 33)
+    rng = np.random.default_rng(25)
+    for layer, fields in ((1, [67] + list(range(31, 40))), (2, [68, 5])):
+        taps = art.layers[layer].wide_taps
+        at = rng.permutation(taps.size)[:taps.size // 3]
+        if layer == 1 or beyond:
+            field = np.array(fields)[rng.integers(0, len(fields), at.size)]
+            taps[at] = (field * 16 + rng.integers(0, 16, at.size)) * rng.choice([-1, 1], at.size)
+    layers = hip.Model(art)
+    monkeypatch.setenv("UOR_FBS_BLOCK_WAVES", "1")
+    steps = hip.Model(art)
+    monkeypatch.setenv("UOR_FBS_BLOCK_WAVES", "0")
+    monkeypatch.setenv("UOR_FBS_LAYER_BYTES", "0")
+    pairs = hip.Model(art)
+    t = synth.uniform_prompts(spec.vocab, 3, 43, 26)
+    st, want_tok, want_kept, want_query = oracle.sequences(art, t, threads=2)
+    assert st == 0
+    for model in (layers, steps, pairs):
+        got = rows(model, t)
+        for g, w in zip(got, (want_tok, want_kept, want_query)):
+            np.testing.assert_array_equal(g, w)
+    # States over all their values, so that the window's largest terms meet the transport's wide form.
+    state = rng.integers(-2**63, 2**63 - 1, (3, layers.state_words), dtype=np.int64) >> 30
+    history = rng.integers(-2**31, 2**31 - 1, (3, layers.history_words), dtype=np.int32)
+    resume = (state, history, np.arange(3, dtype=np.uint32))
+    want = decode(steps, t, 2, resume)
+    for model in (layers, pairs):
+        for g, w in zip(decode(model, t, 2, resume), want):
+            np.testing.assert_array_equal(g, w)
+    assert layers.layer_calls == (0 if beyond else 4) and steps.layer_calls == pairs.layer_calls == 0
+
+
 def test_the_workspace_keeps_to_its_bound(models, monkeypatch):
     # 2 MiB hold some 600 positions of width 128: 50 sequences of 90 run in parts or in stretches of 64.
     art, _, steps = models("w128", monkeypatch)

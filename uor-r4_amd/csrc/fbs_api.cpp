@@ -159,7 +159,7 @@ struct uor_fbs_handle {
   // The layer by layer launches (fbs_layers.hip): their workspace (grown, at most layer_budget) and,
   // for scored rows, job buffers of their own, so that a row launch never moves the buffers that a
   // captured serving launch holds.
-  bool taps_high = true;   // every tap word lies within +-2^27
+  bool taps_high = true;   // every tap_word lies within +-2^27
   bool keep_small = true;  // every keep_q31 is below 2^31: the kernels take it as 32 bits
   unsigned char *layers = nullptr;
   size_t layers_bytes = 0, layer_budget = kLayerBytes;
@@ -732,7 +732,7 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
   M.prog_words = M.p_dec / 2 + kWave * Q;
   M.xbar_words = 2 * (d > mlp ? d : mlp);
   M.identity_rows = r.head == 1;
-  M.taps_fast = 1;
+  M.tap_layers = M.tap_pairs = 0;
   M.gains_fast = 1;
   M.log2d = (d & (d - 1)) == 0 ? (uint32_t)__builtin_ctz(d) : 0xffu;
   // UOR_FBS_WRITER_MEMORY=0 turns the writer's memory of its last query off (for measurement:
@@ -774,11 +774,24 @@ extern "C" int uor_fbs_model_create(const uor_fbs_model *m, const uor_fbs_ext *e
     if ((st = h->upload(taps, (size_t)(r.W + 1) * d, &dl.taps))) return done(st);
     {
       std::vector<uint16_t> rg(d), mg(d);
+      // The taps' words: tap_word's, or tap_pair's for all of a layer that has a tap without one.
       const size_t nt = (size_t)(r.W + 1) * d;
+      int32_t *const words = tap_words.data() + l * nt;
+      bool pairs = false, high = true;
       for (size_t i = 0; i < nt; i++) {
-        tap_words[l * nt + i] = tap_word(taps[i]);
-        if (tap_words[l * nt + i] == kTapWordNone) M.taps_fast = 0;
-        h->taps_high = h->taps_high && tap_words[l * nt + i] < (1 << 27) && tap_words[l * nt + i] > -(1 << 27);
+        words[i] = tap_word(taps[i]);
+        pairs = pairs || words[i] == kTapWordNone;
+        high = high && words[i] < (1 << 27) && words[i] > -(1 << 27);
+      }
+      if (pairs) {
+        for (size_t i = 0; i < nt; i++) {
+          words[i] = tap_pair(taps[i]);
+          pairs = pairs && words[i] != kTapWordNone;
+        }
+        M.tap_pairs |= (uint64_t)pairs << l;
+      } else {
+        M.tap_layers |= 1ull << l;
+        h->taps_high = h->taps_high && high;
       }
       for (uint32_t i = 0; i < d; i++) {
         rg[i] = gain_desc(ly.rec_gain[i]);
@@ -971,8 +984,8 @@ constexpr size_t kLayerLists = 1 << 24;  // drawer-list entries a scan
 
 bool layer_model(const uor_fbs_handle *h, bool rows) {
   const DevModel &M = h->M;
-  return h->pair && h->keep_small && !M.ham.heads && M.raw_gates && M.raw_transition && M.taps_fast && fbs_layers_fit(M) &&
-         M.d % 32 == 0 && (!rows || M.head != 1);
+  return h->pair && h->keep_small && !M.ham.heads && M.raw_gates && M.raw_transition &&
+         (M.tap_layers | M.tap_pairs) == ~0ull >> (64 - M.L) && fbs_layers_fit(M) && M.d % 32 == 0 && (!rows || M.head != 1);
 }
 
 // Whether `len` known tokens of n sequences take less time by layers than by steps. In units of a tenth of

@@ -3,7 +3,7 @@
 //
 // Layout in HBM (all tables uploaded once by uor_fbs_model_create, read by every sequence):
 //   per layer: gains (d i16) and their descriptors (gain_desc; fbs_int.h), window taps ((W+1) x d
-//              i16, tap s = s positions back) and their words (tap_word, all layers together),
+//              i16, tap s = s positions back) and their words (tap_word or tap_pair, all layers together),
 //              conv_bias (d i32), gate_bias (d/4 + d i32), decay_offset (d/4 i32), and the
 //              layer's gather program: per lane, u16 LDS byte offsets that carry out the six
 //              FBS projections (stack_fbs_gather, session.rs:4037-4053) for this lane mapping;
@@ -104,7 +104,6 @@ struct DevModel {
   uint32_t prog_words, p_rec, p_rot, p_mlp, p_down, p_dec;
   uint32_t xbar_words;      // 2 * max(d, m)
   uint32_t identity_rows;   // the nearest head: one drawer holding every token
-  uint32_t taps_fast;       // every window tap has a word (tap_word != kTapWordNone)
   uint32_t gains_fast;      // every norm gain (rec, mlp, final) has a descriptor (gain_desc)
   uint32_t log2d;           // log2(d) when d is a power of two, else 0xff
   uint32_t writer_memory;   // 1: a query equal to the writer's last one takes its result
@@ -112,7 +111,9 @@ struct DevModel {
   const DevLayer *layers;   // L entries
   const int16_t *final_gain;
   const uint16_t *final_gain_desc;
-  const int32_t *tap_words; // L * (W + 1) * d, with taps_fast
+  const int32_t *tap_words; // L * (W + 1) * d: tap_word's or tap_pair's
+  uint64_t tap_layers;      // bit l: layer l's taps all have tap_word's words (at most 64 layers)
+  uint64_t tap_pairs;       // bit l: not so, but all have tap_pair's, which stand in their place
   const uint16_t *table_b;  // vocab * d, biased
   const int16_t *keys;      // D * 16
   const uint32_t *offsets;  // D + 1

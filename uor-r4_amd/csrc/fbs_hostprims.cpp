@@ -132,7 +132,7 @@ int64_t fbs_hp_grid_apply(int64_t v, int16_t code) { return grid_apply(v, code);
 
 // Every valid grid code against n inputs v[] (their low 32 bits): mismatches of the descriptor
 // form in both halves of a word, of the gained norms' publish from its unhalved value, and of the
-// window taps' word.
+// window taps' two words.
 uint64_t fbs_hp_grid_check(const int64_t *v, uint64_t n) {
   uint64_t bad = 0;
   for (int32_t code = -2047; code <= 2047; code++) {
@@ -142,7 +142,14 @@ uint64_t fbs_hp_grid_check(const int64_t *v, uint64_t n) {
     if (tw != kTapWordNone)
       for (uint64_t i = 0; i < n; i++)
         bad += tap_word_apply((int32_t)v[i], tw) != grid_apply((int64_t)(int32_t)v[i], (int16_t)code);
+    const int32_t tp = tap_pair((int16_t)code);
+    if (tp != kTapWordNone)
+      for (uint64_t i = 0; i < n; i++)
+        bad += tap_pair_apply((int32_t)v[i], tp) != grid_apply((int64_t)(int32_t)v[i], (int16_t)code);
+    else
+      bad += tw != kTapWordNone;
     uint16_t t = gain_desc((int16_t)code);
+    bad += (t == kGridDescSlow) != (tp == kTapWordNone);
     if (t == kGridDescSlow) continue;
     const uint32_t word0 = 0xa5a50000u | t, word1 = ((uint32_t)t << 16) | 0x5a5au;
     for (uint64_t i = 0; i < n; i++) {

@@ -148,7 +148,23 @@ FBS_HD int64_t tap_word_apply(int32_t v, int32_t word) {
   return ((int64_t)v * word + (int64_t)(uint32_t)((1 << 27) + (word >> 31))) >> 28;
 }
 
-// grid_apply(v, code) for the tap descriptor in bits 16 h .. 16 h + 11 of `word`.
+// The words of a layer that has a code without a word above (a shift of 1 or of 29 to 37), all of its taps:
+// bits 6-31 the signed multiplier +-(16 + m), bits 0-5 the shift sh - 1, for 1 <= sh <= 62 (and 0 for the
+// zero code), applied as gain_desc_apply does. Ten instructions a term against tap_word's five.
+FBS_HD int32_t tap_pair(int16_t code) {
+  if (code == 0) return 0;
+  const uint32_t c = code < 0 ? (uint32_t)(-(int32_t)code) : (uint32_t)code;
+  const int32_t sh = 4 - ((int32_t)(c >> 4) - kGridExpBias);
+  if (sh < 1 || sh > 62) return kTapWordNone;
+  const int32_t mag = (int32_t)(16 + (c & 15)) * 64;
+  return (code < 0 ? -mag : mag) | (sh - 1);
+}
+FBS_HD int64_t tap_pair_apply(int32_t v, int32_t word) {
+  const int32_t mul = word >> 6;
+  return ((((int64_t)v * mul + (mul >> 31)) >> (word & 63)) + 1) >> 1;
+}
+
+// grid_apply(v, code) for the gain descriptor in bits 16 h .. 16 h + 11 of `word`.
 FBS_HD int64_t gain_desc_apply(int32_t v, uint32_t word, int h) {
   const int32_t mul = (int32_t)(word << (26 - 16 * h)) >> 26;  // sign-extended 6 bits
   const uint32_t shm1 = (word >> (16 * h + 6)) & 63u;

@@ -13,7 +13,7 @@ namespace fbs {
 struct LayerArgs {
   uint32_t n, len;
   uint32_t row, start;        // a row's tokens, the stretch's first
-  uint32_t taps_high;         // every tap word lies within +-2^27
+  uint32_t taps_high;         // every tap_word of the model lies within +-2^27
   uint32_t turns;             // positions a wavefront of the front kernel takes in turn
   uint64_t len_recip;         // floor(2^32 / len): a position's sequence without a division
   const uint32_t *tokens;     // n * row

@@ -316,8 +316,13 @@ __global__ __launch_bounds__(64 * kFrontWaves, Q == 1 ? 4 : 2) void fbs_layer_fr
 // TB/s; five blocks a CU (their LDS) leave a SIMD two or three wavefronts, whose rounds wait for one
 // another. Windows in a kernel of their own (their sums through memory): 360; operands asked for one
 // round ahead: 258.
-// High: every tap word times 16 fits 32 bits (P.taps_high).
-template <bool High>
+// Form: the layer's tap words.
+enum Taps : int {
+  kTapsHigh,  // tap_word's, every one of which times 16 fits 32 bits (P.taps_high)
+  kTapsWord,  // tap_word's
+  kTapsPair,  // tap_pair's
+};
+template <Taps Form>
 __global__ __launch_bounds__(64 * kChainWaves, 2) void fbs_layer_chain(DevModel M, LayerArgs P, uint32_t l) {
   extern __shared__ __align__(16) int32_t lds[];
   const uint32_t lane = threadIdx.x % kWave, wave = uniform32(threadIdx.x / kWave), k = lane % 4;
@@ -370,7 +375,7 @@ __global__ __launch_bounds__(64 * kChainWaves, 2) void fbs_layer_chain(DevModel 
 #pragma unroll
       for (uint32_t j = 0; j < kRound; j++) {
         const int32_t t = taps[i0 + j < W ? i0 + j : W][lv];
-        tap[j] = High ? t << 4 : t;
+        tap[j] = Form == kTapsHigh ? t << 4 : t;
         next[j] = ring[back + kRound - 1 - j][lv];
       }
 #pragma unroll
@@ -379,14 +384,14 @@ __global__ __launch_bounds__(64 * kChainWaves, 2) void fbs_layer_chain(DevModel 
 #pragma unroll
         for (uint32_t u = 0; u < kRound; u++) {
           const int32_t v = rows[(u + kRound - j) % kRound];
-          if constexpr (High) {
+          if constexpr (Form == kTapsHigh) {
             // tap_word_apply with the word times 16: the floor is the sum's high half.
             const uint32_t half = (1u << 31) + (uint32_t)(tap[j] >> 31);
             const int32_t term = (int32_t)(((int64_t)v * tap[j] + (int64_t)(uint64_t)half) >> 32);
             uint64_t carry;
             asm("v_mad_i64_i32 %0, %1, %2, 1, %0" : "+v"(acc[u]), "=s"(carry) : "v"(term));
           } else {
-            acc[u] = wadd64(acc[u], tap_word_apply(v, tap[j]));
+            acc[u] = wadd64(acc[u], Form == kTapsWord ? tap_word_apply(v, tap[j]) : tap_pair_apply(v, tap[j]));
           }
         }
         // The last position's row leaves, the one before the first's enters in its place.
@@ -864,9 +869,11 @@ hipError_t launch_fbs_layers(const DevModel &M, const LayerArgs &P, bool rows, h
   for (l = 0; l < M.L + (rows ? 1u : 0u) && e == hipSuccess; l++) {
     e = run_kernel(front, dim3((P.len + per - 1) / per, P.n), kWave * waves, args, front_lds(M, waves), stream);
     if (l == M.L) break;
+    const void *chain = (M.tap_pairs >> l) & 1 ? (const void *)fbs_layer_chain<kTapsPair>
+                        : P.taps_high          ? (const void *)fbs_layer_chain<kTapsHigh>
+                                               : (const void *)fbs_layer_chain<kTapsWord>;
     if (e == hipSuccess)
-      e = run_kernel(P.taps_high ? (const void *)fbs_layer_chain<true> : (const void *)fbs_layer_chain<false>, dim3((M.d + kWave - 1) / kWave, P.n), kWave * kChainWaves, args,
-                     chain_lds(M), stream);
+      e = run_kernel(chain, dim3((M.d + kWave - 1) / kWave, P.n), kWave * kChainWaves, args, chain_lds(M), stream);
   }
   return e;
 }

@@ -1009,6 +1009,71 @@ __device__ __forceinline__ void add_tap(const int4 &x, const int4 &t, int64_t (&
   acc[2] = wadd64(acc[2], tap_word_apply(x.z, t.z));
   acc[3] = wadd64(acc[3], tap_word_apply(x.w, t.w));
 }
+// Whether layer l's taps all have tap_word's words (else add_tap and the sums below take the general forms).
+__device__ __forceinline__ bool layer_words(const DevModel &M, uint32_t l) { return (M.tap_layers >> l) & 1; }
+__device__ __forceinline__ uint32_t layer_pairs(const DevModel &M, uint32_t l) { return (M.tap_pairs >> l) & 1; }
+
+// A layer whose taps do not: one tap at its words `tw` or codes `taps`, and taps s1..s2 of the window at
+// ring slot `base` of W, from tap_pair's words (rows and words load 8 at a time) or, where some tap has no
+// word at all (`pairs` 0), by the reference routine. Out of line, as few models have such a layer:
+// inlined, the pairs' code slowed the paired kernels of width 512 on layers of tap_word's (34.3 -> 39.2 ms
+// per 49 steps of 4,096 sequences). Width 256, one such layer of six: 1,024 sequences 8.23 ms per 129 steps
+// without it, 8.49 with it, 22.1 where the whole model took the reference routine for it.
+struct Sum4 {
+  int64_t v[4];
+};
+__device__ __noinline__ Sum4 add_tap_general(int4 x, const int32_t *tw, const int16_t *taps, uint32_t pairs, Sum4 a) {
+  const int32_t xs[4] = {x.x, x.y, x.z, x.w};
+  if (pairs) {
+    const int4 t = gload((const int4 *)tw);
+    const int32_t ts[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) a.v[c] = wadd64(a.v[c], tap_pair_apply(xs[c], ts[c]));
+  } else {
+    const short4 t = gload((const short4 *)taps);
+    const int16_t ts[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) a.v[c] = wadd64(a.v[c], grid_apply(xs[c], ts[c]));
+  }
+  return a;
+}
+__device__ __noinline__ Sum4 window_sum_general(const int32_t *ring_l, const int32_t *tw, const int16_t *taps,
+                                                uint32_t pairs, uint32_t base, uint32_t W, uint32_t s1, uint32_t s2,
+                                                uint32_t d, uint32_t ch, Sum4 a) {
+  constexpr uint32_t N = 8;
+  if (pairs) {
+    for (uint32_t s0 = s1; s0 <= s2; s0 += N) {
+      int4 hb[N], tb[N];
+#pragma unroll
+      for (uint32_t i = 0; i < N; i++) {
+        const uint32_t s = s0 + i;
+        if (s <= s2) {
+          const uint32_t sl = base >= s ? base - s : base + W - s;
+          hb[i] = gat<int4>(ring_l, 4 * (sl * d + ch));
+          tb[i] = gat<int4>(tw, 4 * (s * d + ch));
+        }
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < N; i++) {
+        if (s0 + i > s2) break;
+        const int32_t xs[4] = {hb[i].x, hb[i].y, hb[i].z, hb[i].w}, ts[4] = {tb[i].x, tb[i].y, tb[i].z, tb[i].w};
+#pragma unroll
+        for (int c = 0; c < 4; c++) a.v[c] = wadd64(a.v[c], tap_pair_apply(xs[c], ts[c]));
+      }
+    }
+    return a;
+  }
+  for (uint32_t s = s1; s <= s2; s++) {
+    const uint32_t sl = base >= s ? base - s : base + W - s;
+    const int4 x = gat<int4>(ring_l, 4 * (sl * d + ch));
+    const short4 t = gload((const short4 *)(taps + (uint64_t)s * d + ch));
+    const int32_t xs[4] = {x.x, x.y, x.z, x.w};
+    const int16_t ts[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) a.v[c] = wadd64(a.v[c], grid_apply(xs[c], ts[c]));
+  }
+  return a;
+}
 
 // ---------------------------------------------------------------------------------------------
 // One step of the session (RS stack/session.rs:4129-4403, TW 635-675) at ring slot `base`.
@@ -1099,7 +1164,7 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
     int32_t *ring_l = ring + (uint64_t)l * W * d;
     // The layer's loads first: gains, biases and the gather program.
     const int32_t *tw = M.tap_words + (uint64_t)l * (W + 1) * d;
-    short4 g_rec[Q], g_mlp[Q], tap0[Q];
+    short4 g_rec[Q], g_mlp[Q];
     uint2 gd_rec[Q], gd_mlp[Q];
     int4 tw0[Q];
     int4 cbias[Q], rbias[Q];
@@ -1112,7 +1177,6 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       const uint32_t qq = qv[k] ? qi[k] : 0, ch = 4 * qq;
       g_rec[k] = gat<short4>(ly.rec_gain, 2 * ch);
       g_mlp[k] = gat<short4>(ly.mlp_gain, 2 * ch);
-      tap0[k] = gload((const short4 *)(ly.taps + ch));
       gd_rec[k] = gat<uint2>(ly.rec_gain_desc, 2 * ch);
       gd_mlp[k] = gat<uint2>(ly.mlp_gain_desc, 2 * ch);
       tw0[k] = *(const int4 *)(tw + ch);
@@ -1199,12 +1263,13 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
       uint8_t *lt = trace ? trace + (uint64_t)l * (2 * nq + M.nm) : nullptr;
       if (lt) lt[qi[k]] = (uint8_t)root;
       int64_t wide[4];
-      if (M.taps_fast) {
-        wide[0] = cbias[k].x;
-        wide[1] = cbias[k].y;
-        wide[2] = cbias[k].z;
-        wide[3] = cbias[k].w;
-        add_tap(make_int4(drive[k][0], drive[k][1], drive[k][2], drive[k][3]), tw0[k], wide);
+      wide[0] = cbias[k].x;
+      wide[1] = cbias[k].y;
+      wide[2] = cbias[k].z;
+      wide[3] = cbias[k].w;
+      const int4 dr = make_int4(drive[k][0], drive[k][1], drive[k][2], drive[k][3]);
+      if (layer_words(M, l)) {
+        add_tap(dr, tw0[k], wide);
         for (uint32_t s0 = 1; s0 <= W; s0 += kWindowChunk) {
           if (s0 > 1) load_chunk(s0);
 #pragma unroll
@@ -1212,21 +1277,12 @@ __device__ __forceinline__ int step(const DevModel &M, const Lds &S, int32_t *ri
             if (s0 + i <= W) add_tap(hb[i], tb[i], wide);
         }
       } else {
-        // A tap without a word somewhere in the model: the reference routine.
-        const short4 t0 = tap0[k];
-        wide[0] = wadd64(cbias[k].x, grid_apply(drive[k][0], t0.x));
-        wide[1] = wadd64(cbias[k].y, grid_apply(drive[k][1], t0.y));
-        wide[2] = wadd64(cbias[k].z, grid_apply(drive[k][2], t0.z));
-        wide[3] = wadd64(cbias[k].w, grid_apply(drive[k][3], t0.w));
-        for (uint32_t s = 1; s <= W; s++) {
-          const uint32_t sl = base >= s ? base - s : base + W - s;
-          const int4 hh = *(const int4 *)(ring_l + (uint64_t)sl * d + ch);
-          const short4 t = gload((const short4 *)(ly.taps + (uint64_t)s * d + ch));
-          wide[0] = wadd64(wide[0], grid_apply(hh.x, t.x));
-          wide[1] = wadd64(wide[1], grid_apply(hh.y, t.y));
-          wide[2] = wadd64(wide[2], grid_apply(hh.z, t.z));
-          wide[3] = wadd64(wide[3], grid_apply(hh.w, t.w));
-        }
+        const uint32_t pairs = layer_pairs(M, l);
+        Sum4 a{{wide[0], wide[1], wide[2], wide[3]}};
+        a = add_tap_general(dr, tw + ch, ly.taps + ch, pairs, a);
+        a = window_sum_general(ring_l, tw, ly.taps, pairs, base, W, 1, W, d, ch, a);
+#pragma unroll
+        for (int c = 0; c < 4; c++) wide[c] = a.v[c];
       }
       *(int4 *)(ring_l + (uint64_t)base * d + ch) =
           make_int4(drive[k][0], drive[k][1], drive[k][2], drive[k][3]);
@@ -1909,17 +1965,17 @@ __device__ __forceinline__ int step_main(const DevModel &M, const Lds &S, uint32
   return 0;
 }
 
-// Tap k of layer l on the lane's four channels of x: tap words or grid codes.
+// Tap k of layer l on the lane's four channels of x.
 __device__ __forceinline__ void tap4(const DevModel &M, const DevLayer &ly, uint32_t l, uint32_t k,
                                      uint32_t ch, const int4 &x, int64_t (&acc)[4]) {
-  if (M.taps_fast) {
-    add_tap(x, *(const int4 *)(M.tap_words + ((uint64_t)l * (M.W + 1) + k) * M.d + ch), acc);
+  const uint32_t at = k * M.d + ch;
+  const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * M.d + at;
+  if (layer_words(M, l)) {
+    add_tap(x, *(const int4 *)tw, acc);
   } else {
-    const short4 t = gload((const short4 *)(ly.taps + (uint64_t)k * M.d + ch));
-    acc[0] = wadd64(acc[0], grid_apply(x.x, t.x));
-    acc[1] = wadd64(acc[1], grid_apply(x.y, t.y));
-    acc[2] = wadd64(acc[2], grid_apply(x.z, t.z));
-    acc[3] = wadd64(acc[3], grid_apply(x.w, t.w));
+    const Sum4 a = add_tap_general(x, tw, ly.taps + at, layer_pairs(M, l), {{acc[0], acc[1], acc[2], acc[3]}});
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = a.v[c];
   }
 }
 
@@ -1931,8 +1987,8 @@ __device__ __forceinline__ void window_sum(const DevModel &M, const DevLayer &ly
                                            const int32_t *ring_l, uint32_t base, uint32_t s1,
                                            uint32_t ch, int64_t (&acc)[4], uint32_t s2 = 0) {
   const uint32_t d = M.d, W = s2 ? s2 : M.W;  // taps s1..W (the last tap s2 when given)
-  if (M.taps_fast) {
-    const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * d;
+  const int32_t *tw = M.tap_words + (uint64_t)l * (M.W + 1) * d;
+  if (layer_words(M, l)) {
     for (uint32_t s0 = s1; s0 <= W; s0 += N) {
       int4 hb[N], tb[N];  // the rows and the taps' words
 #pragma unroll
@@ -1949,11 +2005,10 @@ __device__ __forceinline__ void window_sum(const DevModel &M, const DevLayer &ly
         if (s0 + i <= W) add_tap(hb[i], tb[i], acc);
     }
   } else {
-    // A tap without a word somewhere in the model: the reference routine.
-    for (uint32_t s = s1; s <= W; s++) {
-      const uint32_t sl = base >= s ? base - s : base + M.W - s;
-      tap4(M, ly, l, s, ch, *(const int4 *)(ring_l + (uint64_t)sl * d + ch), acc);
-    }
+    const Sum4 a = window_sum_general(ring_l, tw, ly.taps, layer_pairs(M, l), base, M.W, s1, W, d, ch,
+                                      {{acc[0], acc[1], acc[2], acc[3]}});
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = a.v[c];
   }
 }
 
