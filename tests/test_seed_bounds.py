@@ -1,7 +1,8 @@
-"""The kernels' reciprocal and reciprocal-square-root estimates (fbs_int.h rsqrt_q46, recip_q63),
-checked over every input they take by tests/seed_bounds.cpp: the error bounds the exact
-corrections downstream rely on, and equality with the same Newton steps in 64-bit products (the
-32-bit forms the kernels use)."""
+"""The kernels' reciprocal and reciprocal-square-root estimates (fbs_int.h rsqrt_q46,
+rsqrt_q46s, rsqrt_q86, recip_q63), checked over every input they take (rsqrt_q86: every high word) by
+tests/seed_bounds.cpp: the error bounds that the exact corrections downstream, and the routines that
+have none, rely on, and equality with the same Newton steps in 64-bit products (the 32-bit forms the
+kernels use)."""
 
 import os
 import subprocess

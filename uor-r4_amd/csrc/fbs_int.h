@@ -6,10 +6,13 @@
 // saturate, products modulo 2^64 / 2^128, floor square roots and floor quotients. The reference
 // forms its roots digit by digit and its quotients by hardware or restoring division; a GPU has
 // neither, so this file computes them from fixed-point reciprocal estimates (a seed table and
-// Newton steps) and then corrects the estimate with exact integer checks. The correction loops
-// make the result exact for every input whatever the estimate's error; the estimates only
-// decide how many correction steps run (at most one or two for every input class the tests
-// sweep). No floating point is used anywhere.
+// Newton steps). The general routines (isqrt128, div128_64, norm_factor, unit_q30_wide) correct
+// the estimate until exact integer checks hold, whatever its error. The kernels' short forms make a fixed
+// number of corrections or none: norm_factor_pow2 and norm_factor_wave rest on the bounds of rsqrt_q46
+// and recip_q63, unit_q30_64 (one step up for the root, steps up only for the quotients) and
+// norm_factor_direct (it refuses what lies too near a whole number) on those of rsqrt_q46s and rsqrt_q86.
+// The four bounds are checked over every input by tests/seed_bounds.cpp (rsqrt_q86's over every high
+// word). No floating point is used anywhere.
 //
 // The functions are __host__ __device__ so that the same code is compiled into the kernels and
 // into a host library that the CPU tests check against the oracle.
@@ -281,7 +284,7 @@ FBS_HD uint32_t rsqrt_q46s(uint32_t t, const uint32_t *tab) {
   }
   return y < 0x7fffffffu ? y : 0x7fffffffu;
 }
-// 2^86 / sqrt(xn) for xn in [2^62, 2^64), in (2^54, 2^55], within (-2, +0.1]: y = rsqrt_q46s of xn's
+// 2^86 / sqrt(xn), from 2^54 to 2^55, for xn in [2^62, 2^64), within (-2, +0.1]: y = rsqrt_q46s of xn's
 // high word is 2^62 / sqrt(xn) (1 + d), |d| < 2^-28; one Newton step y (1 + E / 2) on E =
 // 1 - y^2 xn / 2^124 leaves -1.5 d^2 (at most 0.75 of the result's units), the products' floors in
 // E (3 units of 2^-60, then its top 31 bits) less than 0.1 and the last floor 1.
