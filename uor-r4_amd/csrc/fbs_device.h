@@ -294,14 +294,13 @@ struct ServeScan {
   uint32_t *item_count;
   uint32_t item_cap;
   uint32_t n;                             // sequences of the launch
-  uint32_t gen;                           // the launch's generated steps (the out_tokens stride)
   const uint32_t *job_query;
   uint32_t *job_flag;
   unsigned long long *job_best;
   uint32_t *drawer_count;
   const uint32_t *drawer_list;
   uint32_t list_stride;
-  uint32_t *out_tokens;
+  uint32_t *out_tokens;                   // n: a job's token at its index
   const uint32_t *slots;
   uint8_t *cache;                         // nullable
   uint32_t cache_stride;

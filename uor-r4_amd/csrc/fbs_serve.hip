@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void fbs_serve_finish(DevModel M, ServeScan J)
   const uint32_t slot = J.cache ? J.slots[i] : 0u;
   if (!flag) return;
   J.job_flag[i] = 0;
-  J.out_tokens[(uint64_t)i * (J.gen + 1)] = tok;
+  J.out_tokens[i] = tok;
   if (J.cache) {
     uint32_t *head = (uint32_t *)(J.cache + (uint64_t)slot * J.cache_stride);
     head[1] = M.writer_memory;
