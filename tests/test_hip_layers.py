@@ -4,6 +4,7 @@ the edges of the stretches, widths and windows, fresh and resumed sessions, refu
 contexts. Every output is an integer and equal."""
 
 import ctypes as C
+from contextlib import contextmanager
 from dataclasses import replace
 
 import numpy as np
@@ -27,6 +28,10 @@ SHAPES = {
     "w768": synth.Spec(vocab=2048, width=768, mlp=1024, layers=2, context=96, kept=4, window=24, drawers=64, probes=4),
     # The shortest window over the reference's cells, and the whole-table head.
     "w64": synth.Spec(vocab=4096, width=64, mlp=96, layers=2, context=96, kept=8, window=1),
+    # Taps of up to 4, whose words do not fit the chain's shortest form, over several rounds of taps.
+    "w256t": replace(synth.CONFIGS["c3"], context=96, layers=3, tap_fields=(59, 66)),
+    "w320t": synth.Spec(vocab=2048, width=320, mlp=512, layers=2, context=96, kept=4, window=40, drawers=33, probes=3,
+                        tap_fields=(59, 66)),
 }
 DEEP = synth.Spec(vocab=512, width=1024, mlp=1024, layers=16, context=96, kept=4, window=64, drawers=32, probes=3)
 
@@ -86,6 +91,14 @@ def rows(model, tokens):
     return got
 
 
+@contextmanager
+def by_layers(model, calls):
+    """The calls inside all ran by layers."""
+    before = model.layer_calls
+    yield
+    assert model.layer_calls == before + calls
+
+
 def tokens_for(name, n, length, seed):
     spec = SHAPES[name]
     make = synth.zipf_prompts if spec.zipf_drawers else synth.uniform_prompts
@@ -98,12 +111,14 @@ def test_prompts_equal_the_step_kernels(models, monkeypatch, name, n, length):
     art, layers, steps = models(name, monkeypatch)
     print(f"prompts {name}: {n} of {length}", flush=True)
     a = tokens_for(name, n, length, 5)
-    first = decode(layers, a, 3)
+    with by_layers(layers, 1):
+        first = decode(layers, a, 3)
     for got, want in zip(first, decode(steps, a, 3)):
         np.testing.assert_array_equal(got, want)
     # The sessions resumed by a second prompt, whose choices the oracle makes in one pass.
     b = tokens_for(name, n, 12, 6)
-    second = decode(layers, b, 0, first[1:4])
+    with by_layers(layers, 1):
+        second = decode(layers, b, 0, first[1:4])
     for got, want in zip(second, decode(steps, b, 0, first[1:4])):
         np.testing.assert_array_equal(got, want)
     if name in ("w128", "w96"):
@@ -119,7 +134,8 @@ def test_rows_equal_the_step_kernels(models, monkeypatch, name, n, length):
     art, layers, steps = models(name, monkeypatch)
     print(f"rows {name}: {n} of {length}", flush=True)
     t = tokens_for(name, n, length, 7)
-    got = rows(layers, t)
+    with by_layers(layers, 3):
+        got = rows(layers, t)
     for g, w in zip(got, rows(steps, t)):
         np.testing.assert_array_equal(g, w)
     if name in ("w128", "w96"):
@@ -138,9 +154,10 @@ def test_refused_sequences(models, monkeypatch, name):
     t = tokens_for(name, 8, 24, 8)
     for r, at in ((0, 0), (2, 11), (3, 23), (4, 22), (6, 20)):
         t[r, at] = vocab + r
-    for g, w in zip(rows(layers, t), rows(steps, t)):
+    with by_layers(layers, 4):
+        served, fresh = rows(layers, t), decode(layers, t, 2)
+    for g, w in zip(served, rows(steps, t)):
         np.testing.assert_array_equal(g, w)
-    fresh = decode(layers, t, 2)
     for g, w in zip(fresh, decode(steps, t, 2)):
         np.testing.assert_array_equal(g, w)
     assert [int(s) for s in fresh[4]] == [1, 0, 1, 1, 1, 0, 1, 0]
@@ -148,12 +165,13 @@ def test_refused_sequences(models, monkeypatch, name):
     position = np.array([10, context - 24, context - 24, context, context - 20, context - 12, context - 3, context - 26],
                         np.uint32)
     resume = (warm[1], warm[2], position)
-    held = decode(layers, t, 2, resume)
+    with by_layers(layers, 1):
+        held = decode(layers, t, 2, resume)
     for g, w in zip(held, decode(steps, t, 2, resume)):
         np.testing.assert_array_equal(g, w)
 
 
-@pytest.mark.parametrize("name", ["w128", "w96", "w320", "w512i8"])
+@pytest.mark.parametrize("name", ["w128", "w96", "w320", "w512i8", "w256t", "w320t"])
 def test_sessions_at_the_ends_of_their_range(models, monkeypatch, name):
     # States and window rows over all of their types' values: the transport leaves its fast form's ranges
     # (at the first positions, in some quaternions only) and comes back to them.
@@ -168,7 +186,9 @@ def test_sessions_at_the_ends_of_their_range(models, monkeypatch, name):
     history[4] >>= 12
     resume = (state, history, np.arange(n, dtype=np.uint32))
     t = tokens_for(name, n, 43, 13)
-    for g, w in zip(decode(layers, t, 1, resume), decode(steps, t, 1, resume)):
+    with by_layers(layers, 1):
+        got = decode(layers, t, 1, resume)
+    for g, w in zip(got, decode(steps, t, 1, resume)):
         np.testing.assert_array_equal(g, w)
 
 
@@ -179,9 +199,10 @@ def test_parts_and_stretches_of_a_large_launch(models, monkeypatch, n, length):
     t = tokens_for("w512i8", n, length, 10)
     t[n - 100, 3] = t[n - 5, length - 7] = SHAPES["w512i8"].vocab
     print(f"rows {n} of {length}", flush=True)
-    got = rows(layers, t)
-    print("prompts", flush=True)
-    fed = decode(layers, t, 1)
+    with by_layers(layers, 4):
+        got = rows(layers, t)
+        print("prompts", flush=True)
+        fed = decode(layers, t, 1)
     pick = [0, 700, n - 577, n - 576, n - 101, n - 100, n - 5, n - 1]
     for i, w in enumerate(rows(steps, t[pick])[:4]):
         np.testing.assert_array_equal(got[i][pick], w)
