@@ -37,7 +37,11 @@ from .session_codec import (STACK_SESSION_SCHEMA, CodecError, RecurrenceLayer, S
 
 NO_CHOICE = 0xFFFFFFFF  # session.rs:4406: a nearest-head read step chose no token
 TRACE_UNSET = 0xFFFFFFFF  # a snap trace entry no step has written (session.rs:2580-2584)
-# Launches whose inputs and outputs fit this many bytes pass them in the pool's own pinned buffer.
+# Launches whose inputs and outputs fit this many bytes pass them in the pool's own pinned buffer, which the
+# kernels read and write over the bus; others in one device block, copied in and out. In place is no slower
+# up to here (us a call, in place and by a block): one session of width 128 100 and 123, 900 of width 256
+# with their queries (942 KiB) 217 and 228, a prompt of 509 tokens 15,010 and 15,241, a trace of 674 KiB
+# 3,658 and 3,685.
 IN_PLACE_BYTES = 1 << 20
 TRACE_ZERO = 255  # the launch's trace byte for a zero raw quaternion, whose selection is root 0
 
