@@ -201,9 +201,10 @@ def workload_key(a) -> str:
     return f"{a.config} batch {a.batch} prompt {a.prompt} gen {a.gen} seed {a.seed}"
 
 
-def measured_traffic(a, kernel):
+def measured_traffic(a, kernel, launch_ms=None):
     """HBM bytes per timed launch from the config's committed counter summary, if it covers this
-    exact workload and kernel; None otherwise."""
+    exact workload and kernel and, where `launch_ms` is given, a kernel as fast as this one (its launch
+    within 5 %: the counters of an earlier form are not this one's); None otherwise."""
     try:
         text = open(os.path.join(ROOT, "profiles", TRAFFIC_SUMMARIES[a.config])).read()
     except (KeyError, OSError):
@@ -213,7 +214,18 @@ def measured_traffic(a, kernel):
     t = re.search(r"^traffic_bytes_per_launch: (\d+)$", text, re.M)
     if not w or not k or not t or w.group(1).strip() != workload_key(a) or k.group(1).strip() != kernel:
         return None
+    if launch_ms is not None:
+        ms = re.search(r"At the launch time ([\d.]+) ms", text)
+        if not ms or abs(float(ms.group(1)) / launch_ms - 1) > 0.05:
+            return None
     return int(t.group(1))
+
+
+def traffic_section(a, kernel, launch_ms):
+    """The measured HBM bytes of a launch and their share of the HBM peak (None: no summary of it)."""
+    traffic = measured_traffic(a, kernel, launch_ms)
+    frac = None if traffic is None else round(traffic / (launch_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4)
+    return {"traffic": traffic, "traffic_frac": frac}
 
 
 def algorithmic_bytes_per_token(spec, mean_candidates: float) -> float:
@@ -223,6 +235,19 @@ def algorithmic_bytes_per_token(spec, mean_candidates: float) -> float:
     c = 1 if spec.table == "i8" else 2
     d, L, W = spec.width, spec.layers, spec.window
     return c * d + L * (W * d * 4 + d * 4) + c * d * mean_candidates + 4
+
+
+def layer_bytes_per_position(spec, mean_candidates: float, probes: int) -> float:
+    """Bytes that the layer by layer kernels ask for at one scored position. Per layer and channel: the front
+    kernel writes the residual, drive, transition, output gate and keep (17) and reads back the residual,
+    gate and moved state (16), the chain reads drive, transition and keep (9) and writes the moved
+    state (8). Once: the input row, the residual for the query (4 written, 4 read), the query's words
+    (2), the kept drawers written, read twice and listed. The scan reads a query's words once per 64
+    member rows and a member row once per 32 queries."""
+    c = 1 if spec.table == "i8" else 2
+    d = spec.width
+    return (50 * d * spec.layers + (c + 4 + 4 + 2) * d + 16 * probes
+            + mean_candidates * (2 * d / 64 + c * d / 32) + 4)
 
 
 # Bytes one token moves in an index build by the path's definition: its two 8-value endpoint
@@ -438,15 +463,21 @@ def score_main(a, torch, oracle, art, model, rows, dev, stream, sp) -> dict:
     _, kept, _ = model.sequences(rows[:sample])
     cand = art.drawer_sizes()[kept.astype(np.int64)].sum(-1)
     mean_cand = float(cand.mean())
-    bpt = algorithmic_bytes_per_token(spec, mean_cand) + 4  # plus each position's input id
-    achieved = bpt * positions / (float(np.mean(launch_ms)) / 1e3) / 1e9
+    mean_ms = float(np.mean(launch_ms))
     S = 1
     while S < spec.width // 32:
         S *= 2
-    # Paired models score rows layer by layer, the others by steps.
-    family = "fbs_rows_8" if spec.table == "i8" else "fbs_rows"
-    kernel = ("fbs_layer_front, fbs_layer_chain, fbs_layer_query, fbs_layer_scan" if model.block_waves(R) == 2
-              else f"{family}<{(spec.width // 4 + 63) // 64}, {S}>")
+    if model.layer_calls:  # rows scored layer by layer
+        bpt = layer_bytes_per_position(spec, mean_cand, art.probes)
+        kernel = "fbs_layer_front, fbs_layer_chain, fbs_layer_query, fbs_layer_scan"
+        what = ("bytes the layer kernels ask for (the scan's mostly of the L2); vector instructions, not "
+                "these bytes, bound the launch")
+    else:
+        bpt = algorithmic_bytes_per_token(spec, mean_cand) + 4  # plus each position's input id
+        family = "fbs_rows_8" if spec.table == "i8" else "fbs_rows"
+        kernel = f"{family}<{(spec.width // 4 + 63) // 64}, {S}>"
+        what = "bytes each position asks for (blocks share candidate rows through the caches)"
+    achieved = bpt * positions / (mean_ms / 1e3) / 1e9
     out = {
         "metric": f"teacher-forced scored positions/sec, {R} rows x {n}, width {spec.width} (1 GPU)",
         "value": round(positions / (ms_per_step / 1e3), 1), "unit": "positions/s", "n_gpus": 1,
@@ -461,7 +492,7 @@ def score_main(a, torch, oracle, art, model, rows, dev, stream, sp) -> dict:
         "matches": int(matches.item()),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic(a, kernel),
+                     "what": what, **traffic_section(a, kernel, mean_ms),
                      "bytes_per_position": round(bpt, 1), "mean_candidate_rows": round(mean_cand, 1),
                      "kernel": kernel,
                      "launch_ms": [round(x, 3) for x in launch_ms]},
@@ -794,7 +825,7 @@ def hamming_main(a, torch, oracle) -> dict:
                    "vocab": spec.vocab, "parallelism": "none (1 GPU)"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic(a, ham_kernel),
+                     **traffic_section(a, ham_kernel, float(np.mean(launch_ms))),
                      "bytes_per_token": {k: round(v, 1) for k, v in bpt.items()},
                      "mean_candidate_rows": round(mean_cand, 1),
                      "kernel": ham_kernel,
@@ -1000,7 +1031,6 @@ def main():
     if spec.table == "i8":  # the int8 table's own kernels (fbs_decode_pair8, fbs_decode_8)
         family += "8" if family.endswith("pair") else "_8"
     kernel = f"{family}<{(spec.width // 4 + 63) // 64}, {S}>"
-    traffic = measured_traffic(a, kernel)
 
     out = {
         "metric": f"decoded tokens/sec at batch {B}, width {spec.width} (1 GPU)",
@@ -1029,7 +1059,10 @@ def main():
         # memory off in without_writer_memory.
         "roofline": {
             "bound": "hbm", "achieved": round(achieved_scanned, 1), "peak": HBM_PEAK_GBS,
-            "unit": "GB/s", "frac": round(achieved_scanned / HBM_PEAK_GBS, 4), "traffic": traffic,
+            "unit": "GB/s", "frac": round(achieved_scanned / HBM_PEAK_GBS, 4),
+            "what": "bytes the tokens ask for: blocks share candidate rows through the caches, so that HBM "
+                    "moves fewer (traffic)",
+            **traffic_section(a, kernel, float(np.mean(launch_ms))),
             "algorithmic_bytes_per_launch": round(bpt_scanned * tokens),
             "bytes_per_token": round(bpt_scanned, 1),
             "scanned_candidate_rows": round(scanned_cand, 1),

@@ -56,6 +56,27 @@ def test_measured_traffic_matches_only_its_workload():
     assert bench.measured_traffic(b, "fbs_decode_pair<1, 8>") is None  # another workload
 
 
+def test_measured_traffic_is_of_a_kernel_as_fast(tmp_path, monkeypatch):
+    (tmp_path / "profiles").mkdir()
+    name = bench.TRAFFIC_SUMMARIES["c3"]
+    (tmp_path / "profiles" / name).write_text(
+        "workload: c3 batch 1024 prompt 1024 gen 1024 seed 2026120203\nkernel: k\n"
+        "traffic_bytes_per_launch: 480000000000\n\nAt the launch time 80.000 ms the measured traffic is ...\n")
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    a = _Args()
+    assert bench.traffic_section(a, "k", 80.0) == {"traffic": 480000000000, "traffic_frac": 0.75}
+    assert bench.measured_traffic(a, "k", 83.9) == bench.measured_traffic(a, "k") == 480000000000
+    assert bench.traffic_section(a, "k", 70.0) == {"traffic": None, "traffic_frac": None}
+
+
+def test_layer_bytes_terms():
+    spec = replace(synth.CONFIGS["c4"], layers=1)
+    d = spec.width
+    assert bench.layer_bytes_per_position(spec, 0, 8) == 50 * d + 12 * d + 128 + 4
+    # 64 more candidate rows: the query's words once, 64 rows for 32 queries
+    assert bench.layer_bytes_per_position(spec, 64, 8) - bench.layer_bytes_per_position(spec, 0, 8) == 2 * d + 4 * d
+
+
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True, timeout=120)

@@ -15,7 +15,7 @@
 // reads a member row once for the queries that kept its drawer.
 // Every value is formed by the step's own routines (fbs_run.h), so the results are its bit for bit.
 // At width 256 (6 layers, window 16), 300 prompts of 509 tokens: 19.2 ms by steps, 3.8 by layers (front
-// 430 us a layer, chain 230); 8,192 rows of 128 76 and 40 ms.
+// 448 us a layer, chain 214); 8,192 rows of 128 76 and 40 ms.
 #include "fbs_layers.h"
 
 #include <type_traits>
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64) void fbs_layer_begin(DevModel M, LayerArgs P) {
 }
 
 // Bound by its instructions: 1,413 vector and 358 scalar ones a position and layer at width 256 (most of
-// 8 bytes, 5.3 cycles each) take the 430 us that it measures for 152,700 positions.
+// 8 bytes, 5.3 cycles each) take the 448 us that it measures for 152,400 positions.
 // The end of layer l - 1 (the output gate on the moved state, rec_out, the feed-forward block; none
 // at l = 0, where the position's table row comes in) and the start of layer l (none at l = L), for
 // blockIdx.y's sequence, a wavefront a position.
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(64 * kFrontWaves, Q == 1 ? 4 : 2) void fbs_layer_fr
 //   of a whole quaternion. Eight positions move by transport_fast's form without a branch; where one
 //   left its ranges, they move again from the state before them in 128 bits.
 // Lanes past the width repeat the last quaternion's.
-// 300 sequences of 509 positions, width 256: 230 us. Its bytes, 17 a channel and position, take 130 at 5
+// 300 sequences of 508 positions, width 256: 214 us. Its bytes, 17 a channel and position, take 130 at 5
 // TB/s; five blocks a CU (their LDS) leave a SIMD two or three wavefronts, whose rounds wait for one
 // another. Windows in a kernel of their own (their sums through memory): 360; operands asked for one
 // round ahead: 258.
@@ -678,7 +678,7 @@ __global__ __launch_bounds__(256) void fbs_layer_lists(DevModel M, LayerArgs P, 
 // every query in all lanes, reads 16 bytes for 4 SADs and reduces 64 lanes a query, a third of its
 // instructions: 32,768 queries of width 256 that kept 8 of 256 drawers 433 us, here 310. One-token
 // launches keep it: their thousand queries fill few slices of 32, and a wavefront then waits through
-// four segments of a row one after another (1,024 sessions 2.88 ms per 64 tokens, with this 3.09).
+// four segments of a row one after another (1,024 sessions 2.88 ms per 32 tokens, with this 3.09).
 // Queries in lanes' registers and rows by scalar loads: 529 us, the scalar cache missing on every row.
 // RW: the row words (biased 16-bit pairs) of a segment; rows of more words are scored in segments of
 // RW, the sums carried across. T8: an int8 table, whose rows (code + 128 bytes) widen at the SADs as the
