@@ -264,6 +264,12 @@ def test_the_workspace_keeps_to_its_bound(models, monkeypatch):
     for g, w in zip(rows(small, t), rows(steps, t)):
         np.testing.assert_array_equal(g, w)
     assert small.layer_calls == 4
+    # A sequence at a time would cost more than the steps: none goes by layers.
+    monkeypatch.setenv("UOR_FBS_LAYER_BYTES", str(300 << 10))
+    tiny = hip.Model(art)
+    for g, w in zip(decode(tiny, t, 1) + rows(tiny, t), decode(steps, t, 1) + rows(steps, t)):
+        np.testing.assert_array_equal(g, w)
+    assert tiny.layer_calls == tiny.layer_bytes == 0
     monkeypatch.setenv("UOR_FBS_LAYER_BYTES", "0")
     none = hip.Model(art)
     with pytest.raises(hip.FbsError):

@@ -999,9 +999,11 @@ bool layer_model(const uor_fbs_handle *h, bool rows) {
 // calls that the rule takes: 0.92 to 126 times the steps' speed, but for rows of one repeated token with two
 // small drawers kept (0.87: the writer's memory then spares the steps their scan). The 0.92 are 2,048 prompts
 // of 24 at width 256, two full turns of the grid.
-bool layers_pay(const uor_fbs_handle *h, uint64_t n, uint32_t len, bool rows) {
-  const uint64_t G = h->pair_grid, turns = (n + G - 1) / G, t = len < 64 ? len : 64;
-  return t * (10 * turns * G - (rows ? 4 : 7) * n) >= (rows ? 30 : 40) * G;
+// Run in several parts or stretches, each has its launches.
+bool layers_pay(const uor_fbs_handle *h, uint64_t n, uint64_t len, bool rows, uint32_t part, uint32_t run) {
+  const uint64_t G = h->pair_grid, turns = (n + G - 1) / G, t = len < 1u << 20 ? len : 1u << 20;
+  const uint64_t launches = ((n + part - 1) / part) * ((len + run - 1) / run);
+  return t * (10 * turns * G - (rows ? 4 : 7) * n) >= (rows ? 30 : 40) * G * launches;
 }
 
 bool capturing(hipStream_t stream) {
@@ -1055,8 +1057,8 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
   *taken = false;
   const bool rows = A.mode != kModeDecode;
   const uint32_t len = rows ? A.len : A.len - 1;
-  if (A.slots || A.out_trace || A.out_dtrace || A.out_parts || !layer_model(h, rows) ||
-      !layers_pay(h, A.n, len, rows) || capturing(stream))
+  if (len == 0 || A.slots || A.out_trace || A.out_dtrace || A.out_parts || !layer_model(h, rows) ||
+      !layers_pay(h, A.n, len, rows, A.n, len) || capturing(stream))
     return 0;
   const uint32_t jobs = rows ? layer_jobs(h) : 0;
   if (rows && jobs == 0) return 0;
@@ -1084,6 +1086,7 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
       if (bit < len - most && bytes(part, most + bit) <= room) most += bit;
     const uint32_t stretches = (len + most - 1) / most;
     run = (len + stretches - 1) / stretches;
+    if (!layers_pay(h, A.n, len, rows, part, run)) return 0;
   } while (!h->ensure_layers(bytes(part, run)));
   const bool sessions = !rows || run < len;
   // A call that finds no room for what it can do without says nothing of it.
