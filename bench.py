@@ -45,7 +45,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # passes, scaled by a copy kernel's reading), for the workload each summary names.
 TRAFFIC_SUMMARIES = {
     "c2": "fbs_decode_pair_c2_b1024_traffic.md", "c3": "fbs_decode_pair_c3_b1024_traffic.md",
-    "c4": "fbs_rows_pair_c4_r1048576_traffic.md", "c5": "fbs_decode_pair8_c5_b16384_traffic.md",
+    "c4": "fbs_layers_c4_r1048576_traffic.md", "c5": "fbs_decode_pair8_c5_b16384_traffic.md",
     "hamming": "fbs_decode_pair_ham_c3_b1024_traffic.md"}
 D11_TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "d11_score_rows_m1_traffic.md")
 # BASELINE.json's configs at their full shapes: (sequences, prompt, decode steps); c4 is
@@ -470,8 +470,7 @@ def score_main(a, torch, oracle, art, model, rows, dev, stream, sp) -> dict:
     if model.layer_calls:  # rows scored layer by layer
         bpt = layer_bytes_per_position(spec, mean_cand, art.probes)
         kernel = "fbs_layer_front, fbs_layer_chain, fbs_layer_query, fbs_layer_scan"
-        what = ("bytes the layer kernels ask for (the scan's mostly of the L2); vector instructions, not "
-                "these bytes, bound the launch")
+        what = "bytes the layer kernels ask for; their vector instructions, not these bytes, bound the launch"
     else:
         bpt = algorithmic_bytes_per_token(spec, mean_cand) + 4  # plus each position's input id
         family = "fbs_rows_8" if spec.table == "i8" else "fbs_rows"
