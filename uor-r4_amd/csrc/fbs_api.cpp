@@ -1108,8 +1108,12 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
   h->layer_calls++;
   // The same call under capture runs on the step kernels, where nothing may be allocated: the call that
   // warms up for it leaves the ring that it needs, also where the parts (or rows, which need none) do not.
-  if (h->ensure_ring(A.n < h->pair_grid ? A.n : h->pair_grid))
-    skip();  // rows run without it, a decode's step launches report it
+  // Allocated while the layers run; one that grows before them, as its release waits for the device.
+  const auto leave_ring = [&] {
+    if (h->ensure_ring(A.n < h->pair_grid ? A.n : h->pair_grid))
+      skip();  // rows run without it, a decode's step launches report it
+  };
+  if (h->ring_blocks) leave_ring();
   const size_t ld = (size_t)M.L * M.d;
   for (uint32_t s0 = 0; s0 < A.n; s0 += part) {
     const uint32_t n = A.n - s0 < part ? A.n - s0 : part;
@@ -1160,6 +1164,7 @@ int launch_layers(uor_fbs_handle *h, const RunArgs &A, hipStream_t stream, bool 
       e = launch_fbs_layer_choices(P, stream);
       if (e != hipSuccess) return hip_fail(e, "kernel launch");
     }
+    if (s0 == 0) leave_ring();
     if (rows) continue;
     RunArgs B = A;  // the prompts' last tokens and the generated steps
     B.n = n;
